@@ -4,6 +4,7 @@
  */
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -34,6 +35,7 @@ struct bsim_sim {
     bsim_dev d{};
     std::vector<void *> allocs;
     int64_t device_bytes = 0;
+    int32_t tile = 0, ntiles = 0;   /* as the caller sees them; the device works in units */
     int32_t cycle = 0;
     int32_t finished_at = -1;
     int64_t *ev_fin = nullptr;   /* deliveries of the deliver-only launch */
@@ -365,7 +367,7 @@ bsim_sim *bsim_sim_create(const bsim_network *net, float dt, const bsim_sim_conf
     bsim::Layout L;
     std::string err;
     try {
-        if (bsim::build_layout(net->net, dt, tile, L, err) != 0) {
+        if (bsim::build_layout(net->net, dt, tile, L, err, 0, bsim::default_parts(N, tile)) != 0) {
             fail(BSIM_E_NETWORK, err);
             return nullptr;
         }
@@ -421,7 +423,8 @@ bsim_sim *bsim_sim_create_chains(const bsim_chain_params *p, int32_t count, floa
                                            hipMemcpyHostToDevice);
             return x == hipSuccess ? 0 : fail(BSIM_E_HIP, std::string("synapse upload: ") + hipGetErrorString(x));
         };
-        rc = bsim::build_chains_layout(p, count, dt, tile, dmax, part_synapses, L, first_ids, err, upload);
+        rc = bsim::build_chains_layout(p, count, dt, tile, dmax, part_synapses, L, first_ids, err, upload,
+                                       bsim::default_parts(nn, tile));
     } catch (const std::bad_alloc &) {
         rc = -1;
         err = "out of host memory while building the layout";
@@ -449,6 +452,7 @@ static bsim_sim *sim_from_layout(bsim::Layout &L, const bsim_sim_config &c, bsim
                                  int64_t dev_syn_bytes)
 {
     hipError_t e = hipSuccess;
+    std::vector<uint8_t> res;      /* XCD residue of each unit */
     bsim_sim *sim = new (std::nothrow) bsim_sim();
     if (!sim) {
         if (dev_syn) (void)hipFree(dev_syn);
@@ -469,8 +473,10 @@ static bsim_sim *sim_from_layout(bsim::Layout &L, const bsim_sim_config &c, bsim
     }
     bsim_dev &d = sim->d;
     d.n = L.n;
-    d.tile = L.tile;
-    d.ntiles = L.ntiles;
+    sim->tile = L.tile;
+    sim->ntiles = L.ntiles;
+    d.tile = L.tile / L.parts;
+    d.ntiles = L.ntiles * L.parts;
     d.dmax = L.dmax;
     d.nwords = (L.n + 63) / 64;
     sim->s = L.s;
@@ -490,10 +496,24 @@ static bsim_sim *sim_from_layout(bsim::Layout &L, const bsim_sim_config &c, bsim
     UP(bern_seed, L.bern_seed);
     UP(bern_key, L.bern_key);
     UP(pois_tab, L.pois_tab);
-    UP(tile_base, L.tile_base);
-    UP(tile_nsyn, L.tile_nsyn);
-    UP(tile_res, L.tile_res);
-    d.nslots = L.nslots;
+    res.resize((size_t)d.ntiles);
+    {
+        std::vector<bsim_unit> unit((size_t)d.ntiles);
+        for (int32_t u = 0; u < d.ntiles; u++) {
+            const int32_t t = u / L.parts;
+            bsim_unit &x = unit[u];
+            x.base = L.tile_base[t];
+            x.nsyn = L.tile_nsyn[t];
+            x.rng0 = L.tile_rng[t];
+            x.nrng = L.tile_rng[t + 1] - L.tile_rng[t];
+            x.part = u % L.parts;
+            x.pad[0] = x.pad[1] = 0;
+            res[u] = L.tile_res[t];
+        }
+        UP(unit, unit);
+        UP(tile_res, res);
+    }
+    d.nslots = L.nslots * L.parts;
     if (dev_syn) {
         d.syn = dev_syn;
     } else {
@@ -508,7 +528,6 @@ static bsim_sim *sim_from_layout(bsim::Layout &L, const bsim_sim_config &c, bsim
         std::vector<float>().swap(L.syn_w);
         UP(syn, packed);
     }
-    UP(tile_rng, L.tile_rng);
     UP(rng, L.rng);
     UP(off_tab, L.off_tab);
     UP(src_lo, L.src_lo);
@@ -523,7 +542,7 @@ static bsim_sim *sim_from_layout(bsim::Layout &L, const bsim_sim_config &c, bsim
 #undef UP
     {
         const size_t n = (size_t)(L.n > 0 ? L.n : 1);
-        const size_t nt = (size_t)(L.ntiles > 0 ? L.ntiles : 1);
+        const size_t nt = (size_t)(d.ntiles > 0 ? d.ntiles : 1);
         const size_t nw = (size_t)(d.nwords > 0 ? d.nwords : 1);
         if (!(d.ie = dev_alloc<float>(sim, n, e))) goto hip_fail;
         if (!(d.ii = dev_alloc<float>(sim, n, e))) goto hip_fail;
@@ -538,10 +557,10 @@ static bsim_sim *sim_from_layout(bsim::Layout &L, const bsim_sim_config &c, bsim
             goto hip_fail;
         {
             /* until the first ranking: the tiles of each residue in order */
-            std::vector<int32_t> perm((size_t)(L.nslots > 0 ? L.nslots : 1), -1);
+            std::vector<int32_t> perm((size_t)(d.nslots > 0 ? d.nslots : 1), -1);
             std::vector<int32_t> rank(8, 0);
-            for (int32_t t = 0; t < L.ntiles; t++) {
-                const int x = L.tile_res[t];
+            for (int32_t t = 0; t < d.ntiles; t++) {
+                const int x = res[t];
                 perm[(size_t)8 * rank[x]++ + x] = t;
             }
             d.perm = dev_upload(sim, perm, e);
@@ -915,8 +934,8 @@ int32_t bsim_sim_get_info(const bsim_sim *sim, bsim_sim_info *info)
 {
     if (!sim || !info) return fail(BSIM_E_ARG, "bad argument");
     info->n = sim->d.n;
-    info->tile = sim->d.tile;
-    info->ntiles = sim->d.ntiles;
+    info->tile = sim->tile;
+    info->ntiles = sim->ntiles;
     info->dmax = sim->d.dmax;
     info->s = sim->s;
     info->device_bytes = sim->device_bytes;

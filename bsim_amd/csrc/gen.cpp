@@ -429,7 +429,7 @@ int chains_size(const bsim_chain_params *p, int32_t count, int64_t *neurons, int
 int build_chains_layout(const bsim_chain_params *p, int32_t count, float dt, int32_t tile,
                         int32_t dmax, int64_t part_synapses, Layout &out, int32_t *first_ids,
                         std::string &err,
-                        const std::function<int(const Layout &, int64_t)> &upload)
+                        const std::function<int(const Layout &, int64_t)> &upload, int32_t parts)
 {
     out = Layout();
     /* per-part progress on stderr when BSIM_PROGRESS is set (large sweeps
@@ -471,7 +471,7 @@ int build_chains_layout(const bsim_chain_params *p, int32_t count, float dt, int
             return -1;
         }
         Layout pl;
-        if (build_layout(h, dt, tile, pl, err, dmax) != 0) return -1;
+        if (build_layout(h, dt, tile, pl, err, dmax, parts) != 0) return -1;
         part = bsim_network();          /* the host network is no longer needed */
         if (upload(pl, out.s) != 0) {
             err.clear();                /* the upload set the error message */

@@ -37,7 +37,7 @@ int chains_size(const bsim_chain_params *p, int32_t count, int64_t *neurons, int
 int build_chains_layout(const bsim_chain_params *p, int32_t count, float dt, int32_t tile,
                         int32_t dmax, int64_t part_synapses, Layout &out, int32_t *first_ids,
                         std::string &err,
-                        const std::function<int(const Layout &, int64_t)> &upload);
+                        const std::function<int(const Layout &, int64_t)> &upload, int32_t parts = 1);
 
 }  // namespace bsim
 

@@ -4,11 +4,10 @@
  * Neurons are numbered in creation order (the order BSim's CPU simulator
  * updates them and reports spikes in).  They are cut into tiles of TILE
  * consecutive neurons (TILE a multiple of BSIM_TILE_ALIGN = 64 * BSIM_NWAVE).
- * A tile is the unit of work of one workgroup: it receives the synapses whose
- * target lies in the tile and updates the tile's neurons.  Streaming
- * wavefront q (q < BSIM_NWAVE) owns part q of the tile, local targets
- * [q * TILE/BSIM_NWAVE, (q + 1) * TILE/BSIM_NWAVE), and within it lane l owns
- * the local targets congruent to l modulo 64.
+ * A tile has BSIM_NWAVE parts, part q its local targets [q * TILE/BSIM_NWAVE,
+ * (q + 1) * TILE/BSIM_NWAVE).  The work of one step workgroup, a unit, is a
+ * tile or one part of it: it receives the synapses whose target lies in the
+ * unit and updates the unit's neurons.
  *
  * Target groups: runs of up to 32 consecutive tiles with the same source
  * ranges (the pres with synapses into the tile, merged over gaps of at most
@@ -21,12 +20,15 @@
  * inside a row by tile and part keeps, for every target, the (pre, delay,
  * creation) order of its inputs; keeping a row's pieces for all tiles of the
  * group adjacent lets those tiles share cache lines.  Per group and source
- * range, the row table holds for each (pre, delay) row and each tile of the
- * group one aligned 16-byte vector (BSIM_NWAVE part starts, then the end of
- * the tile's sub-rows), offsets relative to the group's first synapse:
- * vector ((p - lo) * D + d - 1) * ntiles_in_group + k.  A tile's range
+ * range, the row table holds for each (pre, delay) row and each unit of the
+ * group the start of the row's sub-row into the unit, relative to the group's
+ * first synapse, at ((p - lo) * D + d - 1) * units_in_group + unit.  Sub-rows
+ * lie in the order of their entries, so each ends where the next entry
+ * starts; one entry more ends the group's last.  (One 16-byte vector of three
+ * part starts and the end per row and tile took four times the table's bytes:
+ * 3.9 against 1.0 GB for 650,000 neurons and 6.3e8 synapses.)  A tile's range
  * entries (bsim_range, one per source chunk of BSIM_CHUNK pres) point at its
- * vector of row (lo, 1) and give the vector stride per row.
+ * first entry of row (lo, 1) and give the entries per row.
  *
  * Workgroups are dispatched to the 8 XCDs round-robin; every group has an XCD
  * residue and its tiles run in workgroups of that residue, so that they share
@@ -45,9 +47,10 @@
 #include <stdint.h>
 
 #define BSIM_MAX_DELAY 63   /* history word: bits 1..D of a uint64 */
-#define BSIM_NWAVE 3                        /* streaming wavefronts per tile = target parts */
+#define BSIM_NWAVE 3                        /* target parts of a tile */
 #define BSIM_TILE_ALIGN (64 * BSIM_NWAVE)   /* parts of whole 64-lane wavefronts */
-#define BSIM_MAX_TILE (8 * BSIM_TILE_ALIGN) /* at most 8 accumulator slots per lane */
+#define BSIM_MAX_TILE (8 * BSIM_TILE_ALIGN)
+#define BSIM_MAX_UNIT 512                   /* most targets of a step workgroup */
 
 enum { BSIM_KIND_LIF = 0, BSIM_KIND_ARRAY = 1, BSIM_KIND_BERNOULLI = 2, BSIM_KIND_POISSON = 3 };
 
@@ -57,9 +60,19 @@ enum { BSIM_KIND_LIF = 0, BSIM_KIND_ARRAY = 1, BSIM_KIND_BERNOULLI = 2, BSIM_KIN
  * with u < tab[1 + j], or J - 1 when there is none. */
 #define BSIM_POISSON_MAX_RATE 1.0e6f
 
+/* A unit: the targets of one step workgroup -- a whole tile, or one part of
+ * it. */
+typedef struct __attribute__((aligned(32))) bsim_unit {
+    int64_t base;       /* first synapse of the tile's group */
+    uint32_t nsyn;      /* synapses of the group */
+    int32_t rng0, nrng; /* the tile's range entries */
+    int32_t part;       /* part of the tile (0 for a whole tile) */
+    int32_t pad[2];
+} bsim_unit;
+
 typedef struct bsim_range {
     int32_t lo, hi;     /* pre neurons [lo, hi) of one chunk of a source range of the tile */
-    int64_t off_base;   /* off_tab index of the tile's vector of row (lo, 1) */
+    int64_t off_base;   /* off_tab index of the tile's first entry of row (lo, 1) */
     int64_t lbase;      /* first entry of the chunk's active-row list in src_list */
     int32_t uid;        /* source chunk: index into src_* */
     uint32_t wrow;      /* expected deliveries of one active row into the tile, x 16 (host statistics) */
@@ -94,8 +107,8 @@ typedef struct __attribute__((aligned(16))) bsim_lifc {
 /* Kernel arguments (passed by value). */
 typedef struct bsim_dev {
     int32_t n;           /* neurons */
-    int32_t tile;        /* TILE */
-    int32_t ntiles;
+    int32_t tile;        /* targets per unit */
+    int32_t ntiles;      /* units */
     int32_t dmax;        /* D, 1..BSIM_MAX_DELAY */
     int32_t nwords;      /* (n + 63) / 64 */
     int32_t pad0;
@@ -121,13 +134,11 @@ typedef struct bsim_dev {
     /* synapses */
     int32_t nslots;             /* step workgroups (tiles placed by XCD residue) */
     int32_t pad3;
-    const int64_t *tile_base;   /* [ntiles] first synapse of the tile's group */
-    const uint32_t *tile_nsyn;  /* [ntiles] synapses of the tile's group */
-    const uint8_t *tile_res;    /* [ntiles] XCD residue of the tile's group */
+    const bsim_unit *unit;      /* [ntiles] */
+    const uint8_t *tile_res;    /* [ntiles] XCD residue of the unit's group */
     const bsim_syn *syn;        /* [S] target and weight of each synapse, group-major */
-    const int32_t *tile_rng;    /* [ntiles + 1] first source range of each tile */
     const bsim_range *rng;
-    const uint32_t *off_tab;    /* group row tables (16-byte aligned vectors) */
+    const uint32_t *off_tab;    /* group row tables */
     /* source chunks and their active-row lists: the distinct source ranges of
      * all tiles, cut into chunks of at most BSIM_CHUNK pres (a tile's range
      * entries are per chunk).  After the update of cycle t, list u holds the

@@ -135,11 +135,30 @@ static int reset_synapse(const HostNet &net, int64_t k, int32_t N, float dt, flo
     return 0;
 }
 
+int32_t default_parts(int64_t n, int32_t tile)
+{
+    /* A unit's rows cost the same whatever its targets are, so thirds of a tile
+     * do up to three times the row work, but each has a third of the passes and
+     * of every owner thread's adds.  Measured, us per cycle whole / in parts:
+     * TILE 768, 144 tiles of the stress network 1200 / 957 and 1000 tiles of a
+     * sweep 64 / 52; TILE 384, 130 tiles 18.2 / 12.9, 625 tiles 32.8 / 33.5 and
+     * 1950 tiles 52 / 84; TILE 192, 78 tiles 13.8 / 12.0, 169 tiles 16.1 / 19.9.
+     * So: always from TILE 576 up (a whole tile is three or more targets per
+     * owner thread), below that while the parts leave no more than about one
+     * workgroup per compute unit and 192 targets of the tile. */
+    const int64_t tiles = (n + tile - 1) / tile;
+    return tile >= 3 * BSIM_TILE_ALIGN || BSIM_NWAVE * tiles <= 256 * (tile / BSIM_TILE_ALIGN) ? BSIM_NWAVE : 1;
+}
+
 int build_layout(const HostNet &net, float dt, int32_t tile, Layout &L, std::string &err,
-                 int32_t dmax_min)
+                 int32_t dmax_min, int32_t parts)
 {
     const int32_t N = net.n();
     const int64_t S = net.s();
+    if (parts != 1 && parts != BSIM_NWAVE) {
+        err = "internal error: a tile is one unit or one per part";
+        return -1;
+    }
     if (tile <= 0 || tile % BSIM_TILE_ALIGN != 0 || tile > BSIM_MAX_TILE) {
         err = "tile size must be a positive multiple of " + std::to_string(BSIM_TILE_ALIGN) +
               " up to " + std::to_string(BSIM_MAX_TILE);
@@ -153,6 +172,7 @@ int build_layout(const HostNet &net, float dt, int32_t tile, Layout &L, std::str
     L.n = N;
     L.s = S;
     L.tile = tile;
+    L.parts = parts;
     L.ntiles = N > 0 ? (N + tile - 1) / tile : 0;
     L.ncls.assign(N, 0u);
     L.lifc.clear();
@@ -467,12 +487,11 @@ int build_layout(const HostNet &net, float dt, int32_t tile, Layout &L, std::str
         }
     }
     /* group row tables: per group and range, entry
-     * ((p - lo) * D + d - 1) * nk * RW + k * RW + q (RW = NW + 1) holds the
-     * start of part q of tile k's sub-rows of row (p, d), entry q = NW its
-     * end: one aligned 16-byte vector per tile and row.  Offsets relative to
-     * the group's first synapse. */
-    const int32_t RW = NW + 1;
-    static_assert(BSIM_NWAVE + 1 == 4, "a tile's row-table entry is one 16-byte vector");
+     * ((p - lo) * D + d - 1) * nk * parts + k * parts + q holds the start of
+     * tile k's sub-row of row (p, d) (parts == 1) or of its part q's, relative
+     * to the group's first synapse.  A group's synapses are stored in the
+     * order of its entries, so a sub-row ends where the next entry starts; one
+     * entry past the group's last range holds the end of its last sub-row. */
     std::vector<std::vector<int64_t>> gtab_base(NG);
     std::vector<int64_t> gtab_off((size_t)NG + 1, 0);
     for (int32_t g = 0; g < NG; g++) {
@@ -480,9 +499,9 @@ int build_layout(const HostNet &net, float dt, int32_t tile, Layout &L, std::str
         int64_t n = 0;
         for (const auto &r : trng[gstart[g]]) {
             gtab_base[g].push_back(n);
-            n += (int64_t)(r.hi - r.lo) * D * nk * RW;
+            n += (int64_t)(r.hi - r.lo) * D * nk * parts;
         }
-        gtab_off[g + 1] = gtab_off[g] + n;
+        gtab_off[g + 1] = gtab_off[g] + n + 1;
     }
     L.off_tab.assign((size_t)gtab_off[NG], 0u);
     std::vector<uint16_t> gtgt(S);
@@ -504,7 +523,7 @@ int build_layout(const HostNet &net, float dt, int32_t tile, Layout &L, std::str
                         const size_t e = (size_t)trng[t][ri].off_base +
                                          ((size_t)(p - r0.lo) * D + (size_t)(d - 1)) * NW;
                         for (int32_t q = 0; q < NW; q++) {
-                            gt[x++] = pos;
+                            if (q < parts) gt[x++] = pos;
                             const uint32_t a = toff[t][e + q], b = toff[t][e + q + 1];
                             for (uint32_t i = a; i < b; i++) {
                                 gtgt[gs + pos] = L.syn_tgt[L.tile_syn[t] + i];
@@ -512,9 +531,9 @@ int build_layout(const HostNet &net, float dt, int32_t tile, Layout &L, std::str
                                 pos++;
                             }
                         }
-                        gt[x++] = pos;
                     }
         }
+        tab[gtab_off[g + 1] - gtab_off[g] - 1] = pos;
     }
     L.syn_tgt.swap(gtgt);
     L.syn_w.swap(gw);
@@ -568,9 +587,9 @@ int build_layout(const HostNet &net, float dt, int32_t tile, Layout &L, std::str
                     bsim_range rc;
                     rc.lo = c;
                     rc.hi = std::min(r.hi, c + BSIM_CHUNK);
-                    rc.stride = (uint32_t)(nk * RW);
+                    rc.stride = (uint32_t)(nk * parts);
                     rc.off_base = gtab_off[g] + gtab_base[g][ri] +
-                                  (int64_t)(c - r.lo) * D * rc.stride + (int64_t)(t - k0) * RW;
+                                  (int64_t)(c - r.lo) * D * rc.stride + (int64_t)(t - k0) * parts;
                     rc.uid = u;
                     rc.lbase = L.src_list_base[(size_t)u];
                     rc.pad = 0;
@@ -613,7 +632,7 @@ int build_layout(const HostNet &net, float dt, int32_t tile, Layout &L, std::str
 
 int append_layout(Layout &A, Layout &B, std::string &err)
 {
-    if (A.ntiles > 0 && (A.tile != B.tile || A.dmax != B.dmax)) {
+    if (A.ntiles > 0 && (A.tile != B.tile || A.dmax != B.dmax || A.parts != B.parts)) {
         err = "append_layout: parts differ in tile size or delay ring depth";
         return -1;
     }

@@ -66,6 +66,7 @@ struct Layout {
     std::vector<float> syn_w;
     std::vector<int32_t> tile_rng;
     std::vector<bsim_range> rng;
+    int32_t parts = 1;                       /* step workgroups per tile (1 or BSIM_NWAVE) */
     std::vector<uint32_t> off_tab;
     std::vector<int32_t> src_lo, src_hi;     /* distinct source ranges */
     std::vector<int64_t> src_list_base;      /* list capacity (hi - lo) * D each */
@@ -95,11 +96,16 @@ int32_t default_tile(int32_t dmax);
 /* Largest round(delay / dt) over the synapses (at least 1). */
 int32_t max_delay_steps(const HostNet &net, float dt);
 
+/* Step workgroups (units) per tile for a network of n neurons in tiles of
+ * `tile`: 1, or BSIM_NWAVE, one per target part. */
+int32_t default_parts(int64_t n, int32_t tile);
+
 /* Returns 0 or a negative code with a message in err.  The delay ring is at
  * least dmax_min steps deep (a part of a larger layout uses the whole
- * network's depth). */
+ * network's depth).  parts: row-table entries per tile and row (1 or
+ * BSIM_NWAVE). */
 int build_layout(const HostNet &net, float dt, int32_t tile, Layout &out, std::string &err,
-                 int32_t dmax_min = 0);
+                 int32_t dmax_min = 0, int32_t parts = 1);
 
 /* Appends layout B -- built, with the same tile and delay ring depth, for a
  * network placed after A's neurons, with no synapse between the two -- to A:

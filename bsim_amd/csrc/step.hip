@@ -1,16 +1,16 @@
 /*
  * step.hip -- the simulation step on CDNA4 (gfx950).
  *
- * A cycle is two launches.  bsim_step_kernel: one workgroup of BSIM_NWAVE + 1
- * wavefronts per tile of TILE consecutive neurons (layout.h) performs
+ * A cycle is two launches.  bsim_step_kernel: one workgroup per unit of
+ * consecutive neurons (a tile or a third of one, layout.h) performs
  *
- *   (ii) phase (ii) of cycle t-1: every synapse into the tile whose pre fired
+ *   (ii) phase (ii) of cycle t-1: every synapse into the unit whose pre fired
  *        d cycles earlier adds its weight to the target's E or I accumulator,
  *        in the order the reference's CPU simulator applies them
  *        (src/net/Network.cpp:324-327, src/neuron/lif/LIFENeuron.cpp:52-61);
  *   (i)  the LIF_brian update of cycle t (src/neuron/lif/LIFENeuron.cpp:114-160),
  *        which consumes exactly those accumulators, the spike history update
- *        and the ordered compaction of the tile's fired / active neurons into
+ *        and the ordered compaction of the unit's fired / active neurons into
  *        64-bit words by wavefront ballot.
  *
  * bsim_rows_kernel then builds, for every source chunk, the list of its
@@ -18,32 +18,33 @@
  * receive from the chunk; one more workgroup ranks the tiles, heaviest first,
  * by the work the step launch recorded.
  *
- * Phase (ii) for a tile, in windows of up to RCAP rows of the concatenated
- * lists of its source chunks:
- *   stage   the producer wavefront (the last one) reads the list entries and
- *           the row-table entries of window i+1 -- the BSIM_NWAVE + 1 part
- *           boundaries of each row -- into LDS while the others stream window
- *           i; its loads stall no streaming wavefront;
- *   stream  streaming wavefront q walks the staged rows and streams its own
- *           part of each: the concatenated sub-rows form a stream of
- *           positions; per step of 256 positions the sub-rows (64 rows at a
- *           time in the lanes) write the synapse index of each of their
- *           positions into an LDS address list -- from TILE 384 up, 128 rows
- *           at a time write only their first position in the step and a bit
- *           of a position mask, from which each position finds its sub-row
- *           -- and lane i of group g loads position 64 g + i; the loads of
- *           step s+1 are in flight while step s is applied;
- *   apply   the owner of local target x is lane x mod 64 of wavefront q, which
- *           keeps x's E and I accumulators in registers.  For each 64-event
- *           group, the event in lane i sets bit i of its owner's mask by an
- *           LDS atomic OR (order-free); every lane walks its mask upwards --
- *           stream order -- and adds.  No two lanes touch one accumulator, so
- *           the sums need no atomics, no conflict rounds and no barriers
- *           between wavefronts; each wavefront then updates its own part.
- * Every accumulator thus receives its adds one at a time in stream order,
- * (pre, delay, creation) -- the creation order the host verified -- so the
- * sums are the reference's sequential fp32 sums, bit for bit.  The kernel is
- * instantiated for S = TILE / (64 * BSIM_NWAVE) accumulator slots per lane.
+ * Phase (ii) for a unit: the sub-rows of its active rows, in list order, form
+ * one stream of events, which the workgroup takes in passes of PASS = 1,024
+ * positions.  The NEV event wavefronts find each position's synapse and load
+ * it, and sort the pass by target, keeping stream order (event_wave); the NOWN
+ * owner wavefronts, whose threads hold the targets' E and I accumulators in
+ * registers, add a pass's events while the event wavefronts prepare the next
+ * (owner_wave).  Every accumulator thus receives its adds one at a time in
+ * stream order, (pre, delay, creation) -- the creation order the host
+ * verified -- so the sums are the reference's sequential fp32 sums, bit for
+ * bit, with no floating-point atomics.
+ *
+ * What bounds it: a unit is a chain of passes, each a chain of LDS round trips,
+ * a barrier and the synapse loads, so the launch is as long as its longest
+ * unit, or the units' time over the 512 workgroups that fit at a time (two per
+ * compute unit).  Where the parallelism of a unit comes from decides that: one
+ * wavefront per part that walked every row, expanded its own sub-rows and
+ * applied them by masks per 64 events took 3.8 us per 768 events; here the
+ * expansion and the sort of 1,024 events are spread over eight wavefronts,
+ * every row is expanded once and not once per part, and the sequential part,
+ * the adds, is left to the owners: 2 us.  Whole step launch, before and after:
+ * 330,000 neurons at ~100 Hz (3.1e6 events) 83 / 60 us, 110,000 at ~1,600 Hz
+ * with delays up to 50 steps (3.2e7 events) 3,408 / 927, 96 chains of 100 to
+ * 1,000 neurons (2.4e5 events) 46 / 30, 650,000 neurons at ~100 Hz (7e6
+ * events) 106 / 106.  Measured and not used: 4 event wavefronts (71, 1,930, 33,
+ * 121 us for the same, whole tiles), 16 (one workgroup per compute unit), LDS
+ * masks by target instead of ballots (70 against 60 us for the first), four
+ * wavefronts that each take the add of their own targets (71).
  *
  * Arithmetic: compiled with -ffp-contract=off (no FMA contraction) and
  * without denormal flushing, so V = ((Cm*V + v_tmp) + iE*C_E) + iI*C_I rounds
@@ -55,38 +56,31 @@
 #include "layout.h"
 
 #define WAVE 64
-#define NWAVE BSIM_NWAVE              /* streaming wavefronts = target quarters */
-#define NTHREAD (WAVE * (NWAVE + 1))  /* plus one producer wavefront */
-#define ROWW (NWAVE + 1)              /* uint32 per staged row: part starts and end */
-#define NGRP 4                        /* 64-position groups per streaming step */
-#define SSTEP (NGRP * WAVE)
+#define NEV 8                         /* event wavefronts of a step workgroup */
+#define NOWN 4                        /* owner wavefronts */
+#define NTHREAD (WAVE * (NEV + NOWN))
+#define NCOL 16                       /* groups of 64 events in a pass */
+#define PASS (NCOL * WAVE)
+#define NGRP (NCOL / NEV)             /* groups of an event wavefront */
+#define NO_MARK 0xFFFFFFFFu           /* no synapse index: a group has fewer than 2^32 - 1 */
 #define MAXR 128                      /* source ranges per batch */
 #define ROWS_THREADS 1024             /* row-list kernel: 4 pres per thread */
 #define HEAVY_WGS 256                 /* workgroups run at raised wave priority */
+#define STEP_EU 6                     /* wavefronts per SIMD: two workgroups per compute unit */
 static_assert(BSIM_CHUNK == 4 * ROWS_THREADS, "a source chunk is one row-list workgroup");
+static_assert(NCOL == 16 && NCOL % NEV == 0, "a target's histogram row is one 16-byte vector");
 
-#ifndef MARK_MIN_S
-#define MARK_MIN_S 2                  /* slots per lane from which sub-rows are expanded by marks */
-#endif
-static_assert(ROWW == 4 && NWAVE == 3, "a staged row is one 16-byte vector of 3 part starts and the end");
-
-/* Rows per staged window (RCAP): 384 at one accumulator slot per lane (TILE
- * 192, where LDS limits a CU to five workgroups), 512 from two slots up (four
- * workgroups per CU either way, bounded by registers), so that a heavy tile
- * passes fewer window barriers.  RPL rows per producer lane, RW words of
- * packed range indices. */
-template <int S_>
-struct Win {
-    static constexpr int RCAP = S_ >= 2 ? 512 : 384;
-    static constexpr int RPL = RCAP / WAVE;
-    static constexpr int RW = (RPL + 3) / 4;
-};
-
-/* LDS bytes of a workgroup: lbase, obase | stage | rows | tot | alist | cum | stride | omask | pmask */
-__host__ __device__ constexpr size_t lds_bytes(int rcap)
+/* Slots per target: a pass puts PASS / U events on a target of a unit of U on
+ * average, if full; three times that, at least 8. */
+__host__ __device__ constexpr uint32_t slots_of(uint32_t U)
 {
-    return 16 * MAXR + 8 * NWAVE * SSTEP + 4 * (2 * rcap * ROWW + 2 * NWAVE + NWAVE * SSTEP) +
-           4 * (MAXR + 2) + 4 * MAXR + 8 * NWAVE * NGRP * WAVE + 8 * NWAVE * NGRP;
+    return U >= 384 ? 8u : (3u * PASS / U) & ~3u;
+}
+
+/* LDS bytes of a workgroup: lbase, obase | hist | mark | slot | btot, cum, stride, most, last */
+__host__ __device__ constexpr size_t lds_bytes(uint32_t U)
+{
+    return 16 * MAXR + 2 * U * NCOL + 8 * PASS + 4 * slots_of(U) * U + 8 * NEV + 4 * (MAXR + 1) + 4 * MAXR + 16;
 }
 
 __device__ __forceinline__ uint32_t bern_hash(uint64_t seed, uint32_t id, uint32_t t)
@@ -127,19 +121,6 @@ __device__ __forceinline__ uint32_t readlane(uint32_t x, int32_t l)
 __device__ __forceinline__ uint32_t uniform(uint32_t x) { return __builtin_amdgcn_readfirstlane(x); }
 
 __device__ __forceinline__ uint32_t wave_index() { return uniform(threadIdx.x / WAVE); }
-
-/* s_waitcnt vmcnt(0) (GFX9 encoding: vmcnt 0, expcnt and lgkmcnt at their
- * maxima, i.e. not waited for): this wavefront's vector memory loads have
- * completed */
-__device__ __forceinline__ void wait_all_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
-
-/* orders this wavefront's LDS accesses (lanes exchange data through LDS) */
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 /* DPP controls (GFX9 encoding): shift right within a row of 16 lanes, and
  * broadcast lane 15 / 31 into the following rows */
@@ -186,167 +167,471 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x)
     return (uint32_t)v;
 }
 
+/* ---- delivery ------------------------------------------------------------- */
+
 struct Shared {
-    uint32_t *rows;      /* [2][RCAP][ROWW] part boundaries of the staged rows, double-buffered */
-    uint32_t *tot;       /* [2][NWAVE] stream length of each quarter in the window */
-    uint2 *stage;        /* [NWAVE][SSTEP] (local target in quarter, weight bits) */
-    uint64_t *omask;     /* [NWAVE][NGRP][WAVE] events of a group owned by each lane */
-    uint64_t *pmask;     /* [NWAVE][NGRP] step positions where a sub-row starts (mark expansion) */
-    uint32_t *alist;     /* [NWAVE][SSTEP] synapse index of each position of a step */
-    uint32_t *cum;       /* [MAXR + 1] rows before each source range of the batch */
-    uint32_t *stride;    /* [MAXR] row-table entries per row of each source range */
-    int64_t *lbase;      /* [MAXR] first list entry of each source range */
-    int64_t *obase;      /* [MAXR] row-table base of each source range */
+    uint64_t *lbase, *obase;    /* [MAXR] first list entry / table base of each source range of the batch */
+    uint32_t *cum;              /* [MAXR + 1] rows before each source range */
+    uint32_t *stride;           /* [MAXR] table entries per row */
+    uint32_t *mark;             /* [2][PASS] synapse index where a sub-row or group starts, else NO_MARK */
+    uint32_t *hist;             /* [2][U][NCOL / 4] events of each target per group, one byte each */
+    float *slot;                /* [K][U] a pass's weights of each target in stream order */
+    uint32_t *btot;             /* [2][NEV] stream length of each event wavefront's rows of a block */
+    uint32_t *most;             /* [2] largest rank of a pass's events beyond the slots */
+    uint32_t *last;             /* [2] the pass is the batch's last */
 };
 
-/* A window of 64 R staged rows in the lanes of a wavefront: lane j holds
- * rows rw + R j .. rw + R j + R - 1 of the wavefront's sub-row stream. */
-template <int R>
-struct RowWin {
-    int32_t rw;         /* first row (uniform) */
-    uint32_t pos[R];    /* stream position of each sub-row */
-    uint32_t len[R];    /* sub-row length */
-    uint32_t base[R];   /* synapse index of the sub-row minus pos */
-    uint32_t end;       /* stream position after the window (uniform) */
-};
-
-template <int R>
-__device__ __forceinline__ void load_win(const uint32_t *rows, RowWin<R> &W, int32_t rw, uint32_t pos0,
-                                         int32_t nrows)
+__device__ __forceinline__ uint64_t uniform64(uint64_t x)
 {
-    const uint32_t lane = threadIdx.x & (WAVE - 1);
-    const uint32_t q = wave_index();
-    uint32_t s0[R], sum = 0;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        const int32_t j = rw + R * (int32_t)lane + r;
-        uint32_t a = 0, c = 0;
-        if (j < nrows) {
-            if constexpr (R == 1) {
-                a = rows[j * ROWW + q];
-                c = rows[j * ROWW + q + 1];
-            } else {                      /* one 16-byte read per row */
-                const uint4 v = reinterpret_cast<const uint4 *>(rows)[j];
-                a = (q == 0) ? v.x : (q == 1) ? v.y : v.z;
-                c = (q == 0) ? v.y : (q == 1) ? v.z : v.w;
-            }
-        }
-        s0[r] = a;
-        W.len[r] = c - a;
-        sum += W.len[r];
-    }
-    const uint32_t incl = wave_incl_scan(sum);
-    uint32_t p = pos0 + incl - sum;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        W.pos[r] = p;
-        W.base[r] = s0[r] - p;
-        p += W.len[r];
-    }
-    W.rw = rw;
-    W.end = pos0 + readlane(incl, WAVE - 1);
+    return (uint64_t)uniform((uint32_t)x) | ((uint64_t)uniform((uint32_t)(x >> 32)) << 32);
 }
 
-/* Loaded events of one streaming step: NGRP groups of 64. */
-struct Step {
-    uint32_t tl[NGRP];
-    float w[NGRP];
-    bool v[NGRP];
+__device__ __forceinline__ void wg_barrier() { __syncthreads(); }
+
+/* A place in the concatenated active-row lists of a batch of source ranges
+ * (uniform): row j of the batch, in range ri, is list entry lb + j, and list
+ * entry e's table entry is ob + e * st. */
+struct Cursor {
+    int32_t ri;
+    uint32_t next;              /* first row of the range after ri */
+    uint64_t lb, ob;
+    uint32_t st;
 };
 
-/* Loads the events of stream positions [b, b + SSTEP) into lane i of group g
- * (position b + 64 g + i), sliding the row window over the staged rows as
- * needed.  Two ways to find each position's synapse index:
- *   R == 1  every sub-row that intersects the step writes the index of each
- *           of its positions into the wavefront's address list (one pass per
- *           four positions of the window's longest sub-row);
- *   R >= 2  (marks) every such sub-row writes only its first position in the
- *           step: its synapse base into the address list and a bit into the
- *           step's position mask; each position then takes the base of the
- *           last mark at or before it (the highest set mask bit below it).
- *           Costs one pass per window whatever the sub-row lengths.
- * The loads are issued unconditionally (lanes without an event read the
- * tile's first synapse), so that the compiler can count them exactly and the
- * apply of the previous step waits only for its own loads. */
-template <int R>
-__device__ __forceinline__ void load_step(const Shared &S, const uint32_t *rows, RowWin<R> &W, uint32_t b,
-                                          uint32_t tot, int32_t nrows, uint32_t nsyn,
-                                          const bsim_syn *syn, Step &st)
+__device__ __forceinline__ uint32_t range_end(const Shared &S, int32_t ri, int32_t nrb)
+{
+    return ri + 1 < nrb ? S.cum[ri + 1] : 0xFFFFFFFFu;
+}
+
+__device__ __forceinline__ void set_range(const Shared &S, Cursor &c, int32_t ri, int32_t nrb)
+{
+    c.ri = ri;
+    c.next = uniform(range_end(S, ri, nrb));
+    c.lb = uniform64(S.lbase[ri]) - (uint64_t)uniform(S.cum[ri]);
+    c.ob = uniform64(S.obase[ri]);
+    c.st = uniform(S.stride[ri]);
+}
+
+/* List entries of 64 rows (lane l: row l) and where their table entries lie. */
+struct Entries {
+    uint32_t e, st;
+    uint64_t ob;
+    uint32_t n;                 /* rows (uniform) */
+};
+
+/* Loads the list entries of the rows from j0 on.  They mostly lie in one
+ * range, whose values are then uniform. */
+__device__ __forceinline__ void load_entries(const Shared &S, const bsim_dev &d, Cursor &c, int32_t nrb,
+                                             uint32_t j0, uint32_t nrows, Entries &E)
+{
+    E.n = j0 < nrows ? min((uint32_t)WAVE, nrows - j0) : 0u;
+    if (E.n == 0) return;                                     /* uniform */
+    while (j0 >= c.next) set_range(S, c, c.ri + 1, nrb);
+    const uint32_t l = min((uint32_t)(threadIdx.x & (WAVE - 1)), E.n - 1u);
+    if (j0 + E.n <= c.next) {                                 /* uniform */
+        E.e = (d.src_list + (c.lb + j0))[l];
+        E.ob = c.ob;
+        E.st = c.st;
+    } else {
+        int32_t ri = c.ri;
+        uint32_t nx = c.next;
+        while (j0 + l >= nx) nx = range_end(S, ++ri, nrb);
+        E.e = d.src_list[S.lbase[ri] - (uint64_t)S.cum[ri] + (uint64_t)(j0 + l)];
+        E.ob = S.obase[ri];
+        E.st = S.stride[ri];
+    }
+}
+
+typedef uint32_t pair_u32 __attribute__((ext_vector_type(2), aligned(4)));
+
+/* Loads the rows' table entries: each sub-row's start and the start of the one
+ * after it. */
+__device__ __forceinline__ void load_rows(const bsim_dev &d, const Entries &E, pair_u32 &ab)
+{
+    if (E.n == 0) return;                                     /* uniform */
+    ab = *reinterpret_cast<const pair_u32 *>(d.off_tab + E.ob + (uint64_t)(E.e * E.st));
+}
+
+/* A block of NEV * 64 rows, one per thread of the event wavefronts: the row's
+ * sub-row into the unit as its first synapse, its length and its position in
+ * the batch's stream of events. */
+struct Block {
+    uint32_t a, len, pos;
+};
+
+/* The block's sub-rows from its table entries (n rows in this wavefront), with
+ * positions within the wavefront; the wavefront's stream length goes to btot. */
+__device__ __forceinline__ void make_block(const Shared &S, const pair_u32 &ab, uint32_t n, uint32_t buf, Block &k)
 {
     const uint32_t lane = threadIdx.x & (WAVE - 1);
-    const uint32_t q = wave_index();
-    uint32_t *al = S.alist + q * SSTEP;
-    uint64_t *pm = S.pmask + q * NGRP;
-    const uint32_t e = min(b + SSTEP, tot);
-    if (b < tot) {                                            /* uniform */
-        while (true) {
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                const uint32_t lo = max(W.pos[r], b), hi = min(W.pos[r] + W.len[r], e);
-                if constexpr (R == 1) {
-                    const uint32_t n = hi > lo ? hi - lo : 0u;
-                    const uint32_t a0 = W.base[r] + lo;
-                    uint32_t *dst = al + (lo - b);
-                    for (uint32_t x = 0; ballot64(x < n) != 0ull; x += 4) {
-                        if (x < n) dst[x] = a0 + x;
-                        if (x + 1 < n) dst[x + 1] = a0 + x + 1;
-                        if (x + 2 < n) dst[x + 2] = a0 + x + 2;
-                        if (x + 3 < n) dst[x + 3] = a0 + x + 3;
-                    }
-                } else if (hi > lo) {
-                    const uint32_t x = lo - b;
-                    al[x] = W.base[r];
-                    atomicOr((unsigned long long *)&pm[x / WAVE], 1ull << (x & (WAVE - 1)));
-                }
-            }
-            if (W.end >= e) break;                            /* uniform */
-            if (W.rw + R * WAVE >= nrows) break;
-            load_win<R>(rows, W, W.rw + R * WAVE, W.end, nrows);
-        }
+    k.a = ab.x;
+    k.len = lane < n ? ab.y - ab.x : 0u;
+    const uint32_t incl = wave_incl_scan(k.len);
+    k.pos = incl - k.len;
+    if (lane == WAVE - 1) S.btot[buf * NEV + wave_index()] = incl;
+}
+
+/* Positions in the batch's stream, once every wavefront has written btot: at is
+ * the stream's length so far (uniform), advanced past the block. */
+__device__ __forceinline__ void place_block(const Shared &S, uint32_t buf, Block &k, uint32_t &at)
+{
+    const uint32_t lane = threadIdx.x & (WAVE - 1);
+    const uint32_t incl = wave_incl_scan(lane < NEV ? S.btot[buf * NEV + lane] : 0u);
+    const uint32_t w = wave_index();
+    k.pos += at + (w > 0 ? readlane(incl, (int32_t)w - 1) : 0u);
+    at += readlane(incl, WAVE - 1);
+}
+
+/* The events of a pass, stream positions [b, e) with e - b <= PASS: event
+ * wavefront w takes the groups of 64 positions w, w + NEV, ...  Each sub-row
+ * marks its first position in the pass, and every multiple of 64 that it
+ * covers, with the synapse index there (put_marks); a position's synapse lies
+ * past the last mark at or before it in its group, the highest set bit of the
+ * group's ballot (load_events). */
+__device__ __forceinline__ void put_marks(uint32_t *mark, const Block &k, uint32_t b, uint32_t e)
+{
+    const uint32_t lo = max(k.pos, b), hi = min(k.pos + k.len, e);
+    if (hi > lo) {
+        const uint32_t x = lo - b, y = hi - b, a = k.a + (lo - k.pos);
+        mark[x] = a;
+        for (uint32_t g = (x | (WAVE - 1)) + 1u; g < y; g += WAVE) mark[g] = a + (g - x);
     }
-    wave_sync();
-    uint64_t M[NGRP];
-    if constexpr (R > 1) {
-#pragma unroll
-        for (int g = 0; g < NGRP; g++) M[g] = pm[g];
-        wave_sync();
-        if (lane < NGRP) pm[lane] = 0ull;
-    }
+}
+
+struct Step {
+    uint32_t tgt[NGRP];
+    float w[NGRP];
+};
+
+__device__ __forceinline__ void load_events(uint32_t *mark, const bsim_syn *syn, uint32_t nsyn, Step &st)
+{
+    const uint32_t lane = threadIdx.x & (WAVE - 1);
     const uint64_t le = ~0ull >> (WAVE - 1 - lane);           /* bits 0..lane */
-    uint32_t last = 0;          /* the step's position 0 is always marked */
+    uint32_t *mk = mark + wave_index() * WAVE + lane;
+    uint32_t v[NGRP], at[NGRP];
+#pragma unroll
+    for (int g = 0; g < NGRP; g++) v[g] = mk[g * NEV * WAVE];
+#pragma unroll
+    for (int g = 0; g < NGRP; g++) mk[g * NEV * WAVE] = NO_MARK;
 #pragma unroll
     for (int g = 0; g < NGRP; g++) {
-        const uint32_t pr = g * WAVE + lane;
-        const bool v = b + pr < e;
-        uint32_t addr;
-        if constexpr (R == 1) {
-            addr = v ? al[pr] : 0u;
-        } else {
-            const uint64_t mg = M[g] & le;
-            const uint32_t idx = mg ? (uint32_t)(g * WAVE + WAVE - 1 - __clzll(mg)) : last;
-            last = M[g] ? (uint32_t)(g * WAVE + WAVE - 1 - __clzll(M[g])) : last;
-            addr = v ? al[idx] + b + pr : 0u;
-        }
-        addr = (addr < nsyn) ? addr : 0u;
-        st.v[g] = v;
+        const uint64_t m = ballot64(v[g] != NO_MARK) & le;
+        at[g] = (WAVE - 1) - (uint32_t)__clzll((long long)(m | 1ull));
+    }
+#pragma unroll
+    for (int g = 0; g < NGRP; g++) v[g] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(at[g] * 4u), (int)v[g]);
+#pragma unroll
+    for (int g = 0; g < NGRP; g++) {
+        /* lanes past the pass's end load some synapse of the group */
+        uint32_t addr = v[g] + (lane - at[g]);
+        if (addr >= nsyn) addr = 0u;
         const bsim_syn sv = syn[addr];
-        st.tl[g] = sv.tgt;
+        st.tgt[g] = sv.tgt;
         st.w[g] = __uint_as_float(sv.w);
     }
-    wave_sync();
 }
 
-/* E and I accumulators of the S local targets lane, lane + 64, ... of the
- * wavefront's quarter */
+/* The lanes whose NB-bit value x equals this lane's, among the lanes in v. */
+template <int NB>
+__device__ __forceinline__ uint64_t same_lanes(uint32_t x, uint64_t v)
+{
+    const uint32_t nx = ~x;
+    uint32_t lo = (uint32_t)v, hi = (uint32_t)(v >> 32);
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        const int32_t z = __builtin_amdgcn_sbfe((int32_t)nx, b, 1);   /* 0 where the bit is set, else -1 */
+        const uint64_t B = ballot64(z == 0);
+        lo &= (uint32_t)B ^ (uint32_t)z;
+        hi &= (uint32_t)(B >> 32) ^ (uint32_t)z;
+    }
+    return (uint64_t)lo | ((uint64_t)hi << 32);
+}
+
+__device__ __forceinline__ uint32_t byte_sum(uint32_t x, uint32_t acc) { return __builtin_amdgcn_sad_u8(x, 0u, acc); }
+
+/* Event wavefronts: phase (ii) of one batch of nrows active rows.  A pass adds
+ * up to PASS events, in stream order, to their targets' accumulators:
+ *   count    per group of 64 events, a target's first event finds the others of
+ *            its target by ballots and stores how many there are in the group's
+ *            byte of the target's histogram row;
+ *   place    an event's rank among its target's events of the pass is the sum
+ *            of the bytes of the groups before its own plus the events of its
+ *            target in the lanes below; its weight goes to the target's slot
+ *            of that rank;
+ *   add      (owner wavefronts, while these count the next pass) every target's
+ *            owner adds its slots in order.
+ * A target with more events than slots takes further rounds of place and add.
+ * The loads run ahead of the passes: a pass's synapses are loaded during the
+ * pass before, the table entries and list entries one and two blocks ahead of
+ * the rows that the marks are put from. */
+template <int NB>
+__device__ void event_wave(const Shared &S, const bsim_dev &d, const bsim_unit &un, int32_t nrb, uint32_t nrows,
+                           uint32_t U, uint32_t K, uint32_t &par, const bsim_syn *syn, uint32_t &events)
+{
+    const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1), w = wave_index();
+    const uint32_t nsyn = un.nsyn, qoff = (uint32_t)un.part * U;
+    const uint64_t lt = (1ull << lane) - 1ull;
+    uint32_t jn = w * WAVE;                     /* first row of the next block to look up */
+    Cursor c;
+    set_range(S, c, 0, nrb);
+    Entries E;
+    pair_u32 ab = {0u, 0u};
+    Block k0, k1;                               /* blocks not yet used up */
+    uint32_t e0 = 0, e1 = 0, at = 0;            /* ends of k0, k1 and of the stream so far */
+    uint32_t q = 1, buf = 0;                    /* how many of k0, k1 are in use */
+    uint32_t left = nrows > NEV * WAVE ? nrows - NEV * WAVE : 0u;    /* rows past the blocks made */
+    Step X;
+    load_entries(S, d, c, nrb, jn, nrows, E);
+    uint32_t nab = E.n;
+    load_rows(d, E, ab);
+    load_entries(S, d, c, nrb, jn += NEV * WAVE, nrows, E);
+    make_block(S, ab, nab, 0u, k0);
+    nab = E.n;
+    load_rows(d, E, ab);
+    load_entries(S, d, c, nrb, jn += NEV * WAVE, nrows, E);
+    if (left > 0) {                                           /* uniform */
+        make_block(S, ab, nab, buf = 1u, k1);
+        nab = E.n;
+        load_rows(d, E, ab);
+        load_entries(S, d, c, nrb, jn += NEV * WAVE, nrows, E);
+        left = left > NEV * WAVE ? left - NEV * WAVE : 0u;
+        q = 2;
+    }
+    wg_barrier();
+    place_block(S, 0u, k0, at);
+    e0 = at;
+    if (q == 2) {
+        place_block(S, 1u, k1, at);
+        e1 = at;
+    }
+    uint32_t b = 0, n = min(at, (uint32_t)PASS);              /* the pass: n events from position b */
+    uint32_t *mark = S.mark;                                  /* the coming pass's marks */
+    put_marks(mark, k0, 0u, n);
+    if (q == 2) put_marks(mark, k1, 0u, n);
+    while (q > 0 && n >= e0) {
+        k0 = k1;
+        e0 = e1;
+        q--;
+    }
+    wg_barrier();
+    load_events(mark, syn, nsyn, X);
+    while (true) {
+        /* a wavefront may put the next pass's marks while another still reads this one's */
+        mark = mark == S.mark ? S.mark + PASS : S.mark;
+        uint32_t li[NGRP], rk[NGRP];
+        float wt[NGRP];
+#pragma unroll
+        for (int g = 0; g < NGRP; g++) {
+            li[g] = X.tgt[g] - qoff;
+            wt[g] = X.w[g];
+        }
+        /* the next pass and the block after the ones in use.  No load is in
+         * flight here, and the conditional ones follow one another without a
+         * wait in between: the wait counter is in order, and the compiler
+         * waits for every load that it cannot count */
+        const uint32_t nb = b + n;
+        const uint32_t nn = min((q == 2 ? e1 : q == 1 ? e0 : nb) - nb, (uint32_t)PASS);
+        if (q > 0) put_marks(mark, k0, nb, nb + nn);
+        if (q > 1) put_marks(mark, k1, nb, nb + nn);
+        while (q > 0 && nb + nn >= e0) {
+            k0 = k1;
+            e0 = e1;
+            q--;
+        }
+        const bool more = q < 2 && left > 0;
+        Block kn;
+        if (more) {
+            make_block(S, ab, nab, buf ^= 1u, kn);
+            nab = E.n;
+            load_rows(d, E, ab);
+            load_entries(S, d, c, nrb, jn += NEV * WAVE, nrows, E);
+            left = left > NEV * WAVE ? left - NEV * WAVE : 0u;
+        }
+        uint32_t *hist = S.hist + par * (U * (NCOL / 4));
+#pragma unroll
+        for (int g = 0; g < NGRP; g++) {
+            const uint32_t col = w + g * NEV;                 /* uniform */
+            rk[g] = 0u;
+            if (col * WAVE < n) {                             /* uniform */
+                const bool v = col * WAVE + lane < n;
+                if (!v) li[g] = 0u;
+                const uint64_t m = same_lanes<NB>(li[g], ballot64(v));
+                rk[g] = (uint32_t)__popcll(m & lt);
+                if (v && rk[g] == 0u)
+                    reinterpret_cast<uint8_t *>(hist)[li[g] * NCOL + col] = (uint8_t)__popcll(m);
+            }
+        }
+        wg_barrier();
+        if (more) {
+            place_block(S, buf, kn, at);
+            if (q == 0) {
+                k0 = kn;
+                e0 = at;
+            } else {
+                k1 = kn;
+                e1 = at;
+            }
+            q++;
+        }
+        const bool done = nn == 0 && q == 0 && left == 0;     /* uniform */
+        if (!done) load_events(mark, syn, nsyn, X);
+        uint32_t over = 0u;             /* largest rank beyond the slots */
+#pragma unroll
+        for (int g = 0; g < NGRP; g++) {
+            const uint32_t col = w + g * NEV;                 /* uniform */
+            if (col * WAVE < n) {                             /* uniform */
+                const bool v = col * WAVE + lane < n;
+                const uint4 h = reinterpret_cast<const uint4 *>(hist)[li[g]];
+                const uint32_t x = col / 4, mask = (1u << (8u * (col % 4))) - 1u;
+                uint32_t r = rk[g];
+                r = byte_sum(h.x & (x > 0 ? ~0u : mask), r);
+                r = byte_sum(h.y & (x > 1 ? ~0u : x == 1 ? mask : 0u), r);
+                r = byte_sum(h.z & (x > 2 ? ~0u : x == 2 ? mask : 0u), r);
+                r = byte_sum(h.w & (x == 3 ? mask : 0u), r);
+                rk[g] = r;
+                if (v && r < K) S.slot[r * U + li[g]] = wt[g];
+                if (v && r >= K) over = max(over, r);
+            }
+        }
+        if (over) atomicMax(&S.most[par], over);
+        if (tid == 0) {
+            S.most[par ^ 1u] = 0u;
+            S.last[par] = done ? 1u : 0u;
+        }
+        wg_barrier();
+        for (uint32_t r0 = K, most = uniform(S.most[par]); most >= r0; r0 += K) {
+            wg_barrier();
+#pragma unroll
+            for (int g = 0; g < NGRP; g++)
+                if ((w + g * NEV) * WAVE + lane < n && rk[g] - r0 < K)
+                    S.slot[(rk[g] - r0) * U + li[g]] = wt[g];
+            wg_barrier();
+        }
+        par ^= 1u;
+        if (done) break;
+        b = nb;
+        n = nn;
+    }
+    events += at;
+}
+
+/* E and I accumulators of an owner thread's targets: o, o + NOWN * 64, ... of
+ * the unit, o its index among the owner threads. */
 template <int S_>
 struct Acc {
     float e[S_], i[S_];
 };
 
-/* The state of a streaming wavefront's neurons that phase (i) reads, loaded
+/* Owner wavefronts: the passes of one batch. */
+template <int S_>
+__device__ void owner_wave(const Shared &S, uint32_t U, uint32_t K, uint32_t &par, Acc<S_> &acc)
+{
+    const uint32_t o = threadIdx.x - NEV * WAVE;
+    wg_barrier();
+    wg_barrier();
+    while (true) {
+        wg_barrier();
+        wg_barrier();
+        const uint32_t most = uniform(S.most[par]), last = uniform(S.last[par]);
+        uint32_t *hist = S.hist + par * (U * (NCOL / 4));
+        uint32_t tot[S_];
+        for (uint32_t r0 = 0;; r0 += K) {
+#pragma unroll
+            for (int j = 0; j < S_; j++) {
+                const uint32_t i = o + j * (NOWN * WAVE);
+                if (uniform(i) >= U) continue;                /* U is whole wavefronts */
+                /* a slot past the target's events counts as 0: the sums, which
+                 * start at +0 and never become -0, do not change by it */
+                const float *sl = S.slot + i;
+                float x[4];
+#pragma unroll
+                for (uint32_t y = 0; y < 4; y++) x[y] = sl[y * U];
+                if (r0 == 0) {                                /* uniform */
+                    const uint4 h = reinterpret_cast<const uint4 *>(hist)[i];
+                    reinterpret_cast<uint4 *>(hist)[i] = make_uint4(0u, 0u, 0u, 0u);
+                    tot[j] = byte_sum(h.x, byte_sum(h.y, byte_sum(h.z, byte_sum(h.w, 0u))));
+                }
+                const uint32_t n = min(tot[j] > r0 ? tot[j] - r0 : 0u, K);
+                uint32_t r = 0;
+                while (true) {
+                    float z[4];
+#pragma unroll
+                    for (uint32_t y = 0; y < 4; y++) z[y] = x[y];
+                    const bool go = ballot64(r + 4 < n) != 0ull;              /* uniform; then r + 4 < K */
+                    if (go) {
+#pragma unroll
+                        for (uint32_t y = 0; y < 4; y++) x[y] = sl[(r + 4 + y) * U];
+                    }
+#pragma unroll
+                    for (uint32_t y = 0; y < 4; y++) {
+                        const float a = r + y < n ? z[y] : 0.0f;
+                        acc.e[j] += a >= 0.0f ? a : 0.0f;
+                        acc.i[j] += a >= 0.0f ? 0.0f : a;
+                    }
+                    if (!go) break;
+                    r += 4;
+                }
+            }
+            if (most < r0 + K) break;                         /* uniform */
+            wg_barrier();
+            wg_barrier();
+        }
+        par ^= 1u;
+        if (last) break;
+    }
+}
+
+/* Phase (ii) of one batch of up to MAXR source ranges of the unit. */
+template <int NB, int S_>
+__device__ void deliver_batch(const Shared &S, const bsim_dev &d, const bsim_unit &un, int32_t r0, int32_t nrb,
+                              uint32_t U, uint32_t K, uint32_t &par, const bsim_syn *syn,
+                              uint32_t &events, uint32_t &rows, Acc<S_> &acc)
+{
+    const uint32_t tid = threadIdx.x;
+    const uint32_t w = wave_index();
+    if (w == 0) {
+        /* range metadata and the cumulative row counts of the batch */
+        constexpr int PER = MAXR / WAVE;
+        uint32_t c[PER], sum = 0;
+#pragma unroll
+        for (int x = 0; x < PER; x++) {
+            const int32_t i = (int32_t)tid * PER + x;
+            c[x] = 0u;
+            if (i < nrb) {
+                const bsim_range r = d.rng[r0 + i];
+                c[x] = d.rng_count[r0 + i];
+                S.lbase[i] = (uint64_t)r.lbase;
+                S.obase[i] = (uint64_t)r.off_base + (uint64_t)un.part;
+                S.stride[i] = r.stride;
+            }
+            sum += c[x];
+        }
+        const uint32_t incl = wave_incl_scan(sum);
+        uint32_t run = incl - sum;
+#pragma unroll
+        for (int x = 0; x < PER; x++) {
+            const int32_t i = (int32_t)tid * PER + x;
+            if (i < nrb) S.cum[i] = run;
+            run += c[x];
+        }
+        if (tid == WAVE - 1) S.cum[nrb] = incl;
+    }
+    wg_barrier();
+    const uint32_t nrows = uniform(S.cum[nrb]);
+    rows += nrows;
+    if (nrows > 0) {                                          /* uniform */
+        if (w < NEV)
+            event_wave<NB>(S, d, un, nrb, nrows, U, K, par, syn, events);
+        else
+            owner_wave<S_>(S, U, K, par, acc);
+    }
+    wg_barrier();               /* the next batch writes the range metadata */
+}
+
+/* The state of an owner thread's neurons that phase (i) reads, loaded
  * before phase (ii) so that its latency is hidden behind the delivery (no
  * other workgroup writes these words during the launch: a neuron belongs to
- * one tile, and the history words read are the previous cycle's copy).  Kept
+ * one unit, and the history words read are the previous cycle's copy).  Kept
  * in registers up to PREFETCH_MAX_S slots per lane. */
 #ifndef PREFETCH_MAX_S
 #define PREFETCH_MAX_S 1
@@ -363,10 +648,9 @@ template <int S_>
 __device__ __forceinline__ void load_nstate(const bsim_dev &d, int32_t base, const uint64_t *hist_in,
                                             NState<S_> &ns)
 {
-    const int32_t lane = (int32_t)(threadIdx.x & (WAVE - 1));
 #pragma unroll
     for (int j = 0; j < S_; j++) {
-        const int32_t nid = base + j * WAVE + lane;
+        const int32_t nid = base + j * (NOWN * WAVE) + (int32_t)threadIdx.x - NEV * WAVE;
         const bool valid = nid < d.n;
         const int32_t x = valid ? nid : 0;
         ns.cls[j] = d.ncls[x];
@@ -379,289 +663,8 @@ __device__ __forceinline__ void load_nstate(const bsim_dev &d, int32_t base, con
     }
 }
 
-/* Adds one owned event to the accumulator of its slot (E if w >= 0, else I)
- * when `valid`.  Written as selects over statically indexed accumulators, so
- * that they stay in registers for every S_ and no branch separates the staged
- * reads of a round. */
-template <int S_>
-__device__ __forceinline__ void add_event(Acc<S_> &acc, uint2 ev, bool valid)
-{
-    const float x = __uint_as_float(ev.y);
-    const uint32_t slot = ev.x >> 6;
-    const bool exc = x >= 0.0f;
-#pragma unroll
-    for (int j = 0; j < S_; j++) {
-        /* with one slot per lane an owned event's local target is below 64:
-         * its slot is 0 and needs no test */
-        const bool mine = valid && (S_ == 1 || slot == (uint32_t)j);
-        const float ae = acc.e[j] + x, ai = acc.i[j] + x;
-        acc.e[j] = (mine && exc) ? ae : acc.e[j];
-        acc.i[j] = (mine && !exc) ? ai : acc.i[j];
-    }
-}
-
-/* Applies one streaming step: every lane applies, in stream order, the events
- * whose target it owns.  For each group, the event in lane i sets bit i of its
- * owner's mask with an LDS atomic OR (order-free); the owner walks its mask
- * upwards, i.e. in stream order. */
-template <int S_>
-__device__ __forceinline__ void apply_step(const Shared &S, const Step &st, uint32_t qbase, Acc<S_> &acc)
-{
-    const uint32_t lane = threadIdx.x & (WAVE - 1);
-    const uint32_t q = wave_index();
-    uint2 *stg = S.stage + q * SSTEP;
-    uint64_t *om = S.omask + q * (NGRP * WAVE);
-    const uint64_t mybit = 1ull << lane;
-#pragma unroll
-    for (int g = 0; g < NGRP; g++) {
-        const uint32_t li = st.tl[g] - qbase;     /* local target within the quarter */
-        stg[g * WAVE + lane] = make_uint2(li, __float_as_uint(st.w[g]));
-        if (st.v[g]) atomicOr((unsigned long long *)&om[g * WAVE + (li & (WAVE - 1))], (unsigned long long)mybit);
-    }
-    wave_sync();
-    uint64_t M[NGRP];
-#pragma unroll
-    for (int g = 0; g < NGRP; g++) {
-        M[g] = om[g * WAVE + lane];
-        om[g * WAVE + lane] = 0ull;
-    }
-#pragma unroll
-    for (int g = 0; g < NGRP; g++) {
-        uint64_t m = M[g];
-        while (m) {
-            /* up to 2 owned events per round: their staged reads are issued
-             * together, the adds stay in stream order */
-            const uint32_t i0 = (uint32_t)__builtin_ctzll(m);
-            m &= m - 1;
-            uint32_t i1 = i0;
-            const bool h1 = m != 0ull;
-            if (h1) { i1 = (uint32_t)__builtin_ctzll(m); m &= m - 1; }
-            const uint2 e0 = stg[g * WAVE + i0];
-            const uint2 e1 = stg[g * WAVE + i1];
-            add_event<S_>(acc, e0, true);
-            add_event<S_>(acc, e1, h1);
-        }
-    }
-    wave_sync();
-}
-
-/* Streams this wavefront's quarter of the staged rows [0, nrows).  The loads
- * of step s+1 are in flight while step s is applied.  No load is issued past
- * the last step: a load left in flight at the end of the stream would still be
- * pending when the next window starts (the workgroup barrier waits for LDS
- * only), and its destination registers, reused there, would make the compiler
- * wait for every load in flight at the top of each step -- the step pipeline
- * would then hold one step's loads at a time. */
-template <int S_>
-__device__ void stream_rows(const Shared &S, const uint32_t *rows, int32_t nrows, uint32_t tot,
-                            uint32_t qbase, uint32_t nsyn, const bsim_syn *syn,
-                            Acc<S_> &acc)
-{
-    if (tot == 0) return;                                     /* uniform */
-    constexpr int R = (S_ >= MARK_MIN_S) ? 2 : 1;
-    RowWin<R> W;
-    load_win<R>(rows, W, 0, 0, nrows);
-    Step A, B;
-    load_step(S, rows, W, 0, tot, nrows, nsyn, syn, A);
-    uint32_t b = 0;
-    while (true) {
-        if (b + SSTEP >= tot) {                               /* uniform: A is the last step */
-            apply_step<S_>(S, A, qbase, acc);
-            break;
-        }
-        load_step(S, rows, W, b + SSTEP, tot, nrows, nsyn, syn, B);
-        apply_step<S_>(S, A, qbase, acc);
-        b += SSTEP;
-        if (b + SSTEP >= tot) {                               /* uniform: B is the last step */
-            apply_step<S_>(S, B, qbase, acc);
-            break;
-        }
-        load_step(S, rows, W, b + SSTEP, tot, nrows, nsyn, syn, A);
-        apply_step<S_>(S, B, qbase, acc);
-        b += SSTEP;
-    }
-}
-
-/* ---- the producer wavefront: staging of row windows ---------------------- */
-
-/* Row j of a window of the current range batch belongs to the source range
- * whose cumulative row interval holds it: the largest i with cum[i] <= j
- * (ranges without active rows repeat the count and are passed over). */
-__device__ __forceinline__ int32_t range_of(const Shared &S, uint32_t j, int32_t nrb)
-{
-    int32_t a = 0, b = nrb - 1;
-    while (a < b) {
-        const int32_t m = (a + b + 1) >> 1;
-        if (S.cum[m] <= j) a = m; else b = m - 1;
-    }
-    return a;
-}
-
-/* The source range index of each of a lane's rows (< MAXR = 128) is found
- * once per window, when its list entries are read, and kept packed four to a
- * register (RW words) until the window is staged. */
-static_assert(MAXR <= 256, "range indices are packed in bytes");
-template <int RW>
-__device__ __forceinline__ int32_t range_at(const uint32_t (&R)[RW], int x)
-{
-    return (int32_t)((R[x / 4] >> (8 * (x % 4))) & 0xFFu);
-}
-
-/* Active-row list entries of window `win` (lane holds rows lane + 64 x) and
- * the source range of each row (R).  The rows of a lane ascend from window
- * to window, so their ranges are found by walking forward from the range of
- * the lane's last row in the previous window (ri, carried by the caller; a
- * search for the first window). */
-template <int RCAP, int RPL = RCAP / WAVE, int RW = (RPL + 3) / 4>
-__device__ __forceinline__ void prod_entries(const Shared &S, const bsim_dev &d, int32_t win,
-                                             uint32_t nrows_tot, int32_t nrb, uint32_t (&E)[RPL],
-                                             uint32_t (&R)[RW], int32_t &ri)
-{
-    const uint32_t lane = threadIdx.x & (WAVE - 1);
-    if (win == 0) ri = range_of(S, lane, nrb);
-#pragma unroll
-    for (int w = 0; w < RW; w++) R[w] = 0u;
-#pragma unroll
-    for (int x = 0; x < RPL; x++) {
-        const uint32_t j = (uint32_t)win * RCAP + lane + WAVE * x;
-        E[x] = 0u;
-        if (j < nrows_tot) {
-            while (ri + 1 < nrb && S.cum[ri + 1] <= j) ri++;
-            E[x] = d.src_list[S.lbase[ri] + (j - S.cum[ri])];
-        }
-        R[x / 4] |= (uint32_t)ri << (8 * (x % 4));      /* ri < nrb <= MAXR */
-    }
-}
-
-/* Stages window `win` into LDS buffer `buf`: the row-table entry of each of
- * its rows (from the list entries E) -- the part starts and the end of the
- * tile's sub-rows, one aligned 16-byte load -- and the stream length of each
- * part.  The rows of a lane ascend, so their source range is found by walking
- * forward.  Every lane uses all of its E and Tb registers, including those of
- * rows past the window's end (zeros; the slots of the buffer they fill are
- * never read), so that no load of the producer is still pending, as far as
- * the compiler can tell, when the registers are reused by the streaming code
- * that shares the program. */
-template <int RCAP, int RPL = RCAP / WAVE, int RW = (RPL + 3) / 4>
-__device__ __forceinline__ void prod_stage(const Shared &S, const bsim_dev &d, int32_t buf, int32_t win,
-                                           uint32_t nrows_tot, const uint32_t (&E)[RPL],
-                                           const uint32_t (&R)[RW])
-{
-    const uint32_t lane = threadIdx.x & (WAVE - 1);
-    uint4 *rows = reinterpret_cast<uint4 *>(S.rows + buf * (RCAP * ROWW));
-    uint4 Tb[RPL];
-#pragma unroll
-    for (int x = 0; x < RPL; x++) {
-        const uint32_t j = (uint32_t)win * RCAP + lane + WAVE * x;
-        const int32_t ri = range_at<RW>(R, x);
-        const int64_t e0 = S.obase[ri] + (int64_t)E[x] * S.stride[ri];
-        Tb[x] = make_uint4(0u, 0u, 0u, 0u);
-        if (j < nrows_tot) Tb[x] = *reinterpret_cast<const uint4 *>(d.off_tab + e0);
-    }
-    uint32_t ql[NWAVE];
-#pragma unroll
-    for (int q = 0; q < NWAVE; q++) ql[q] = 0u;
-#pragma unroll
-    for (int x = 0; x < RPL; x++) {
-        const uint32_t jj = lane + WAVE * x;
-        rows[jj] = Tb[x];
-        ql[0] += Tb[x].y - Tb[x].x;
-        ql[1] += Tb[x].z - Tb[x].y;
-        ql[2] += Tb[x].w - Tb[x].z;
-    }
-#pragma unroll
-    for (int q = 0; q < NWAVE; q++) {
-        const uint32_t sum = readlane(wave_incl_scan(ql[q]), WAVE - 1);
-        if (lane == 0) S.tot[buf * NWAVE + q] = sum;
-    }
-}
-
-/* Phase (ii) of one batch of up to MAXR source ranges of the tile: wavefront
- * NWAVE stages window i+1 of the concatenated active-row lists while
- * wavefronts 0..NWAVE-1 stream window i. */
-template <int S_>
-__device__ void deliver_batch(const Shared &S, const bsim_dev &d, int32_t r0, int32_t nrb,
-                              uint32_t qbase, uint32_t nsyn, const bsim_syn *syn,
-                              int64_t &events, uint32_t &rows, Acc<S_> &acc)
-{
-    const uint32_t lane = threadIdx.x & (WAVE - 1);
-    const uint32_t w = wave_index();
-    const bool prod = w == NWAVE;
-    if (prod) {
-        /* range metadata and the cumulative row counts of the batch */
-        uint32_t c[MAXR / WAVE];
-#pragma unroll
-        for (int x = 0; x < MAXR / WAVE; x++) {
-            const int32_t i = (int32_t)lane * (MAXR / WAVE) + x;
-            c[x] = 0u;
-            if (i < nrb) {
-                const bsim_range r = d.rng[r0 + i];
-                c[x] = d.rng_count[r0 + i];
-                S.lbase[i] = r.lbase;
-                S.obase[i] = r.off_base;
-                S.stride[i] = r.stride;
-            }
-        }
-        uint32_t sum = 0;
-#pragma unroll
-        for (int x = 0; x < MAXR / WAVE; x++) sum += c[x];
-        const uint32_t incl = wave_incl_scan(sum);
-        uint32_t run = incl - sum;
-#pragma unroll
-        for (int x = 0; x < MAXR / WAVE; x++) {
-            const int32_t i = (int32_t)lane * (MAXR / WAVE) + x;
-            if (i < nrb) S.cum[i] = run;
-            run += c[x];
-        }
-        if (lane == WAVE - 1) S.cum[nrb] = incl;
-    }
-    __syncthreads();
-    constexpr int RCAP = Win<S_>::RCAP, RPL = Win<S_>::RPL, RW = Win<S_>::RW;
-    const uint32_t nrows_tot = uniform(S.cum[nrb]);
-    rows += nrows_tot;
-    const int32_t nwin = (int32_t)((nrows_tot + RCAP - 1) / RCAP);
-    if (nwin == 0) return;                                    /* uniform */
-    /* The producer issues the list entries of the window after next (En)
-     * before it stages the next one (from E), and ends each turn with all of
-     * its loads complete: the staging waits for its row-table loads, issued
-     * after those entries, so the wait costs nothing, and the compiler, which
-     * sees one program for all wavefronts, then knows that no load of the
-     * producer is pending in the streaming code (otherwise it makes the
-     * streaming wavefronts wait for loads that only the producer issued). */
-    uint32_t E[RPL], En[RPL];
-    uint32_t R[RW], Rn[RW];
-    int32_t ri = 0;
-    if (prod) {
-        prod_entries<RCAP>(S, d, 0, nrows_tot, nrb, E, R, ri);
-        if (nwin > 1) prod_entries<RCAP>(S, d, 1, nrows_tot, nrb, En, Rn, ri);
-        prod_stage<RCAP>(S, d, 0, 0, nrows_tot, E, R);
-        wait_all_loads();
-    }
-    __syncthreads();
-    for (int32_t i = 0; i < nwin; i++) {
-        const int32_t buf = i & 1;
-        if (prod) {
-            if (i + 1 < nwin) {
-#pragma unroll
-                for (int x = 0; x < RPL; x++) E[x] = En[x];
-#pragma unroll
-                for (int x = 0; x < RW; x++) R[x] = Rn[x];
-                if (i + 2 < nwin) prod_entries<RCAP>(S, d, i + 2, nrows_tot, nrb, En, Rn, ri);
-                prod_stage<RCAP>(S, d, buf ^ 1, i + 1, nrows_tot, E, R);
-            }
-            wait_all_loads();
-        } else {
-            const int32_t nrows = (int32_t)min((uint32_t)RCAP, nrows_tot - (uint32_t)i * RCAP);
-            const uint32_t qtot = uniform(S.tot[buf * NWAVE + w]);
-            events += qtot;
-            stream_rows<S_>(S, S.rows + buf * (RCAP * ROWW), nrows, qtot, qbase, nsyn, syn, acc);
-        }
-        __syncthreads();
-    }
-}
-
-template <int S_>
-__global__ __launch_bounds__(NTHREAD) void bsim_step_kernel(bsim_dev d, int32_t t, int32_t flags)
+template <int NB, int S_>
+__global__ __launch_bounds__(NTHREAD, STEP_EU) void bsim_step_kernel(bsim_dev d, int32_t t, int32_t flags)
 {
     extern __shared__ __align__(16) uint32_t lds[];
     const bool clocked = t < 0;
@@ -673,27 +676,24 @@ __global__ __launch_bounds__(NTHREAD) void bsim_step_kernel(bsim_dev d, int32_t 
      * wavefronts get issue priority on their compute unit, so that they are
      * not slowed down by the light tiles that fill the unit around them */
     if (blockIdx.x < HEAVY_WGS) __builtin_amdgcn_s_setprio(3);
-    const int32_t T = d.tile;
+    const uint32_t U = (uint32_t)d.tile, K = slots_of(U);
     const int32_t k = d.perm[blockIdx.x];       /* -1: an empty slot */
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & (WAVE - 1);
     const uint32_t w = wave_index();
-    const uint32_t qbase = w * ((uint32_t)T / NWAVE);
 
     Shared S;
     {
-        int64_t *p8 = reinterpret_cast<int64_t *>(lds);
-        S.lbase = p8;                                 p8 += MAXR;
-        S.obase = p8;                                 p8 += MAXR;
-        S.stage = reinterpret_cast<uint2 *>(p8);
-        uint32_t *p = reinterpret_cast<uint32_t *>(p8) + NWAVE * SSTEP * 2;
-        S.rows = p;                                   p += 2 * Win<S_>::RCAP * ROWW;
-        S.tot = p;                                    p += 2 * NWAVE;
-        S.alist = p;                                  p += NWAVE * SSTEP;
-        S.cum = p;                                    p += MAXR + 2;
-        S.stride = p;                                 p += MAXR;
-        S.omask = reinterpret_cast<uint64_t *>(p);    /* 8-byte aligned: see lds_bytes */
-        S.pmask = S.omask + NWAVE * NGRP * WAVE;
+        S.lbase = reinterpret_cast<uint64_t *>(lds);
+        S.obase = S.lbase + MAXR;
+        S.hist = reinterpret_cast<uint32_t *>(S.obase + MAXR);
+        S.mark = S.hist + 2 * U * (NCOL / 4);
+        S.slot = reinterpret_cast<float *>(S.mark + 2 * PASS);
+        S.btot = reinterpret_cast<uint32_t *>(S.slot + K * U);
+        S.cum = S.btot + 2 * NEV;
+        S.stride = S.cum + MAXR + 1;
+        S.most = S.stride + MAXR;
+        S.last = S.most + 2;
     }
 
     Acc<S_> acc;
@@ -702,52 +702,51 @@ __global__ __launch_bounds__(NTHREAD) void bsim_step_kernel(bsim_dev d, int32_t 
         acc.e[j] = 0.0f;
         acc.i[j] = 0.0f;
     }
-    if (w < NWAVE) {
-#pragma unroll
-        for (int g = 0; g < NGRP; g++) S.omask[(w * NGRP + g) * WAVE + lane] = 0ull;
-        if (lane < NGRP) S.pmask[w * NGRP + lane] = 0ull;
-    }
 
     constexpr bool PRE = S_ <= PREFETCH_MAX_S;
     NState<PRE ? S_ : 1> ns;
     if constexpr (PRE) {
-        if ((flags & 2) && w < NWAVE && k >= 0)
-            load_nstate<S_>(d, k * T + (int32_t)qbase, d.hist + (int64_t)((t - 1) & 1) * d.n, ns);
+        if ((flags & 2) && w >= NEV && k >= 0)
+            load_nstate<S_>(d, k * (int32_t)U, d.hist + (int64_t)((t - 1) & 1) * d.n, ns);
     }
 
     /* ---- phase (ii) of cycle t-1 ---------------------------------------- */
     if ((flags & 1) && k >= 0) {
-        const int64_t syn0 = d.tile_base[k];
-        const uint32_t nsyn = d.tile_nsyn[k];
-        const bsim_syn *syn = d.syn + syn0;
-        int64_t events = 0;
-        uint32_t rows = 0;
-        const int32_t r0 = d.tile_rng[k], r1 = d.tile_rng[k + 1];
-        for (int32_t rb = r0; rb < r1; rb += MAXR)
-            deliver_batch<S_>(S, d, rb, min(MAXR, r1 - rb), qbase, nsyn, syn, events, rows, acc);
-        if (lane == 0 && w < NWAVE)
-            atomicAdd((unsigned long long *)&d.ev_count[k], (unsigned long long)events);
-        /* the tile's work in this launch, when the row-list launch that
-         * follows ranks the tiles (it runs for cycle t + 1): its deliveries
+        const bsim_unit un = d.unit[k];
+        for (uint32_t i = tid; i < 2 * U; i += NTHREAD)
+            reinterpret_cast<uint4 *>(S.hist)[i] = make_uint4(0u, 0u, 0u, 0u);
+        for (uint32_t i = tid; i < 2 * PASS; i += NTHREAD) S.mark[i] = NO_MARK;
+        if (tid < 4) S.most[tid] = 0u;          /* most and last */
+        const bsim_syn *syn = d.syn + un.base;
+        uint32_t events = 0, rows = 0, par = 0;
+        for (int32_t rb = 0; rb < un.nrng; rb += MAXR)
+            deliver_batch<NB, S_>(S, d, un, un.rng0 + rb, min(MAXR, un.nrng - rb), U, K, par, syn, events,
+                                  rows, acc);
+        /* the unit's work in this launch, when the row-list launch that
+         * follows ranks the units (it runs for cycle t + 1): its deliveries
          * plus a fixed cost of two deliveries per active row, x 16 */
-        const int32_t re = d.rank_every;
-        if (clocked && (re == 1 || (re > 1 && (t + 1) % re == 0)) && lane == 0)
-            atomicAdd((unsigned long long *)&d.tile_load[k],
-                      w < NWAVE ? (unsigned long long)events * 16ull : (unsigned long long)rows * 32ull);
+        if (tid == 0 && rows > 0) {
+            const int32_t re = d.rank_every;
+            d.ev_count[k] += (int64_t)events;   /* one workgroup per unit and launch */
+            if (clocked && (re == 1 || (re > 1 && (t + 1) % re == 0)))
+                d.tile_load[k] = (uint64_t)events * 16ull + (uint64_t)rows * 32ull;
+        }
     }
 
-    /* ---- phase (i) of cycle t: wavefront w updates its own quarter ---------- */
-    if ((flags & 2) && w < NWAVE && k >= 0) {
+    /* ---- phase (i) of cycle t: each owner thread updates its targets -------- */
+    if ((flags & 2) && w >= NEV && k >= 0) {
         const int32_t D = d.dmax;
         const uint64_t dmask = (D >= 63) ? (~0ull >> 1) : ((1ull << D) - 1ull);
-        const int32_t base = k * T + (int32_t)qbase;
+        const int32_t base = k * (int32_t)U;
         const uint64_t *hist_in = d.hist + (int64_t)((t - 1) & 1) * d.n;
         uint64_t *hist_out = d.hist + (int64_t)(t & 1) * d.n;
         uint64_t *act_out = d.active + (int64_t)(t & 1) * d.nwords;
         const bool rec = d.raster != nullptr && t >= d.rec_t0 && t < d.rec_t0 + d.rec_steps;
 #pragma unroll
         for (int j = 0; j < S_; j++) {
-            const int32_t n0 = base + j * WAVE;
+            const uint32_t i0 = (w - NEV) * WAVE + j * (NOWN * WAVE);
+            if (i0 >= U) continue;                            /* uniform */
+            const int32_t n0 = base + (int32_t)i0;
             const int32_t nid = n0 + (int32_t)lane;
             const bool valid = nid < d.n;
             bool fired = false;
@@ -834,7 +833,8 @@ __global__ __launch_bounds__(NTHREAD) void bsim_step_kernel(bsim_dev d, int32_t 
             }
         }
     }
-    if (clocked && tid == 0)        /* the cycle was read by every wavefront at its start */
+    if (clocked) wg_barrier();      /* every wavefront has read the cycle */
+    if (clocked && tid == 0)
         (void)__hip_atomic_fetch_add(d.done + BSIM_DONE_STRIDE * (blockIdx.x % 8u), (uint64_t)1,
                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -1008,28 +1008,22 @@ extern "C" hipError_t bsim_launch_rows(const bsim_dev *d, hipStream_t stream)
     return hipGetLastError();
 }
 
-extern "C" size_t bsim_step_lds_bytes(int32_t tile)
-{
-    return tile >= 2 * NWAVE * WAVE ? lds_bytes(Win<2>::RCAP) : lds_bytes(Win<1>::RCAP);
-}
-
 extern "C" hipError_t bsim_launch_step(const bsim_dev *d, int32_t t, int32_t flags,
                                        hipStream_t stream)
 {
     if (d->ntiles <= 0) return hipSuccess;
+    const uint32_t U = (uint32_t)d->tile;
+    if (U == 0 || U % WAVE != 0 || U > BSIM_MAX_UNIT) return hipErrorInvalidValue;
     const dim3 grid(d->nslots), block(NTHREAD);
-    const size_t lds = bsim_step_lds_bytes(d->tile);
+    const size_t lds = lds_bytes(U);
     (void)hipGetLastError();       /* the check below then reports this launch alone */
-    switch (d->tile / (NWAVE * WAVE)) {
-    case 1: hipLaunchKernelGGL(bsim_step_kernel<1>, grid, block, lds, stream, *d, t, flags); break;
-    case 2: hipLaunchKernelGGL(bsim_step_kernel<2>, grid, block, lds, stream, *d, t, flags); break;
-    case 3: hipLaunchKernelGGL(bsim_step_kernel<3>, grid, block, lds, stream, *d, t, flags); break;
-    case 4: hipLaunchKernelGGL(bsim_step_kernel<4>, grid, block, lds, stream, *d, t, flags); break;
-    case 5: hipLaunchKernelGGL(bsim_step_kernel<5>, grid, block, lds, stream, *d, t, flags); break;
-    case 6: hipLaunchKernelGGL(bsim_step_kernel<6>, grid, block, lds, stream, *d, t, flags); break;
-    case 7: hipLaunchKernelGGL(bsim_step_kernel<7>, grid, block, lds, stream, *d, t, flags); break;
-    case 8: hipLaunchKernelGGL(bsim_step_kernel<8>, grid, block, lds, stream, *d, t, flags); break;
-    default: return hipErrorInvalidValue;
-    }
+#define STEP(NB, S_) hipLaunchKernelGGL((bsim_step_kernel<NB, S_>), grid, block, lds, stream, *d, t, flags)
+#define OWN(X) (((X) + NOWN * WAVE - 1) / (NOWN * WAVE))
+    if (U <= 64) STEP(6, OWN(64));
+    else if (U <= 128) STEP(7, OWN(128));
+    else if (U <= 256) STEP(8, OWN(256));
+    else STEP(9, OWN(512));
+#undef OWN
+#undef STEP
     return hipGetLastError();
 }

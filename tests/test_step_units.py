@@ -1,0 +1,96 @@
+"""The step kernel at the sizes where its passes, slots and units change:
+whole tiles and tiles in parts, a target with more events in a pass than it has
+slots, a sub-row longer than a pass, more source ranges than one batch holds,
+blocks of rows without a synapse into the unit.  Bit for bit against the
+oracle, as everything the step computes is.
+"""
+import numpy as np
+import pytest
+
+import oracle
+from bsim_amd import netspec
+
+from test_gpu_parity import DT, assert_same, run_gpu, say
+
+pytestmark = pytest.mark.gpu
+
+LIF = netspec.lif_row(0.0, 0.0, 0.0, 0.02, 0.02, 3e-4, 5e-3, 8e-3, 1.0, 0.0)
+
+
+def sources(b, n, steps, rng, p=0.3):
+    """n array sources that fire at random cycles."""
+    return b.population(np.zeros((n, netspec.LIF_NPARAM)), kind=netspec.ARRAY,
+                        spikes=[np.nonzero(rng.random(steps) < p)[0] for _ in range(n)])
+
+
+def lif(b, n, rng):
+    rows = np.tile(LIF, (n, 1))
+    rows[:, 9] = rng.uniform(0.3, 1.4, n)
+    return b.population(rows)
+
+
+def connect(b, pre, post, rng, dmax, scale):
+    """Creation order (pre, delay): mixed signs, integer delays."""
+    k = rng.integers(1, dmax + 1, len(pre))
+    order = np.lexsort((post, k, pre))
+    pre, post, k = pre[order], post[order], k[order]
+    w = np.where(rng.random(len(pre)) < 0.4, -1.0, 1.0) * rng.uniform(0.0, scale, len(pre))
+    b.connect(pre, post, w.astype(np.float32), k.astype(np.float32) * np.float32(DT),
+              (w < 0).astype(np.int8))
+
+
+def net(kind, steps):
+    rng = np.random.Generator(np.random.PCG64(sum(map(ord, kind))))
+    b = netspec.Builder()
+    if kind == "one_target":            # every event of a pass on one target, ranks far past its slots
+        s = 2600
+        sources(b, s, steps, rng, 0.5)
+        lif(b, 3, rng)
+        connect(b, np.repeat(np.arange(s), 2), np.full(2 * s, s + 1), rng, 2, 2e-3)
+    elif kind == "long_rows":           # sub-rows of up to 2,300 events, longer than a pass
+        s, n = 12, 1150
+        sources(b, s, steps, rng)
+        lif(b, n, rng)
+        pre = np.repeat(np.arange(s), 2 * n)
+        post = s + np.tile(np.repeat(np.arange(n), 2), s)
+        k = np.ones(len(pre))
+        w = rng.uniform(-0.02, 0.03, len(pre)).astype(np.float32)
+        b.connect(pre, post, w, k.astype(np.float32) * np.float32(DT), (w < 0).astype(np.int8))
+    elif kind == "many_ranges":         # 290 source ranges: three batches
+        s, n, gap = 290, 150, 300
+        sources(b, s * gap, 1, rng, 0.0)
+        b.arr[:s * gap:gap] = [np.nonzero(rng.random(steps) < 0.4)[0].astype(np.int32) for _ in range(s)]
+        lif(b, n, rng)
+        connect(b, np.repeat(np.arange(s) * gap, 40), s * gap + rng.integers(0, n, 40 * s), rng, 4, 0.05)
+    else:                               # "empty_blocks": 3,000 active rows, few with a synapse into a unit
+        s, n = 3000, 700
+        sources(b, s, steps, rng, 0.6)
+        lif(b, n, rng)
+        connect(b, np.arange(s), s + np.where(np.arange(s) < s - 40, n - 1, rng.integers(0, n, s)), rng, 1, 0.01)
+    return b.build()
+
+
+@pytest.mark.parametrize("tile", [192, 384, 768, 1536])
+@pytest.mark.parametrize("kind", ["one_target", "long_rows", "many_ranges", "empty_blocks"])
+def test_edges_of_passes_and_slots(kind, tile):
+    steps = 40
+    spec = net(kind, steps)
+    rec = [spec.n - 3, spec.n - 2, spec.n - 1]
+    say(f"[gpu] {kind} n={spec.n} s={spec.s} tile={tile}")
+    r = run_gpu(spec, steps, rec, tile)
+    o = oracle.run(spec, DT, steps, rec_ids=rec, mode="csr", tile=256, threads=8)
+    assert o.events > 1000
+    assert_same(r, o, kind)
+
+
+@pytest.mark.parametrize("npop,tile", [(2, 192), (7, 384)])
+def test_whole_tiles(npop, tile):
+    """Enough tiles that each is one unit, and the tile after the last population ragged."""
+    spec = netspec.standard(npop=npop, n=10007, fanout=24, w0=12.0, dmax=7, drive_rate_hz=200.0,
+                            n_drive=500, drive_fanout=40, drive_w=2.0, seed=5, i_offset=(14.5, 16.5))
+    steps, rec = 220, [600, spec.n - 1]
+    say(f"[gpu] whole tiles npop={npop} n={spec.n} s={spec.s} tile={tile}")
+    r = run_gpu(spec, steps, rec, tile)
+    o = oracle.run(spec, DT, steps, rec_ids=rec, mode="csr", tile=256, threads=8)
+    assert o.events > 10_000
+    assert_same(r, o, "whole tiles")
