@@ -26,9 +26,8 @@ stream synchronisations.  One JSON line is printed:
                recorded by the library around each launch on the simulation's
                stream during --roofline-steps (200) single launches right
                after the pre-roll -- the same cycles in every run, whatever K
-               and W; peak = 8 TB/s (MI355X HBM3E).  The cycle's second kernel
-               (active-row lists) is timed the same way and reported beside
-               it.  Then W warm-up cycles, then the K timed ones.
+               and W; peak = 8 TB/s (MI355X HBM3E).  row_list_kernel_us is 0: the
+               step kernel is the cycle's only one.  Then W warm-up cycles, then the K timed ones.
   cpu_baseline the oracle's event-driven CSR form (oracle/stsim.c) on the
                host's cores, timed over the same cycles of the same network
                that the GPU timed (the first --cpu-steps of them when K is
@@ -543,7 +542,7 @@ def main():
     mean_ms = step_us * 1e-3
     ev_per_launch = (evr1 - evr0) / R
     achieved = ev_per_launch * BYTES_PER_EVENT / (mean_ms * 1e-3) / 1e9
-    print(f"[bench] step kernel mean {step_us:.2f} us, row-list kernel mean {rows_us:.2f} us "
+    print(f"[bench] step kernel mean {step_us:.2f} us "
           f"over {R} launches (cycles {a.preroll}..{a.preroll + R}), {ev_per_launch:.0f} "
           f"events/launch", file=sys.stderr, flush=True)
     traffic, traffic_ev = read_traffic(a.workload, info["tile"], ev_per_launch)

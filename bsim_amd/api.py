@@ -487,7 +487,8 @@ class Simulation:
 
     def time_steps(self, n):
         """Advances n cycles one launch at a time with HIP events around each
-        kernel; returns the mean (step kernel, row-list kernel) durations in us."""
+        kernel; returns the mean step kernel duration in us, and 0 (there was a
+        second, row-list kernel)."""
         a, b = C.c_double(), C.c_double()
         r = lib().bsim_sim_time_steps(self._h, int(n), C.byref(a), C.byref(b))
         if r < 0:

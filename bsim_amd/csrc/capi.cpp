@@ -17,7 +17,6 @@
 #include "internal.h"
 #include "network.h"
 
-extern "C" hipError_t bsim_launch_rows(const bsim_dev *d, hipStream_t stream);
 extern "C" hipError_t bsim_launch_step(const bsim_dev *d, int32_t t, int32_t flags,
                                        hipStream_t stream);
 
@@ -327,12 +326,14 @@ extern "C" {
 
 /* Checks the simulation config and makes its device current (0, or a
  * failure code). */
-/* Tile schedule: the row-list launch ranks the tiles heaviest first every
- * kRankEvery cycles, by their work in the step launch before it (the volleys
- * of the standard network move slowly against 2 cycles: on C1, every 2nd
- * cycle ran 114.3 us per cycle, every cycle 114.8, every 4th 116.4);
- * bsim_sim_set_schedule changes it. */
+/* Tile schedule: the units are ranked heaviest first every kRankEvery cycles,
+ * by their work in the launch before (the volleys of the standard network move
+ * slowly against 2 cycles); bsim_sim_set_schedule changes it. */
 static const int32_t kRankEvery = 2;
+
+/* Step workgroups that run at a time: two per compute unit.  Up to as many
+ * units start at once, and their order is nothing. */
+static const int32_t kResident = 512;
 
 static int32_t check_config(const bsim_sim_config &c, int32_t N, const char *who)
 {
@@ -514,6 +515,19 @@ static bsim_sim *sim_from_layout(bsim::Layout &L, const bsim_sim_config &c, bsim
         UP(tile_res, res);
     }
     d.nslots = L.nslots * L.parts;
+    {
+        /* an event thread takes two rows at a time where a unit has many rows
+         * of few events: a block of 512 rows then leaves a pass of 1,024 events
+         * short.  Otherwise one, so that few active rows are spread over more
+         * wavefronts.  us per cycle with one / two, by synapses per row and
+         * unit (the row table has an entry for each) and rows of a tile: 0.73
+         * and 5e5 1,048 / 946, 0.39 and 5e4 64 / 52, 0.75 and 9e4 194 / 154;
+         * 1.37 and 4e4 13.2 / 13.3, 1.49 and 7e3 7.8 / 9.1, 2.4 and 6e4
+         * 61.5 / 69.2 */
+        int64_t rows = 0;
+        for (const auto &r : L.rng) rows += (int64_t)(r.hi - r.lo) * L.dmax;
+        d.wrows = (double)L.s < 1.25 * (double)L.off_tab.size() && rows >= (int64_t)32768 * L.ntiles ? 2 : 1;
+    }
     if (dev_syn) {
         d.syn = dev_syn;
     } else {
@@ -530,12 +544,6 @@ static bsim_sim *sim_from_layout(bsim::Layout &L, const bsim_sim_config &c, bsim
     }
     UP(rng, L.rng);
     UP(off_tab, L.off_tab);
-    UP(src_lo, L.src_lo);
-    UP(src_hi, L.src_hi);
-    UP(src_list_base, L.src_list_base);
-    UP(chunk_tiles_off, L.chunk_tiles_off);
-    UP(chunk_rng, L.chunk_rng);
-    d.nsrc = (int32_t)L.src_lo.size();
     /* state */
     UP(v, L.v_init);
     UP(arr_cur, L.arr_cur0);
@@ -549,7 +557,8 @@ static bsim_sim *sim_from_layout(bsim::Layout &L, const bsim_sim_config &c, bsim
         if (!(d.refrac = dev_alloc<int32_t>(sim, n, e))) goto hip_fail;
         if (!(d.fire_count = dev_alloc<int32_t>(sim, n, e))) goto hip_fail;
         if (!(d.hist = dev_alloc<uint64_t>(sim, 2 * n, e))) goto hip_fail;
-        if (!(d.active = dev_alloc<uint64_t>(sim, 2 * nw, e))) goto hip_fail;
+        if (!(d.seg = dev_alloc<uint16_t>(sim, 2 * nw * 64 * (size_t)d.dmax, e))) goto hip_fail;
+        if (!(d.seg_count = dev_alloc<uint32_t>(sim, 2 * nw, e))) goto hip_fail;
         if (!(d.ev_count = dev_alloc<int64_t>(sim, nt, e))) goto hip_fail;
         if (!(sim->ev_fin = dev_alloc<int64_t>(sim, nt, e))) goto hip_fail;
         if (!(d.done = dev_alloc<uint64_t>(sim, 8 * BSIM_DONE_STRIDE, e))) goto hip_fail;
@@ -563,25 +572,22 @@ static bsim_sim *sim_from_layout(bsim::Layout &L, const bsim_sim_config &c, bsim
                 const int x = res[t];
                 perm[(size_t)8 * rank[x]++ + x] = t;
             }
+            perm.insert(perm.end(), perm.begin(), perm.end());        /* both orders */
             d.perm = dev_upload(sim, perm, e);
             if (e != hipSuccess) goto hip_fail;
         }
         d.rank_every = kRankEvery;
-        d.done_inv = d.nslots >= 8 ? 8.0 / (double)d.nslots : 0.0;
-        if (!(d.tile_load = dev_alloc<uint64_t>(sim, nt, e))) goto hip_fail;
-        if ((e = hipMemsetAsync(d.tile_load, 0, nt * sizeof(uint64_t), sim->stream)) != hipSuccess) goto hip_fail;
+        d.rank_wgs = d.nslots > kResident ? 8 : 0;
+        d.done_inv = d.nslots >= 8 ? 8.0 / (double)(d.nslots + d.rank_wgs) : 0.0;
+        if (!(d.tile_load = dev_alloc<uint64_t>(sim, 2 * nt, e))) goto hip_fail;
+        if ((e = hipMemsetAsync(d.tile_load, 0, 2 * nt * sizeof(uint64_t), sim->stream)) != hipSuccess) goto hip_fail;
         if (!(d.tile_cls = dev_alloc<uint8_t>(sim, nt, e))) goto hip_fail;
-        const size_t nre = (size_t)(L.rng.empty() ? 1 : L.rng.size());
-        if (!(d.rng_count = dev_alloc<uint32_t>(sim, nre, e))) goto hip_fail;
-        if ((e = hipMemsetAsync(d.rng_count, 0, nre * sizeof(uint32_t), sim->stream)) != hipSuccess) goto hip_fail;
-        if (!(d.src_list = dev_alloc<uint32_t>(sim, (size_t)(L.src_list_len > 0 ? L.src_list_len : 1), e)))
-            goto hip_fail;
         if ((e = hipMemsetAsync(d.ie, 0, n * 4, sim->stream)) != hipSuccess) goto hip_fail;
         if ((e = hipMemsetAsync(d.ii, 0, n * 4, sim->stream)) != hipSuccess) goto hip_fail;
         if ((e = hipMemsetAsync(d.refrac, 0, n * 4, sim->stream)) != hipSuccess) goto hip_fail;
         if ((e = hipMemsetAsync(d.fire_count, 0, n * 4, sim->stream)) != hipSuccess) goto hip_fail;
         if ((e = hipMemsetAsync(d.hist, 0, 2 * n * 8, sim->stream)) != hipSuccess) goto hip_fail;
-        if ((e = hipMemsetAsync(d.active, 0, 2 * nw * 8, sim->stream)) != hipSuccess) goto hip_fail;
+        if ((e = hipMemsetAsync(d.seg_count, 0, 2 * nw * 4, sim->stream)) != hipSuccess) goto hip_fail;
         if ((e = hipMemsetAsync(d.ev_count, 0, nt * 8, sim->stream)) != hipSuccess) goto hip_fail;
         if ((e = hipMemsetAsync(sim->ev_fin, 0, nt * 8, sim->stream)) != hipSuccess) goto hip_fail;
         if (c.rec_steps > 0) {
@@ -623,8 +629,7 @@ hip_fail:
 
 /* Cycles per captured graph: runs of this many cycles are replayed from one
  * hipGraph of identical clocked launches (the step kernel reads and advances
- * the device-side cycle counter; the row-list kernel after it builds the
- * next cycle's active-row lists and ranks the tiles). */
+ * the device-side cycle counter). */
 static const int32_t kGraphCycles = 64;
 
 static hipError_t build_graph(bsim_sim *sim)
@@ -634,7 +639,6 @@ static hipError_t build_graph(bsim_sim *sim)
     hipError_t le = hipSuccess;
     for (int32_t i = 0; i < kGraphCycles && le == hipSuccess; i++) {
         le = bsim_launch_step(&sim->d, -1, 0, sim->stream);
-        if (le == hipSuccess) le = bsim_launch_rows(&sim->d, sim->stream);
     }
     hipGraph_t g = nullptr;
     e = hipStreamEndCapture(sim->stream, &g);
@@ -674,7 +678,6 @@ int32_t bsim_sim_step(bsim_sim *sim, int32_t n)
     }
     for (; n > 0; n--) {
         e = bsim_launch_step(&sim->d, -1, 0, sim->stream);
-        if (e == hipSuccess) e = bsim_launch_rows(&sim->d, sim->stream);
         if (e != hipSuccess) return fail(BSIM_E_HIP, std::string("step launch: ") + hipGetErrorString(e));
         sim->cycle++;
     }
@@ -685,31 +688,27 @@ int32_t bsim_sim_time_steps(bsim_sim *sim, int32_t n, double *step_us, double *r
 {
     if (!sim || n <= 0) return fail(BSIM_E_ARG, "bsim_sim_time_steps: bad argument");
     if (int32_t rc = use_device(sim)) return rc;
-    std::vector<hipEvent_t> ev((size_t)n * 3, nullptr);
+    std::vector<hipEvent_t> ev((size_t)n * 2, nullptr);
     hipError_t e = hipSuccess;
     for (size_t i = 0; i < ev.size() && e == hipSuccess; i++) e = hipEventCreate(&ev[i]);
     for (int32_t i = 0; i < n && e == hipSuccess; i++) {
-        e = hipEventRecord(ev[3 * i], sim->stream);
+        e = hipEventRecord(ev[2 * i], sim->stream);
         if (e == hipSuccess) e = bsim_launch_step(&sim->d, -1, 0, sim->stream);
-        if (e == hipSuccess) e = hipEventRecord(ev[3 * i + 1], sim->stream);
-        if (e == hipSuccess) e = bsim_launch_rows(&sim->d, sim->stream);
-        if (e == hipSuccess) e = hipEventRecord(ev[3 * i + 2], sim->stream);
+        if (e == hipSuccess) e = hipEventRecord(ev[2 * i + 1], sim->stream);
         if (e == hipSuccess) sim->cycle++;
     }
     if (e == hipSuccess) e = hipStreamSynchronize(sim->stream);
-    double a = 0.0, b = 0.0;
+    double a = 0.0;
     for (int32_t i = 0; i < n && e == hipSuccess; i++) {
-        float x = 0.f, y = 0.f;
-        e = hipEventElapsedTime(&x, ev[3 * i], ev[3 * i + 1]);
-        if (e == hipSuccess) e = hipEventElapsedTime(&y, ev[3 * i + 1], ev[3 * i + 2]);
+        float x = 0.f;
+        e = hipEventElapsedTime(&x, ev[2 * i], ev[2 * i + 1]);
         a += x;
-        b += y;
     }
     for (hipEvent_t x : ev)
         if (x) hipEventDestroy(x);
     if (e != hipSuccess) return fail(BSIM_E_HIP, std::string("time_steps: ") + hipGetErrorString(e));
     if (step_us) *step_us = a * 1e3 / n;
-    if (rows_us) *rows_us = b * 1e3 / n;
+    if (rows_us) *rows_us = 0.0;   /* the step kernel makes the lists itself */
     return 0;
 }
 
@@ -955,7 +954,7 @@ int32_t bsim_sim_set_schedule(bsim_sim *sim, int32_t rank_every)
     /* the captured launches hold the kernel arguments: capture again; the
      * loads of a tile ranked later start from zero */
     if ((e = hipStreamSynchronize(sim->stream)) != hipSuccess ||
-        (e = hipMemsetAsync(sim->d.tile_load, 0, (size_t)(sim->d.ntiles > 0 ? sim->d.ntiles : 1) * 8,
+        (e = hipMemsetAsync(sim->d.tile_load, 0, (size_t)(sim->d.ntiles > 0 ? sim->d.ntiles : 1) * 16,
                             sim->stream)) != hipSuccess ||
         (e = hipStreamSynchronize(sim->stream)) != hipSuccess)
         return fail(BSIM_E_HIP, std::string("bsim_sim_set_schedule: ") + hipGetErrorString(e));

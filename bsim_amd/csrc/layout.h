@@ -35,11 +35,11 @@
  * the XCD's L2.
  *
  * Spike history: hist[n] bit j = neuron n fired j cycles ago (bit 0 = this
- * cycle).  After updating cycle t, a tile writes its neurons' history words
- * and one bit per neuron in the "active" bitmap: set iff any of bits 1..D of
- * the history is set, i.e. iff some (n, d) row delivers in phase (ii) of cycle
- * t.  Both are double-buffered by cycle parity, so that a launch reads the
- * previous cycle's copy while it writes the current one.
+ * cycle).  After updating cycle t, a unit writes its neurons' history words
+ * and, for each block of 64 neurons, the list of (n, d) rows that deliver in
+ * phase (ii) of cycle t: n's history has bit d set.  Both are double-buffered
+ * by cycle parity, so that a launch reads the previous cycle's copy while it
+ * writes the current one.
  */
 #ifndef BSIM_LAYOUT_H
 #define BSIM_LAYOUT_H
@@ -73,8 +73,8 @@ typedef struct __attribute__((aligned(32))) bsim_unit {
 typedef struct bsim_range {
     int32_t lo, hi;     /* pre neurons [lo, hi) of one chunk of a source range of the tile */
     int64_t off_base;   /* off_tab index of the tile's first entry of row (lo, 1) */
-    int64_t lbase;      /* first entry of the chunk's active-row list in src_list */
-    int32_t uid;        /* source chunk: index into src_* */
+    int64_t lbase;      /* rows (p, d) of the chunks before this one (host) */
+    int32_t uid;        /* source chunk: index into src_* (host) */
     uint32_t wrow;      /* expected deliveries of one active row into the tile, x 16 (host statistics) */
     uint32_t stride;    /* off_tab entries per (pre, delay) row of the group */
     uint32_t pad;
@@ -90,7 +90,7 @@ typedef struct __attribute__((aligned(8))) bsim_syn {
 } bsim_syn;
 
 #define BSIM_MAX_RANGE (1 << 26)   /* pres per source range: row index fits 32 bits */
-#define BSIM_CHUNK 4096             /* pres per source chunk (one row-list workgroup) */
+#define BSIM_CHUNK 4096             /* pres per source chunk: 64 blocks of 64 */
 
 /* LIF_brian constants shared by the neurons of one parameter set (usually a
  * population): the reference keeps them per neuron (GLIFENeurons.h:7-24);
@@ -130,41 +130,33 @@ typedef struct bsim_dev {
     int32_t *arr_cur;
     int32_t *fire_count;
     uint64_t *hist;             /* [2][n] by cycle parity */
-    uint64_t *active;           /* [2][nwords] by cycle parity */
     /* synapses */
-    int32_t nslots;             /* step workgroups (tiles placed by XCD residue) */
-    int32_t pad3;
+    int32_t nslots;             /* step workgroups (units placed by XCD residue) */
+    int32_t wrows;              /* rows that an event thread takes at a time, 1 or 2 */
     const bsim_unit *unit;      /* [ntiles] */
     const uint8_t *tile_res;    /* [ntiles] XCD residue of the unit's group */
     const bsim_syn *syn;        /* [S] target and weight of each synapse, group-major */
     const bsim_range *rng;
     const uint32_t *off_tab;    /* group row tables */
-    /* source chunks and their active-row lists: the distinct source ranges of
-     * all tiles, cut into chunks of at most BSIM_CHUNK pres (a tile's range
-     * entries are per chunk).  After the update of cycle t, list u holds the
-     * row index (p - lo) * D + d - 1 of every (pre, delay) of chunk u that
-     * delivers in phase (ii) of cycle t, ascending; it is shared by every
-     * tile that receives from the chunk */
-    int32_t nsrc;
-    int32_t pad2;
-    const int32_t *src_lo, *src_hi;
-    const int64_t *src_list_base;
-    uint32_t *src_list;
-    uint32_t *rng_count;        /* [range entries] rows in the entry's chunk list this cycle */
+    /* active rows, by cycle parity: after the update of cycle t, the list of
+     * block b (neurons 64 b .. 64 b + 63) holds (p % 64) << 6 | d - 1 for every
+     * (p, d) of the block that delivers in phase (ii) of cycle t, ascending */
+    uint16_t *seg;              /* [2][nwords][64 * dmax] */
+    uint32_t *seg_count;        /* [2][nwords] */
     /* accounting / recording */
     int64_t *ev_count;          /* [ntiles] deliveries performed */
     uint64_t *done;             /* [8 * BSIM_DONE_STRIDE]: step workgroups finished by clocked
                                    launches, per XCD residue x at done[BSIM_DONE_STRIDE * x];
-                                   each grows by nslots / 8 per launch */
-    double done_inv;            /* 8 / nslots */
-    int32_t *perm;              /* [nslots] tile of each step workgroup (-1: none) */
-    uint64_t *tile_load;        /* [ntiles] work of the launch before a ranking (x 16) */
-    int32_t rank_every;         /* tiles ranked heaviest first every this many cycles (0: never,
-                                   the tiles stay in their initial order) */
-    int32_t pad5;
-    uint8_t *tile_cls;          /* [ntiles] its half-octave class */
-    const int64_t *chunk_tiles_off;  /* [nsrc + 1] tiles that read each chunk: */
-    const int32_t *chunk_rng;        /*   the tile's range entry for the chunk */
+                                   each grows by (nslots + rank_wgs) / 8 per launch */
+    double done_inv;            /* 8 / (nslots + rank_wgs) */
+    int32_t *perm;              /* [2][nslots] unit of each slot (-1: none): two orders, of the last
+                                   ranking and the one before */
+    uint64_t *tile_load;        /* [2][ntiles] work of a launch before a ranking (x 16), by cycle parity */
+    int32_t rank_every;         /* units ranked heaviest first every this many cycles (0: never,
+                                   the units stay in their initial order) */
+    int32_t rank_wgs;           /* workgroups before the slots' (the first ranks): 8, or 0 where every unit
+                                   runs at once and order is nothing */
+    uint8_t *tile_cls;          /* [ntiles] half-octave class of a unit's work */
     uint64_t *raster;           /* [rec_steps][nwords] fired bitmaps, or NULL */
     int32_t rec_steps;
     int32_t rec_t0;             /* cycle of raster/trace row 0 */

@@ -423,8 +423,9 @@ int build_layout(const HostNet &net, float dt, int32_t tile, Layout &L, std::str
                 f++;
             }
             bsim_range r;
-            r.lo = p0;
-            r.hi = plast + 1;
+            /* whole blocks of 64 pres, as the active-row lists have them */
+            r.lo = p0 & ~63;
+            r.hi = (plast | 63) + 1;
             r.off_base = (int64_t)toff[t].size();
             r.uid = 0;
             r.wrow = 0;

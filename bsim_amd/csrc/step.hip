@@ -1,7 +1,7 @@
 /*
  * step.hip -- the simulation step on CDNA4 (gfx950).
  *
- * A cycle is two launches.  bsim_step_kernel: one workgroup per unit of
+ * A cycle is one launch of bsim_step_kernel: one workgroup per unit of
  * consecutive neurons (a tile or a third of one, layout.h) performs
  *
  *   (ii) phase (ii) of cycle t-1: every synapse into the unit whose pre fired
@@ -10,13 +10,20 @@
  *        (src/net/Network.cpp:324-327, src/neuron/lif/LIFENeuron.cpp:52-61);
  *   (i)  the LIF_brian update of cycle t (src/neuron/lif/LIFENeuron.cpp:114-160),
  *        which consumes exactly those accumulators, the spike history update
- *        and the ordered compaction of the unit's fired / active neurons into
- *        64-bit words by wavefront ballot.
+ *        and the ordered compaction of each 64 neurons' fired bits (by wavefront
+ *        ballot) and active (pre, delay) rows, the list that the next launch's
+ *        units read.
  *
- * bsim_rows_kernel then builds, for every source chunk, the list of its
- * active (pre, delay) rows for the next phase (ii), shared by all tiles that
- * receive from the chunk; one more workgroup ranks the tiles, heaviest first,
- * by the work the step launch recorded.
+ * One more workgroup orders the units for the launches to come, heaviest
+ * first, by the work that the launch before recorded, where they are more than
+ * run at a time.
+ *
+ * A unit finds its active rows from the lists of the blocks of 64 pres that its
+ * source chunks cover.  A second launch per cycle, which merged them into one
+ * list per 4,096 pres, took 4 us of a cycle of a few dozen neurons and 8 to 11
+ * of large ones, with the launch's own start: us per cycle with it and without,
+ * 48 neurons 11.3 / 7.7, 9,896 10.8 / 7.8, 230,000 in 96 chains 33.0 / 28.5,
+ * 330,000 63.2 / 61.4, 650,000 113 / 111.
  *
  * Phase (ii) for a unit: the sub-rows of its active rows, in list order, form
  * one stream of events, which the workgroup takes in passes of PASS = 1,024
@@ -63,11 +70,11 @@
 #define PASS (NCOL * WAVE)
 #define NGRP (NCOL / NEV)             /* groups of an event wavefront */
 #define NO_MARK 0xFFFFFFFFu           /* no synapse index: a group has fewer than 2^32 - 1 */
-#define MAXR 128                      /* source ranges per batch */
-#define ROWS_THREADS 1024             /* row-list kernel: 4 pres per thread */
-#define HEAVY_WGS 256                 /* workgroups run at raised wave priority */
+#define MAXR 32                       /* source chunks per batch */
+#define BLKS (BSIM_CHUNK / WAVE)      /* blocks of 64 pres per source chunk */
+#define NRES 8                        /* XCDs: workgroup w runs on XCD (w + c) mod 8 */
 #define STEP_EU 6                     /* wavefronts per SIMD: two workgroups per compute unit */
-static_assert(BSIM_CHUNK == 4 * ROWS_THREADS, "a source chunk is one row-list workgroup");
+static_assert(BLKS == WAVE, "a lane per block of a source chunk");
 static_assert(NCOL == 16 && NCOL % NEV == 0, "a target's histogram row is one 16-byte vector");
 
 /* Slots per target: a pass puts PASS / U events on a target of a unit of U on
@@ -77,10 +84,11 @@ __host__ __device__ constexpr uint32_t slots_of(uint32_t U)
     return U >= 384 ? 8u : (3u * PASS / U) & ~3u;
 }
 
-/* LDS bytes of a workgroup: lbase, obase | hist | mark | slot | btot, cum, stride, most, last */
+/* LDS bytes of a workgroup: chunk | hist | mark | slot | blk_end | blk_mark | btot, ctot, most, last */
 __host__ __device__ constexpr size_t lds_bytes(uint32_t U)
 {
-    return 16 * MAXR + 2 * U * NCOL + 8 * PASS + 4 * slots_of(U) * U + 8 * NEV + 4 * (MAXR + 1) + 4 * MAXR + 16;
+    return 16 * MAXR + 2 * U * NCOL + 8 * PASS + 4 * slots_of(U) * U + 4 * MAXR * BLKS + 4 * NEV * WAVE + 8 * NEV +
+           4 * MAXR + 16;
 }
 
 __device__ __forceinline__ uint32_t bern_hash(uint64_t seed, uint32_t id, uint32_t t)
@@ -131,11 +139,10 @@ __device__ __forceinline__ uint32_t wave_index() { return uniform(threadIdx.x / 
 /* The device clock: the cycle of the coming clocked step launch.  Every
  * workgroup of a clocked launch adds one to the completion counter of its XCD
  * residue x = workgroup % 8 when it ends (an atomic whose result nobody waits
- * for); each residue holds nslots / 8 workgroups, so its counter grows by
- * that much per launch.  While any workgroup of launch t runs, its own
- * residue's counter lies in [t nslots / 8, (t + 1) nslots / 8) -- it has not
- * added its one yet -- so the quotient is t; a row-list launch, after its
- * step launch has completed, reads t + 1 from any counter.  Plain (scalar,
+ * for); each residue holds 1 / 8 of the grid, so its counter grows by that
+ * much per launch.  While any workgroup of launch t runs, its own residue's
+ * counter lies in [t grid / 8, (t + 1) grid / 8) -- it has not added its one
+ * yet -- so the quotient is t.  Plain (scalar,
  * cached) loads: a launch sees the counts of the launches before it, and a
  * value cached during the launch is still within its interval.  (A single
  * counter whose last incrementer advanced the cycle made every workgroup wait
@@ -143,8 +150,8 @@ __device__ __forceinline__ uint32_t wave_index() { return uniform(threadIdx.x / 
  * deliveries.) */
 __device__ __forceinline__ int32_t device_cycle(const bsim_dev &d, uint32_t x)
 {
-    /* count / (nslots / 8) without an integer division: the quotient's
-     * fractional part is a multiple of 8 / nslots, so half of that added
+    /* count / (grid / 8) without an integer division: the quotient's
+     * fractional part is a multiple of 8 / grid, so half of that added
      * before truncation absorbs the rounding of the product (below 2^-20 for
      * cycles below 2^31, against a half step of at least 2^-19 for grids of
      * up to 2^18 workgroups per residue) */
@@ -169,76 +176,87 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x)
 
 /* ---- delivery ------------------------------------------------------------- */
 
+/* A source chunk of the batch: where its row table starts in off_tab (low and
+ * high word), its first block of 64 pres, table entries per row. */
+struct __attribute__((aligned(16))) Chunk {
+    uint32_t ob_lo, ob_hi, blk, st;
+};
+
 struct Shared {
-    uint64_t *lbase, *obase;    /* [MAXR] first list entry / table base of each source range of the batch */
-    uint32_t *cum;              /* [MAXR + 1] rows before each source range */
-    uint32_t *stride;           /* [MAXR] table entries per row */
-    uint32_t *mark;             /* [2][PASS] synapse index where a sub-row or group starts, else NO_MARK */
+    Chunk *chunk;               /* [MAXR] */
     uint32_t *hist;             /* [2][U][NCOL / 4] events of each target per group, one byte each */
+    uint32_t *mark;             /* [2][PASS] synapse index where a sub-row or group starts, else NO_MARK */
     float *slot;                /* [K][U] a pass's weights of each target in stream order */
+    uint32_t *blk_end;          /* [MAXR][BLKS] active rows of a chunk up to the end of each of its blocks */
+    uint32_t *blk_mark;         /* [NEV][64] first rows of blocks among 64 rows (load_entries), else NO_MARK */
     uint32_t *btot;             /* [2][NEV] stream length of each event wavefront's rows of a block */
+    uint32_t *ctot;             /* [MAXR] active rows of each chunk */
     uint32_t *most;             /* [2] largest rank of a pass's events beyond the slots */
     uint32_t *last;             /* [2] the pass is the batch's last */
 };
 
-__device__ __forceinline__ uint64_t uniform64(uint64_t x)
+/* orders this wavefront's LDS accesses (lanes exchange data through LDS) */
+__device__ __forceinline__ void wave_sync()
 {
-    return (uint64_t)uniform((uint32_t)x) | ((uint64_t)uniform((uint32_t)(x >> 32)) << 32);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 __device__ __forceinline__ void wg_barrier() { __syncthreads(); }
 
-/* A place in the concatenated active-row lists of a batch of source ranges
- * (uniform): row j of the batch, in range ri, is list entry lb + j, and list
- * entry e's table entry is ob + e * st. */
-struct Cursor {
-    int32_t ri;
-    uint32_t next;              /* first row of the range after ri */
-    uint64_t lb, ob;
-    uint32_t st;
+/* The batch's active rows: those of its chunks in order, of a chunk's blocks of
+ * 64 pres in order, of a block as its list has them.  Lane c < nrb holds the
+ * rows up to the end of chunk c; at: the chunk that the next rows start in. */
+struct Rows {
+    uint32_t end;
+    int32_t nrb, at;
 };
 
-__device__ __forceinline__ uint32_t range_end(const Shared &S, int32_t ri, int32_t nrb)
-{
-    return ri + 1 < nrb ? S.cum[ri + 1] : 0xFFFFFFFFu;
-}
+__device__ __forceinline__ uint32_t chunk_end(const Rows &R, int32_t c) { return c < 0 ? 0u : readlane(R.end, c); }
 
-__device__ __forceinline__ void set_range(const Shared &S, Cursor &c, int32_t ri, int32_t nrb)
-{
-    c.ri = ri;
-    c.next = uniform(range_end(S, ri, nrb));
-    c.lb = uniform64(S.lbase[ri]) - (uint64_t)uniform(S.cum[ri]);
-    c.ob = uniform64(S.obase[ri]);
-    c.st = uniform(S.stride[ri]);
-}
-
-/* List entries of 64 rows (lane l: row l) and where their table entries lie. */
+/* List entries of WR times 64 rows (lane l: rows l, 64 + l, ...): e = (p % 64)
+ * << 6 | d - 1 of the row, cb = chunk << 6 | block of its pre. */
+template <int WR>
 struct Entries {
-    uint32_t e, st;
-    uint64_t ob;
+    uint32_t e[WR], cb[WR];
     uint32_t n;                 /* rows (uniform) */
 };
 
-/* Loads the list entries of the rows from j0 on.  They mostly lie in one
- * range, whose values are then uniform. */
-__device__ __forceinline__ void load_entries(const Shared &S, const bsim_dev &d, Cursor &c, int32_t nrb,
-                                             uint32_t j0, uint32_t nrows, Entries &E)
+/* Loads the list entries of the rows from j0 on.  Every block that has any of
+ * 64 of them marks its first (with the block, and how many of its rows come
+ * before); a row's block is that of the last mark at or before it. */
+template <int WR>
+__device__ __forceinline__ void load_entries(const Shared &S, const bsim_dev &d, const uint16_t *seg, Rows &R,
+                                             uint32_t j0, uint32_t nrows, Entries<WR> &E)
 {
-    E.n = j0 < nrows ? min((uint32_t)WAVE, nrows - j0) : 0u;
-    if (E.n == 0) return;                                     /* uniform */
-    while (j0 >= c.next) set_range(S, c, c.ri + 1, nrb);
-    const uint32_t l = min((uint32_t)(threadIdx.x & (WAVE - 1)), E.n - 1u);
-    if (j0 + E.n <= c.next) {                                 /* uniform */
-        E.e = (d.src_list + (c.lb + j0))[l];
-        E.ob = c.ob;
-        E.st = c.st;
-    } else {
-        int32_t ri = c.ri;
-        uint32_t nx = c.next;
-        while (j0 + l >= nx) nx = range_end(S, ++ri, nrb);
-        E.e = d.src_list[S.lbase[ri] - (uint64_t)S.cum[ri] + (uint64_t)(j0 + l)];
-        E.ob = S.obase[ri];
-        E.st = S.stride[ri];
+    E.n = j0 < nrows ? min((uint32_t)(WR * WAVE), nrows - j0) : 0u;
+    const uint32_t lane = threadIdx.x & (WAVE - 1), cap = WAVE * (uint32_t)d.dmax;
+    uint32_t *mk = S.blk_mark + wave_index() * WAVE;
+#pragma unroll
+    for (int i = 0; i < WR; i++) {
+        if (E.n <= (uint32_t)(i * WAVE)) continue;            /* uniform */
+        const uint32_t b = j0 + i * WAVE, e1 = b + min((uint32_t)WAVE, E.n - i * WAVE);
+        while (chunk_end(R, R.at) <= b) R.at++;
+        for (int32_t c = R.at;; c++) {
+            const uint32_t base = chunk_end(R, c - 1), ce = chunk_end(R, c);
+            const uint32_t e = base + S.blk_end[c * BLKS + lane];
+            const uint32_t s = lane > 0 ? base + S.blk_end[c * BLKS + lane - 1] : base;
+            const uint32_t lo = max(s, b), hi = min(e, e1);
+            if (hi > lo) mk[lo - b] = (uint32_t)c << 6 | lane | (lo - s) << 11;
+            if (ce >= e1) break;
+        }
+        wave_sync();
+        const uint32_t v = mk[lane];
+        mk[lane] = NO_MARK;
+        wave_sync();
+        const uint64_t m = ballot64(v != NO_MARK) & (~0ull >> (WAVE - 1 - lane));
+        const uint32_t at = (WAVE - 1) - (uint32_t)__clzll((long long)(m | 1ull));
+        const uint32_t f = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(at * 4u), (int)v);
+        E.cb[i] = f & (MAXR * BLKS - 1);
+        /* lanes past the last row load an entry of its block's list */
+        const uint32_t x = min((f >> 11) + lane - at, cap - 1u);
+        E.e[i] = seg[(uint64_t)(S.chunk[E.cb[i] >> 6].blk + (E.cb[i] & 63u)) * cap + x];
     }
 }
 
@@ -246,39 +264,58 @@ typedef uint32_t pair_u32 __attribute__((ext_vector_type(2), aligned(4)));
 
 /* Loads the rows' table entries: each sub-row's start and the start of the one
  * after it. */
-__device__ __forceinline__ void load_rows(const bsim_dev &d, const Entries &E, pair_u32 &ab)
+template <int WR>
+__device__ __forceinline__ void load_rows(const Shared &S, const bsim_dev &d, const Entries<WR> &E, pair_u32 (&ab)[WR])
 {
-    if (E.n == 0) return;                                     /* uniform */
-    ab = *reinterpret_cast<const pair_u32 *>(d.off_tab + E.ob + (uint64_t)(E.e * E.st));
+#pragma unroll
+    for (int i = 0; i < WR; i++) {
+        if (E.n <= (uint32_t)(i * WAVE)) continue;            /* uniform */
+        const uint4 ch = *reinterpret_cast<const uint4 *>(S.chunk + (E.cb[i] >> 6));
+        /* an entry past the end of its block's list is any word: kept within the
+         * block's rows */
+        const uint32_t row = ((E.cb[i] & 63u) * WAVE + (E.e[i] >> 6 & 63u)) * (uint32_t)d.dmax +
+                             min(E.e[i] & 63u, (uint32_t)d.dmax - 1u);
+        ab[i] = *reinterpret_cast<const pair_u32 *>(d.off_tab + ((uint64_t)ch.y << 32 | ch.x) + (uint64_t)(row * ch.w));
+    }
 }
 
-/* A block of NEV * 64 rows, one per thread of the event wavefronts: the row's
+/* A block of NEV * 64 * WR rows, WR per thread of the event wavefronts: the row's
  * sub-row into the unit as its first synapse, its length and its position in
  * the batch's stream of events. */
+template <int WR>
 struct Block {
-    uint32_t a, len, pos;
+    uint32_t a[WR], len[WR], pos[WR];
 };
 
 /* The block's sub-rows from its table entries (n rows in this wavefront), with
  * positions within the wavefront; the wavefront's stream length goes to btot. */
-__device__ __forceinline__ void make_block(const Shared &S, const pair_u32 &ab, uint32_t n, uint32_t buf, Block &k)
+template <int WR>
+__device__ __forceinline__ void make_block(const Shared &S, const pair_u32 (&ab)[WR], uint32_t n, uint32_t buf,
+                                           Block<WR> &k)
 {
     const uint32_t lane = threadIdx.x & (WAVE - 1);
-    k.a = ab.x;
-    k.len = lane < n ? ab.y - ab.x : 0u;
-    const uint32_t incl = wave_incl_scan(k.len);
-    k.pos = incl - k.len;
-    if (lane == WAVE - 1) S.btot[buf * NEV + wave_index()] = incl;
+    uint32_t at = 0;
+#pragma unroll
+    for (int i = 0; i < WR; i++) {
+        k.a[i] = ab[i].x;
+        k.len[i] = i * WAVE + lane < n ? ab[i].y - ab[i].x : 0u;
+        const uint32_t incl = wave_incl_scan(k.len[i]);
+        k.pos[i] = at + incl - k.len[i];
+        at += readlane(incl, WAVE - 1);
+    }
+    if (lane == 0) S.btot[buf * NEV + wave_index()] = at;
 }
 
 /* Positions in the batch's stream, once every wavefront has written btot: at is
  * the stream's length so far (uniform), advanced past the block. */
-__device__ __forceinline__ void place_block(const Shared &S, uint32_t buf, Block &k, uint32_t &at)
+template <int WR>
+__device__ __forceinline__ void place_block(const Shared &S, uint32_t buf, Block<WR> &k, uint32_t &at)
 {
     const uint32_t lane = threadIdx.x & (WAVE - 1);
     const uint32_t incl = wave_incl_scan(lane < NEV ? S.btot[buf * NEV + lane] : 0u);
-    const uint32_t w = wave_index();
-    k.pos += at + (w > 0 ? readlane(incl, (int32_t)w - 1) : 0u);
+    const uint32_t w = wave_index(), before = at + (w > 0 ? readlane(incl, (int32_t)w - 1) : 0u);
+#pragma unroll
+    for (int i = 0; i < WR; i++) k.pos[i] += before;
     at += readlane(incl, WAVE - 1);
 }
 
@@ -288,13 +325,17 @@ __device__ __forceinline__ void place_block(const Shared &S, uint32_t buf, Block
  * covers, with the synapse index there (put_marks); a position's synapse lies
  * past the last mark at or before it in its group, the highest set bit of the
  * group's ballot (load_events). */
-__device__ __forceinline__ void put_marks(uint32_t *mark, const Block &k, uint32_t b, uint32_t e)
+template <int WR>
+__device__ __forceinline__ void put_marks(uint32_t *mark, const Block<WR> &k, uint32_t b, uint32_t e)
 {
-    const uint32_t lo = max(k.pos, b), hi = min(k.pos + k.len, e);
-    if (hi > lo) {
-        const uint32_t x = lo - b, y = hi - b, a = k.a + (lo - k.pos);
-        mark[x] = a;
-        for (uint32_t g = (x | (WAVE - 1)) + 1u; g < y; g += WAVE) mark[g] = a + (g - x);
+#pragma unroll
+    for (int i = 0; i < WR; i++) {
+        const uint32_t lo = max(k.pos[i], b), hi = min(k.pos[i] + k.len[i], e);
+        if (hi > lo) {
+            const uint32_t x = lo - b, y = hi - b, a = k.a[i] + (lo - k.pos[i]);
+            mark[x] = a;
+            for (uint32_t g = (x | (WAVE - 1)) + 1u; g < y; g += WAVE) mark[g] = a + (g - x);
+        }
     }
 }
 
@@ -364,37 +405,36 @@ __device__ __forceinline__ uint32_t byte_sum(uint32_t x, uint32_t acc) { return 
  * The loads run ahead of the passes: a pass's synapses are loaded during the
  * pass before, the table entries and list entries one and two blocks ahead of
  * the rows that the marks are put from. */
-template <int NB>
-__device__ void event_wave(const Shared &S, const bsim_dev &d, const bsim_unit &un, int32_t nrb, uint32_t nrows,
-                           uint32_t U, uint32_t K, uint32_t &par, const bsim_syn *syn, uint32_t &events)
+template <int NB, int WR>
+__device__ void event_wave(const Shared &S, const bsim_dev &d, const bsim_unit &un, Rows &R, uint32_t nrows,
+                           const uint16_t *seg, uint32_t U, uint32_t K, uint32_t &par, const bsim_syn *syn, uint32_t &events)
 {
     const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1), w = wave_index();
     const uint32_t nsyn = un.nsyn, qoff = (uint32_t)un.part * U;
     const uint64_t lt = (1ull << lane) - 1ull;
-    uint32_t jn = w * WAVE;                     /* first row of the next block to look up */
-    Cursor c;
-    set_range(S, c, 0, nrb);
-    Entries E;
-    pair_u32 ab = {0u, 0u};
-    Block k0, k1;                               /* blocks not yet used up */
+    constexpr uint32_t BROWS = NEV * WAVE * WR; /* rows of a block */
+    uint32_t jn = w * (WR * WAVE);                     /* first row of the next block to look up */
+    Entries<WR> E;
+    pair_u32 ab[WR];
+    Block<WR> k0, k1;                               /* blocks not yet used up */
     uint32_t e0 = 0, e1 = 0, at = 0;            /* ends of k0, k1 and of the stream so far */
     uint32_t q = 1, buf = 0;                    /* how many of k0, k1 are in use */
-    uint32_t left = nrows > NEV * WAVE ? nrows - NEV * WAVE : 0u;    /* rows past the blocks made */
+    uint32_t left = nrows > BROWS ? nrows - BROWS : 0u;    /* rows past the blocks made */
     Step X;
-    load_entries(S, d, c, nrb, jn, nrows, E);
+    load_entries(S, d, seg, R, jn, nrows, E);
     uint32_t nab = E.n;
-    load_rows(d, E, ab);
-    load_entries(S, d, c, nrb, jn += NEV * WAVE, nrows, E);
+    load_rows(S, d, E, ab);
+    load_entries(S, d, seg, R, jn += BROWS, nrows, E);
     make_block(S, ab, nab, 0u, k0);
     nab = E.n;
-    load_rows(d, E, ab);
-    load_entries(S, d, c, nrb, jn += NEV * WAVE, nrows, E);
+    load_rows(S, d, E, ab);
+    load_entries(S, d, seg, R, jn += BROWS, nrows, E);
     if (left > 0) {                                           /* uniform */
         make_block(S, ab, nab, buf = 1u, k1);
         nab = E.n;
-        load_rows(d, E, ab);
-        load_entries(S, d, c, nrb, jn += NEV * WAVE, nrows, E);
-        left = left > NEV * WAVE ? left - NEV * WAVE : 0u;
+        load_rows(S, d, E, ab);
+        load_entries(S, d, seg, R, jn += BROWS, nrows, E);
+        left = left > BROWS ? left - BROWS : 0u;
         q = 2;
     }
     wg_barrier();
@@ -439,13 +479,13 @@ __device__ void event_wave(const Shared &S, const bsim_dev &d, const bsim_unit &
             q--;
         }
         const bool more = q < 2 && left > 0;
-        Block kn;
+        Block<WR> kn;
         if (more) {
             make_block(S, ab, nab, buf ^= 1u, kn);
             nab = E.n;
-            load_rows(d, E, ab);
-            load_entries(S, d, c, nrb, jn += NEV * WAVE, nrows, E);
-            left = left > NEV * WAVE ? left - NEV * WAVE : 0u;
+            load_rows(S, d, E, ab);
+            load_entries(S, d, seg, R, jn += BROWS, nrows, E);
+            left = left > BROWS ? left - BROWS : 0u;
         }
         uint32_t *hist = S.hist + par * (U * (NCOL / 4));
 #pragma unroll
@@ -581,51 +621,44 @@ __device__ void owner_wave(const Shared &S, uint32_t U, uint32_t K, uint32_t &pa
     }
 }
 
-/* Phase (ii) of one batch of up to MAXR source ranges of the unit. */
-template <int NB, int S_>
+/* Phase (ii) of one batch of up to MAXR source chunks of the unit: the event
+ * wavefronts sum the chunks' block counts, one chunk at a time each. */
+template <int NB, int WR, int S_>
 __device__ void deliver_batch(const Shared &S, const bsim_dev &d, const bsim_unit &un, int32_t r0, int32_t nrb,
-                              uint32_t U, uint32_t K, uint32_t &par, const bsim_syn *syn,
+                              int32_t list, uint32_t U, uint32_t K, uint32_t &par, const bsim_syn *syn,
                               uint32_t &events, uint32_t &rows, Acc<S_> &acc)
 {
-    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = threadIdx.x & (WAVE - 1);
     const uint32_t w = wave_index();
-    if (w == 0) {
-        /* range metadata and the cumulative row counts of the batch */
-        constexpr int PER = MAXR / WAVE;
-        uint32_t c[PER], sum = 0;
-#pragma unroll
-        for (int x = 0; x < PER; x++) {
-            const int32_t i = (int32_t)tid * PER + x;
-            c[x] = 0u;
-            if (i < nrb) {
-                const bsim_range r = d.rng[r0 + i];
-                c[x] = d.rng_count[r0 + i];
-                S.lbase[i] = (uint64_t)r.lbase;
-                S.obase[i] = (uint64_t)r.off_base + (uint64_t)un.part;
-                S.stride[i] = r.stride;
+    const uint32_t *cnt = d.seg_count + (int64_t)list * d.nwords;
+    if (w < NEV) {
+        for (int32_t c = (int32_t)w; c < nrb; c += NEV) {
+            const bsim_range r = d.rng[r0 + c];
+            const uint32_t blk = (uint32_t)r.lo / WAVE, nblk = (uint32_t)(r.hi - r.lo) / WAVE;
+            const uint32_t incl = wave_incl_scan(lane < nblk ? cnt[blk + lane] : 0u);
+            S.blk_end[c * BLKS + lane] = incl;
+            if (lane == WAVE - 1) {
+                const uint64_t ob = (uint64_t)r.off_base + (uint64_t)un.part;
+                S.ctot[c] = incl;
+                S.chunk[c] = Chunk{(uint32_t)ob, (uint32_t)(ob >> 32), blk, r.stride};
             }
-            sum += c[x];
         }
-        const uint32_t incl = wave_incl_scan(sum);
-        uint32_t run = incl - sum;
-#pragma unroll
-        for (int x = 0; x < PER; x++) {
-            const int32_t i = (int32_t)tid * PER + x;
-            if (i < nrb) S.cum[i] = run;
-            run += c[x];
-        }
-        if (tid == WAVE - 1) S.cum[nrb] = incl;
     }
     wg_barrier();
-    const uint32_t nrows = uniform(S.cum[nrb]);
+    Rows R;
+    R.nrb = nrb;
+    R.at = 0;
+    R.end = wave_incl_scan((int32_t)lane < nrb ? S.ctot[lane] : 0u);
+    const uint32_t nrows = readlane(R.end, WAVE - 1);
     rows += nrows;
     if (nrows > 0) {                                          /* uniform */
         if (w < NEV)
-            event_wave<NB>(S, d, un, nrb, nrows, U, K, par, syn, events);
+            event_wave<NB, WR>(S, d, un, R, nrows, d.seg + (int64_t)list * d.nwords * (WAVE * d.dmax), U, K, par, syn,
+                           events);
         else
             owner_wave<S_>(S, U, K, par, acc);
     }
-    wg_barrier();               /* the next batch writes the range metadata */
+    wg_barrier();               /* the next batch writes the chunks */
 }
 
 /* The state of an owner thread's neurons that phase (i) reads, loaded
@@ -663,7 +696,68 @@ __device__ __forceinline__ void load_nstate(const bsim_dev &d, int32_t base, con
     }
 }
 
-template <int NB, int S_>
+/* This workgroup of a clocked launch has ended (see device_cycle). */
+__device__ __forceinline__ void count_done(const bsim_dev &d)
+{
+    (void)__hip_atomic_fetch_add(d.done + BSIM_DONE_STRIDE * (blockIdx.x % 8u), (uint64_t)1, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+}
+
+/* Orders the units by their work in the launch before, heaviest first, so that
+ * the hardware dispatches the heavy units of the coming launches before the
+ * light ones (results do not depend on the order; the firing volleys move
+ * slowly against two cycles).  Counting sort over half-octave classes; within
+ * a class the order is arbitrary.  Runs in one workgroup, beside the others of
+ * the launch, and clears the loads that it has read.  The classes of the units
+ * are kept in LDS where they fit. */
+#define RANK_CLASSES 64
+
+__device__ __forceinline__ uint32_t load_class(uint64_t x)
+{
+    if (x < 16) return 0;
+    const uint32_t e = 63u - (uint32_t)__builtin_clzll(x);        /* floor(log2 x) >= 4 */
+    const uint32_t h = (uint32_t)(x >> (e - 1)) & 1u;              /* next bit */
+    return min(2u * (e - 4u) + h + 1u, (uint32_t)RANK_CLASSES - 1u);
+}
+
+__device__ void rank_units(const bsim_dev &d, uint64_t *load, int32_t *perm, uint32_t *lds, uint32_t lds_size)
+{
+    uint32_t *cnt = lds, *fill = cnt + NRES * RANK_CLASSES, *rtot = fill + NRES * RANK_CLASSES;
+    uint8_t *cls = (uint32_t)d.ntiles <= lds_size - 4u * (2 * NRES * RANK_CLASSES + NRES)
+                       ? reinterpret_cast<uint8_t *>(rtot + NRES) : d.tile_cls;
+    const uint32_t tid = threadIdx.x;
+    for (uint32_t i = tid; i < NRES * RANK_CLASSES; i += NTHREAD) cnt[i] = 0u;
+    __syncthreads();
+    for (int32_t k = tid; k < d.ntiles; k += NTHREAD) {
+        const uint32_t c = load_class(load[k]);
+        load[k] = 0ull;
+        cls[k] = (uint8_t)c;
+        atomicAdd(&cnt[d.tile_res[k] * RANK_CLASSES + c], 1u);
+    }
+    __syncthreads();
+    /* exclusive prefix of each residue's class counts, heaviest class first */
+    static_assert(RANK_CLASSES == WAVE && NRES * RANK_CLASSES <= NTHREAD, "a wavefront per residue");
+    if (tid < NRES * RANK_CLASSES) {
+        const uint32_t x = tid / RANK_CLASSES, c = RANK_CLASSES - 1u - tid % RANK_CLASSES;
+        const uint32_t v = cnt[x * RANK_CLASSES + c], incl = wave_incl_scan(v);
+        fill[x * RANK_CLASSES + c] = incl - v;
+        if (c == 0) rtot[x] = incl;
+    }
+    __syncthreads();
+    /* unit of residue x at rank i goes to slot NRES * i + x */
+    for (int32_t k = tid; k < d.ntiles; k += NTHREAD) {
+        const uint32_t x = d.tile_res[k];
+        const uint32_t pos = atomicAdd(&fill[x * RANK_CLASSES + cls[k]], 1u);
+        perm[NRES * pos + x] = k;
+    }
+    /* the remaining slots of each residue are empty */
+    const int32_t per = d.nslots / NRES;
+    for (int32_t i = tid; i < d.nslots; i += NTHREAD) {
+        if (i / NRES >= (int32_t)rtot[i % NRES] && i / NRES < per) perm[i] = -1;
+    }
+}
+
+template <int NB, int WR, int S_>
 __global__ __launch_bounds__(NTHREAD, STEP_EU) void bsim_step_kernel(bsim_dev d, int32_t t, int32_t flags)
 {
     extern __shared__ __align__(16) uint32_t lds[];
@@ -672,27 +766,38 @@ __global__ __launch_bounds__(NTHREAD, STEP_EU) void bsim_step_kernel(bsim_dev d,
         t = device_cycle(d, blockIdx.x % 8u);
         flags = (t > 0 ? 1 : 0) | 2;
     }
-    /* the heaviest tiles come first (bsim_rows_kernel ranks them): their
-     * wavefronts get issue priority on their compute unit, so that they are
-     * not slowed down by the light tiles that fill the unit around them */
-    if (blockIdx.x < HEAVY_WGS) __builtin_amdgcn_s_setprio(3);
+    const int32_t re = d.rank_every;
+    if ((int32_t)blockIdx.x < d.rank_wgs) {
+        if (clocked) {
+            /* orders the units for the launches from the next one on, by the
+             * work that the launch before recorded */
+            if (blockIdx.x == 0 && re > 0 && t > 0 && t % re == 0)
+                rank_units(d, d.tile_load + (int64_t)((t - 1) & 1) * d.ntiles,
+                           d.perm + (int64_t)((t / re) & 1) * d.nslots, lds, (uint32_t)lds_bytes((uint32_t)d.tile));
+            wg_barrier();
+            if (threadIdx.x == 0) count_done(d);
+        }
+        return;
+    }
     const uint32_t U = (uint32_t)d.tile, K = slots_of(U);
-    const int32_t k = d.perm[blockIdx.x];       /* -1: an empty slot */
+    /* the unit, -1: an empty slot; which order: the last ranking's */
+    const int32_t order = re > 0 && t > 0 ? ((t - 1) / re) & 1 : 0;
+    const int32_t k = d.perm[(int64_t)order * d.nslots + blockIdx.x - d.rank_wgs];
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & (WAVE - 1);
     const uint32_t w = wave_index();
 
     Shared S;
     {
-        S.lbase = reinterpret_cast<uint64_t *>(lds);
-        S.obase = S.lbase + MAXR;
-        S.hist = reinterpret_cast<uint32_t *>(S.obase + MAXR);
+        S.chunk = reinterpret_cast<Chunk *>(lds);
+        S.hist = reinterpret_cast<uint32_t *>(S.chunk + MAXR);
         S.mark = S.hist + 2 * U * (NCOL / 4);
         S.slot = reinterpret_cast<float *>(S.mark + 2 * PASS);
-        S.btot = reinterpret_cast<uint32_t *>(S.slot + K * U);
-        S.cum = S.btot + 2 * NEV;
-        S.stride = S.cum + MAXR + 1;
-        S.most = S.stride + MAXR;
+        S.blk_end = reinterpret_cast<uint32_t *>(S.slot + K * U);
+        S.blk_mark = S.blk_end + MAXR * BLKS;
+        S.btot = S.blk_mark + NEV * WAVE;
+        S.ctot = S.btot + 2 * NEV;
+        S.most = S.ctot + MAXR;
         S.last = S.most + 2;
     }
 
@@ -716,20 +821,21 @@ __global__ __launch_bounds__(NTHREAD, STEP_EU) void bsim_step_kernel(bsim_dev d,
         for (uint32_t i = tid; i < 2 * U; i += NTHREAD)
             reinterpret_cast<uint4 *>(S.hist)[i] = make_uint4(0u, 0u, 0u, 0u);
         for (uint32_t i = tid; i < 2 * PASS; i += NTHREAD) S.mark[i] = NO_MARK;
+        if (w < NEV) S.blk_mark[tid] = NO_MARK;
         if (tid < 4) S.most[tid] = 0u;          /* most and last */
         const bsim_syn *syn = d.syn + un.base;
         uint32_t events = 0, rows = 0, par = 0;
         for (int32_t rb = 0; rb < un.nrng; rb += MAXR)
-            deliver_batch<NB, S_>(S, d, un, un.rng0 + rb, min(MAXR, un.nrng - rb), U, K, par, syn, events,
+            deliver_batch<NB, WR, S_>(S, d, un, un.rng0 + rb, min(MAXR, un.nrng - rb), (t - 1) & 1, U, K, par,
+                                  syn, events,
                                   rows, acc);
-        /* the unit's work in this launch, when the row-list launch that
-         * follows ranks the units (it runs for cycle t + 1): its deliveries
-         * plus a fixed cost of two deliveries per active row, x 16 */
+        /* the unit's work in this launch, when the next one ranks the units:
+         * its deliveries plus a fixed cost of two deliveries per active row,
+         * x 16 */
         if (tid == 0 && rows > 0) {
-            const int32_t re = d.rank_every;
             d.ev_count[k] += (int64_t)events;   /* one workgroup per unit and launch */
-            if (clocked && (re == 1 || (re > 1 && (t + 1) % re == 0)))
-                d.tile_load[k] = (uint64_t)events * 16ull + (uint64_t)rows * 32ull;
+            if (clocked && re > 0 && (t + 1) % re == 0)
+                d.tile_load[(int64_t)(t & 1) * d.ntiles + k] = (uint64_t)events * 16ull + (uint64_t)rows * 32ull;
         }
     }
 
@@ -740,7 +846,8 @@ __global__ __launch_bounds__(NTHREAD, STEP_EU) void bsim_step_kernel(bsim_dev d,
         const int32_t base = k * (int32_t)U;
         const uint64_t *hist_in = d.hist + (int64_t)((t - 1) & 1) * d.n;
         uint64_t *hist_out = d.hist + (int64_t)(t & 1) * d.n;
-        uint64_t *act_out = d.active + (int64_t)(t & 1) * d.nwords;
+        uint32_t *cnt_out = d.seg_count + (int64_t)(t & 1) * d.nwords;
+        uint16_t *seg_out = d.seg + (int64_t)(t & 1) * d.nwords * (WAVE * D);
         const bool rec = d.raster != nullptr && t >= d.rec_t0 && t < d.rec_t0 + d.rec_steps;
 #pragma unroll
         for (int j = 0; j < S_; j++) {
@@ -826,186 +933,20 @@ __global__ __launch_bounds__(NTHREAD, STEP_EU) void bsim_step_kernel(bsim_dev d,
                 }
             }
             const uint64_t fm = ballot64(fired);
-            const uint64_t am = ballot64(valid && ((h >> 1) & dmask) != 0);
-            if (lane == 0 && n0 < d.n) {
-                act_out[n0 / 64] = am;
-                if (rec) d.raster[(int64_t)(t - d.rec_t0) * d.nwords + n0 / 64] = fm;
+            /* the block's list of active rows: each neuron's delays that
+             * deliver in phase (ii) of this cycle, in order */
+            uint64_t m = valid ? (h >> 1) & dmask : 0ull;
+            const uint32_t c = (uint32_t)__popcll(m), incl = wave_incl_scan(c);
+            if (n0 < d.n) {                                   /* uniform */
+                uint16_t *out = seg_out + (int64_t)(n0 / 64) * (WAVE * D) + (incl - c);
+                for (; m; m &= m - 1) *out++ = (uint16_t)(lane << 6 | (uint32_t)__builtin_ctzll(m));
+                if (lane == WAVE - 1) cnt_out[n0 / 64] = incl;
+                if (lane == 0 && rec) d.raster[(int64_t)(t - d.rec_t0) * d.nwords + n0 / 64] = fm;
             }
         }
     }
     if (clocked) wg_barrier();      /* every wavefront has read the cycle */
-    if (clocked && tid == 0)
-        (void)__hip_atomic_fetch_add(d.done + BSIM_DONE_STRIDE * (blockIdx.x % 8u), (uint64_t)1,
-                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-/* Orders the tiles by their work in the step launch just finished, heaviest
- * first, so that the hardware dispatches the heavy tiles of the coming launch
- * before the light ones (results do not depend on the order; the firing
- * volleys move slowly against one cycle).  A tile's work, accumulated by its
- * own step workgroup, is its deliveries plus a fixed cost of two deliveries
- * per active row.  Counting sort over half-octave classes; within a class the
- * order is arbitrary.  Runs in one workgroup of ROWS_THREADS threads, which
- * also clears the loads for the next ranking. */
-#define RANK_CLASSES 128
-
-__device__ __forceinline__ uint32_t load_class(uint64_t x)
-{
-    if (x < 2) return 0;
-    const uint32_t e = 63u - (uint32_t)__builtin_clzll(x);        /* floor(log2 x) >= 1 */
-    const uint32_t h = (uint32_t)(x >> (e - 1)) & 1u;              /* next bit */
-    return min(2u * e + h, (uint32_t)RANK_CLASSES - 1u);
-}
-
-#define RANK_LDS_TILES 16384   /* tile classes kept in LDS up to this many tiles */
-#define NRES 8                  /* XCDs: workgroup w runs on XCD (w + c) mod 8 */
-#define RANK_REG 4              /* tiles per thread kept in registers, up to RANK_REG * ROWS_THREADS tiles */
-
-__device__ void rank_tiles(const bsim_dev &d)
-{
-    __shared__ uint32_t cnt[NRES][RANK_CLASSES], fill[NRES][RANK_CLASSES], rtot[NRES];
-    __shared__ uint8_t cls_lds[RANK_LDS_TILES];
-    const uint32_t tid = threadIdx.x;
-    const bool in_lds = d.ntiles <= RANK_LDS_TILES;
-    uint8_t *cls = in_lds ? cls_lds : d.tile_cls;
-    const bool in_regs = d.ntiles <= RANK_REG * ROWS_THREADS;
-    uint32_t xr[RANK_REG], cr[RANK_REG];
-    for (uint32_t i = tid; i < NRES * RANK_CLASSES; i += ROWS_THREADS) (&cnt[0][0])[i] = 0u;
-    if (in_regs) {              /* all loads of a thread issued together */
-        uint64_t ld[RANK_REG];
-#pragma unroll
-        for (int i = 0; i < RANK_REG; i++) {
-            const int32_t k = (int32_t)tid + i * ROWS_THREADS;
-            ld[i] = (k < d.ntiles) ? d.tile_load[k] : 0ull;
-            xr[i] = (k < d.ntiles) ? d.tile_res[k] : 0u;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < RANK_REG; i++) {
-            const int32_t k = (int32_t)tid + i * ROWS_THREADS;
-            cr[i] = load_class(ld[i]);
-            if (k < d.ntiles) {
-                d.tile_load[k] = 0ull;
-                atomicAdd(&cnt[xr[i]][cr[i]], 1u);
-            }
-        }
-    } else {
-        __syncthreads();
-        for (int32_t k = tid; k < d.ntiles; k += ROWS_THREADS) {
-            /* written by other workgroups' atomics in L2; this workgroup never read it */
-            const uint32_t c = load_class(d.tile_load[k]);
-            cls[k] = (uint8_t)c;
-            d.tile_load[k] = 0ull;
-            atomicAdd(&cnt[d.tile_res[k]][c], 1u);
-        }
-    }
-    __syncthreads();
-    /* exclusive prefix of each residue's class counts, heaviest class first:
-     * thread t takes residue t / RANK_CLASSES, class RANK_CLASSES - 1 - t mod
-     * RANK_CLASSES (two wavefronts per residue) */
-    static_assert(NRES * RANK_CLASSES == ROWS_THREADS && RANK_CLASSES == 2 * WAVE, "one thread per class");
-    {
-        __shared__ uint32_t half[ROWS_THREADS / WAVE];
-        const uint32_t x = tid / RANK_CLASSES, c = RANK_CLASSES - 1u - tid % RANK_CLASSES;
-        const uint32_t v = cnt[x][c];
-        const uint32_t incl = wave_incl_scan(v);
-        if ((tid & (WAVE - 1)) == WAVE - 1) half[tid / WAVE] = incl;
-        __syncthreads();
-        const uint32_t carry = ((tid / WAVE) & 1u) ? half[tid / WAVE - 1] : 0u;
-        fill[x][c] = carry + incl - v;
-        if (tid % RANK_CLASSES == RANK_CLASSES - 1u) rtot[x] = carry + incl;
-    }
-    __syncthreads();
-    /* tile of residue x at rank i goes to workgroup NRES * i + x */
-    if (in_regs) {
-#pragma unroll
-        for (int i = 0; i < RANK_REG; i++) {
-            const int32_t k = (int32_t)tid + i * ROWS_THREADS;
-            if (k < d.ntiles) {
-                const uint32_t pos = atomicAdd(&fill[xr[i]][cr[i]], 1u);
-                d.perm[NRES * pos + xr[i]] = k;
-            }
-        }
-    } else {
-        for (int32_t k = tid; k < d.ntiles; k += ROWS_THREADS) {
-            const uint32_t x = d.tile_res[k];
-            const uint32_t pos = atomicAdd(&fill[x][cls[k]], 1u);
-            d.perm[NRES * pos + x] = k;
-        }
-    }
-    /* the remaining slots of each residue are empty */
-    const int32_t per = d.nslots / NRES;
-    for (int32_t sidx = tid; sidx < d.nslots; sidx += ROWS_THREADS) {
-        const int32_t x = sidx % NRES, i = sidx / NRES;
-        if (i >= (int32_t)rtot[x] && i < per) d.perm[sidx] = -1;
-    }
-}
-
-/* The row-list kernel, launched after every update: one workgroup per source
- * chunk (at most BSIM_CHUNK = 4 * ROWS_THREADS pres) builds the chunk's list
- * of active (pre, delay) rows, ascending, from the history words the update
- * just wrote: every thread reads the words of 4 consecutive pres (coalesced),
- * counts their active delays, and a workgroup prefix places the rows.  The
- * lists are read by every tile that receives from the chunk. */
-__global__ __launch_bounds__(ROWS_THREADS) void bsim_rows_kernel(bsim_dev d)
-{
-    __shared__ uint32_t scr[ROWS_THREADS / WAVE];
-    const int32_t u = blockIdx.x;
-    /* the coming step launch's cycle (the step launch before this one has
-     * completed, so it is the same for every workgroup of this launch) */
-    const int32_t cyc = device_cycle(d, 0);
-    /* one workgroup more than source chunks: it ranks the tiles every
-     * d.rank_every cycles, from the work the step launch just recorded,
-     * while the others build the lists */
-    if (u == d.nsrc) {
-        const bool rank = d.rank_every == 1 || (d.rank_every > 1 && cyc % d.rank_every == 0);
-        if (rank) rank_tiles(d);
-        return;
-    }
-    const uint32_t tid = threadIdx.x;
-    const uint32_t lane = tid & (WAVE - 1);
-    const uint32_t w = tid / WAVE;
-    const int32_t lo = d.src_lo[u], hi = d.src_hi[u];
-    const int32_t par = (cyc - 1) & 1;             /* parity of the last update */
-    const uint64_t *hist = d.hist + (int64_t)par * d.n;
-    uint32_t *out = d.src_list + d.src_list_base[u];
-    const int32_t D = d.dmax;
-    const uint64_t dmask = (D >= 63) ? (~0ull >> 1) : ((1ull << D) - 1ull);
-    const int32_t p0 = lo + 4 * (int32_t)tid;
-    uint64_t m[4];
-    uint32_t cnt = 0;
-#pragma unroll
-    for (int x = 0; x < 4; x++) {
-        m[x] = (p0 + x < hi) ? ((hist[p0 + x] >> 1) & dmask) : 0ull;
-        cnt += (uint32_t)__popcll(m[x]);
-    }
-    const uint32_t incl = wave_incl_scan(cnt);
-    if (lane == WAVE - 1) scr[w] = incl;
-    __syncthreads();
-    uint32_t pos = incl - cnt, tot = 0;
-#pragma unroll
-    for (int i = 0; i < ROWS_THREADS / WAVE; i++) {
-        const uint32_t x = scr[i];
-        pos += ((uint32_t)i < w) ? x : 0u;
-        tot += x;
-    }
-#pragma unroll
-    for (int x = 0; x < 4; x++) {
-        const uint32_t rb = (uint32_t)(p0 + x - lo) * (uint32_t)D;
-        for (uint64_t mm = m[x]; mm; mm &= mm - 1) out[pos++] = rb + (uint32_t)__builtin_ctzll(mm);
-    }
-    /* for every tile that reads this chunk: the list's length in the tile's
-     * range entry */
-    for (int64_t x = d.chunk_tiles_off[u] + tid; x < d.chunk_tiles_off[u + 1]; x += ROWS_THREADS)
-        d.rng_count[d.chunk_rng[x]] = tot;
-}
-
-extern "C" hipError_t bsim_launch_rows(const bsim_dev *d, hipStream_t stream)
-{
-    if (d->nsrc <= 0) return hipSuccess;
-    (void)hipGetLastError();       /* the check below then reports this launch alone */
-    hipLaunchKernelGGL(bsim_rows_kernel, dim3(d->nsrc + 1), dim3(ROWS_THREADS), 0, stream, *d);
-    return hipGetLastError();
+    if (clocked && tid == 0) count_done(d);
 }
 
 extern "C" hipError_t bsim_launch_step(const bsim_dev *d, int32_t t, int32_t flags,
@@ -1014,15 +955,21 @@ extern "C" hipError_t bsim_launch_step(const bsim_dev *d, int32_t t, int32_t fla
     if (d->ntiles <= 0) return hipSuccess;
     const uint32_t U = (uint32_t)d->tile;
     if (U == 0 || U % WAVE != 0 || U > BSIM_MAX_UNIT) return hipErrorInvalidValue;
-    const dim3 grid(d->nslots), block(NTHREAD);
+    const dim3 grid(d->nslots + d->rank_wgs), block(NTHREAD);
     const size_t lds = lds_bytes(U);
     (void)hipGetLastError();       /* the check below then reports this launch alone */
-#define STEP(NB, S_) hipLaunchKernelGGL((bsim_step_kernel<NB, S_>), grid, block, lds, stream, *d, t, flags)
 #define OWN(X) (((X) + NOWN * WAVE - 1) / (NOWN * WAVE))
-    if (U <= 64) STEP(6, OWN(64));
-    else if (U <= 128) STEP(7, OWN(128));
-    else if (U <= 256) STEP(8, OWN(256));
-    else STEP(9, OWN(512));
+#define STEP(NB, X)                                                                                             \
+    do {                                                                                                        \
+        if (d->wrows == 2)                                                                                      \
+            hipLaunchKernelGGL((bsim_step_kernel<NB, 2, OWN(X)>), grid, block, lds, stream, *d, t, flags);      \
+        else                                                                                                    \
+            hipLaunchKernelGGL((bsim_step_kernel<NB, 1, OWN(X)>), grid, block, lds, stream, *d, t, flags);      \
+    } while (0)
+    if (U <= 64) STEP(6, 64);
+    else if (U <= 128) STEP(7, 128);
+    else if (U <= 256) STEP(8, 256);
+    else STEP(9, 512);
 #undef OWN
 #undef STEP
     return hipGetLastError();

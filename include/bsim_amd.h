@@ -180,9 +180,9 @@ int32_t bsim_sim_read_state(bsim_sim *sim, float *v, float *ie, float *ii, int32
                             int32_t *fire_count);
 
 /* Advances n cycles one launch at a time with a pair of HIP events around
- * each of the cycle's two kernels on the simulation's stream (the step
- * kernel, then the active-row list kernel), synchronises, and returns their
- * mean durations in microseconds.  For measurement; bsim_sim_step is the
+ * the cycle's kernel on the simulation's stream, synchronises, and returns
+ * its mean duration in microseconds in step_us, and 0 in rows_us (the step
+ * kernel makes the active-row lists itself).  For measurement; bsim_sim_step is the
  * production path (graph-replayed, no events). */
 int32_t bsim_sim_time_steps(bsim_sim *sim, int32_t n, double *step_us, double *rows_us);
 
@@ -217,9 +217,11 @@ void *bsim_sim_stream(bsim_sim *sim);
 /* Tile schedule (no counterpart in the reference, whose per-type launches
  * take the neurons and synapses in id order with a fixed grid,
  * SingleGPUSimulator.cu:100, 165-171): the order in which the
- * step's workgroups take the tiles.  Every rank_every cycles the row-list
- * launch ranks the tiles by their work in the step launch before it,
- * heaviest first (the default, 2); 0 keeps the tiles in their last order.
+ * step's workgroups take the tiles.  Every rank_every cycles one
+ * workgroup ranks the tiles for the launches after it by their work in the
+ * launch before, heaviest first (the default, 2); 0 keeps the tiles in their
+ * first order.  So many workgroups run at a time that a small network's
+ * order is nothing; it is not ranked.
  * Results do not depend on it.  Takes effect from the next step. */
 int32_t bsim_sim_set_schedule(bsim_sim *sim, int32_t rank_every);
 
