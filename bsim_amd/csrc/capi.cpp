@@ -453,7 +453,7 @@ static bsim_sim *sim_from_layout(bsim::Layout &L, const bsim_sim_config &c, bsim
                                  int64_t dev_syn_bytes)
 {
     hipError_t e = hipSuccess;
-    std::vector<uint8_t> res;      /* XCD residue of each unit */
+    std::vector<int32_t> perm;
     bsim_sim *sim = new (std::nothrow) bsim_sim();
     if (!sim) {
         if (dev_syn) (void)hipFree(dev_syn);
@@ -497,24 +497,36 @@ static bsim_sim *sim_from_layout(bsim::Layout &L, const bsim_sim_config &c, bsim
     UP(bern_seed, L.bern_seed);
     UP(bern_key, L.bern_key);
     UP(pois_tab, L.pois_tab);
-    res.resize((size_t)d.ntiles);
+    d.nslots = L.nslots * L.parts;
+    d.rank_wgs = d.nslots > kResident ? 8 : 0;
     {
-        std::vector<bsim_unit> unit((size_t)d.ntiles);
+        /* the units of each residue in order (until the first ranking) */
+        std::vector<bsim_unit> unit((size_t)(d.rank_wgs ? d.ntiles : d.nslots));
+        std::vector<uint8_t> res((size_t)d.ntiles);
+        std::vector<int32_t> used(8, 0);
+        for (auto &x : unit) x.id = -1;
+        perm.assign((size_t)std::max(d.nslots, 1), -1);
         for (int32_t u = 0; u < d.ntiles; u++) {
             const int32_t t = u / L.parts;
-            bsim_unit &x = unit[u];
+            res[u] = L.tile_res[t];
+            const int32_t slot = 8 * used[res[u]]++ + res[u];
+            perm[(size_t)slot] = u;
+            bsim_unit &x = unit[(size_t)(d.rank_wgs ? u : slot)];
             x.base = L.tile_base[t];
             x.nsyn = L.tile_nsyn[t];
+            x.id = u;
             x.rng0 = L.tile_rng[t];
             x.nrng = L.tile_rng[t + 1] - L.tile_rng[t];
             x.part = u % L.parts;
-            x.pad[0] = x.pad[1] = 0;
-            res[u] = L.tile_res[t];
+            for (int32_t c = 0; c < std::min(x.nrng, BSIM_UNIT_CHUNKS); c++) {
+                const bsim_range &r = L.rng[(size_t)x.rng0 + c];
+                x.chunk[c] = bsim_chunk{r.off_base + x.part, (uint32_t)r.lo / 64, (uint32_t)(r.hi - r.lo) / 64,
+                                        r.stride, 0};
+            }
         }
         UP(unit, unit);
         UP(tile_res, res);
     }
-    d.nslots = L.nslots * L.parts;
     {
         /* an event thread takes two rows at a time where a unit has many rows
          * of few events: a block of 512 rows then leaves a pass of 1,024 events
@@ -564,20 +576,10 @@ static bsim_sim *sim_from_layout(bsim::Layout &L, const bsim_sim_config &c, bsim
         if (!(d.done = dev_alloc<uint64_t>(sim, 8 * BSIM_DONE_STRIDE, e))) goto hip_fail;
         if ((e = hipMemsetAsync(d.done, 0, 8 * BSIM_DONE_STRIDE * sizeof(uint64_t), sim->stream)) != hipSuccess)
             goto hip_fail;
-        {
-            /* until the first ranking: the tiles of each residue in order */
-            std::vector<int32_t> perm((size_t)(d.nslots > 0 ? d.nslots : 1), -1);
-            std::vector<int32_t> rank(8, 0);
-            for (int32_t t = 0; t < d.ntiles; t++) {
-                const int x = res[t];
-                perm[(size_t)8 * rank[x]++ + x] = t;
-            }
-            perm.insert(perm.end(), perm.begin(), perm.end());        /* both orders */
-            d.perm = dev_upload(sim, perm, e);
-            if (e != hipSuccess) goto hip_fail;
-        }
+        perm.insert(perm.end(), perm.begin(), perm.end());        /* both orders */
+        d.perm = dev_upload(sim, perm, e);
+        if (e != hipSuccess) goto hip_fail;
         d.rank_every = kRankEvery;
-        d.rank_wgs = d.nslots > kResident ? 8 : 0;
         d.done_inv = d.nslots >= 8 ? 8.0 / (double)(d.nslots + d.rank_wgs) : 0.0;
         if (!(d.tile_load = dev_alloc<uint64_t>(sim, 2 * nt, e))) goto hip_fail;
         if ((e = hipMemsetAsync(d.tile_load, 0, 2 * nt * sizeof(uint64_t), sim->stream)) != hipSuccess) goto hip_fail;

@@ -60,14 +60,28 @@ enum { BSIM_KIND_LIF = 0, BSIM_KIND_ARRAY = 1, BSIM_KIND_BERNOULLI = 2, BSIM_KIN
  * with u < tab[1 + j], or J - 1 when there is none. */
 #define BSIM_POISSON_MAX_RATE 1.0e6f
 
+/* A source chunk of a unit. */
+typedef struct bsim_chunk {
+    int64_t off_base;   /* off_tab index of the unit's entry of the chunk's first row */
+    uint32_t blk;       /* first block of 64 pres */
+    uint32_t nblk;      /* blocks */
+    uint32_t stride;    /* off_tab entries per (pre, delay) row of the group */
+    uint32_t pad;
+} bsim_chunk;
+
+#define BSIM_UNIT_CHUNKS 4
+
 /* A unit: the targets of one step workgroup -- a whole tile, or one part of
- * it. */
+ * it.  Its first chunks are here and not only among the range entries: one
+ * dependent load less for most units. */
 typedef struct __attribute__((aligned(32))) bsim_unit {
     int64_t base;       /* first synapse of the tile's group */
     uint32_t nsyn;      /* synapses of the group */
+    int32_t id;         /* the unit, -1: none */
     int32_t rng0, nrng; /* the tile's range entries */
     int32_t part;       /* part of the tile (0 for a whole tile) */
-    int32_t pad[2];
+    int32_t pad;
+    bsim_chunk chunk[BSIM_UNIT_CHUNKS];
 } bsim_unit;
 
 typedef struct bsim_range {
@@ -133,7 +147,7 @@ typedef struct bsim_dev {
     /* synapses */
     int32_t nslots;             /* step workgroups (units placed by XCD residue) */
     int32_t wrows;              /* rows that an event thread takes at a time, 1 or 2 */
-    const bsim_unit *unit;      /* [ntiles] */
+    const bsim_unit *unit;      /* [ntiles], or [nslots] in slot order where every unit has a workgroup */
     const uint8_t *tile_res;    /* [ntiles] XCD residue of the unit's group */
     const bsim_syn *syn;        /* [S] target and weight of each synapse, group-major */
     const bsim_range *rng;
@@ -154,8 +168,8 @@ typedef struct bsim_dev {
     uint64_t *tile_load;        /* [2][ntiles] work of a launch before a ranking (x 16), by cycle parity */
     int32_t rank_every;         /* units ranked heaviest first every this many cycles (0: never,
                                    the units stay in their initial order) */
-    int32_t rank_wgs;           /* workgroups before the slots' (the first ranks): 8, or 0 where every unit
-                                   runs at once and order is nothing */
+    int32_t rank_wgs;           /* workgroups before the others (the first ranks): 8, or 0 where every
+                                   unit has a workgroup and order is nothing */
     uint8_t *tile_cls;          /* [ntiles] half-octave class of a unit's work */
     uint64_t *raster;           /* [rec_steps][nwords] fired bitmaps, or NULL */
     int32_t rec_steps;

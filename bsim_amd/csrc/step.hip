@@ -31,7 +31,13 @@
  * it, and sort the pass by target, keeping stream order (event_wave); the NOWN
  * owner wavefronts, whose threads hold the targets' E and I accumulators in
  * registers, add a pass's events while the event wavefronts prepare the next
- * (owner_wave).  Every accumulator thus receives its adds one at a time in
+ * (owner_wave), and update the targets in the end (update_unit).  The two kinds
+ * of wavefront have no code in common from the workgroup's first batch to its
+ * end (event_unit, owner_unit): with one body for both, branching at each
+ * phase, the compiler kept the state of either alive in the other, 69 vector
+ * registers and no room to load anything early, against 52; us per cycle of
+ * 48 neurons 8.2 / 7.2, 9,896 9.1 / 7.2, 330,000 61.3 / 59.9, a sweep of
+ * 300 chains 45.2 / 42.4.  Every accumulator thus receives its adds one at a time in
  * stream order, (pre, delay, creation) -- the creation order the host
  * verified -- so the sums are the reference's sequential fp32 sums, bit for
  * bit, with no floating-point atomics.
@@ -88,7 +94,7 @@ __host__ __device__ constexpr uint32_t slots_of(uint32_t U)
 __host__ __device__ constexpr size_t lds_bytes(uint32_t U)
 {
     return 16 * MAXR + 2 * U * NCOL + 8 * PASS + 4 * slots_of(U) * U + 4 * MAXR * BLKS + 4 * NEV * WAVE + 8 * NEV +
-           4 * MAXR + 16;
+           8 * MAXR + 16;
 }
 
 __device__ __forceinline__ uint32_t bern_hash(uint64_t seed, uint32_t id, uint32_t t)
@@ -190,7 +196,7 @@ struct Shared {
     uint32_t *blk_end;          /* [MAXR][BLKS] active rows of a chunk up to the end of each of its blocks */
     uint32_t *blk_mark;         /* [NEV][64] first rows of blocks among 64 rows (load_entries), else NO_MARK */
     uint32_t *btot;             /* [2][NEV] stream length of each event wavefront's rows of a block */
-    uint32_t *ctot;             /* [MAXR] active rows of each chunk */
+    uint32_t *ctot;             /* [2][MAXR] active rows of each chunk */
     uint32_t *most;             /* [2] largest rank of a pass's events beyond the slots */
     uint32_t *last;             /* [2] the pass is the batch's last */
 };
@@ -406,11 +412,10 @@ __device__ __forceinline__ uint32_t byte_sum(uint32_t x, uint32_t acc) { return 
  * pass before, the table entries and list entries one and two blocks ahead of
  * the rows that the marks are put from. */
 template <int NB, int WR>
-__device__ void event_wave(const Shared &S, const bsim_dev &d, const bsim_unit &un, Rows &R, uint32_t nrows,
+__device__ void event_wave(const Shared &S, const bsim_dev &d, uint32_t qoff, uint32_t nsyn, Rows &R, uint32_t nrows,
                            const uint16_t *seg, uint32_t U, uint32_t K, uint32_t &par, const bsim_syn *syn, uint32_t &events)
 {
     const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1), w = wave_index();
-    const uint32_t nsyn = un.nsyn, qoff = (uint32_t)un.part * U;
     const uint64_t lt = (1ull << lane) - 1ull;
     constexpr uint32_t BROWS = NEV * WAVE * WR; /* rows of a block */
     uint32_t jn = w * (WR * WAVE);                     /* first row of the next block to look up */
@@ -621,44 +626,37 @@ __device__ void owner_wave(const Shared &S, uint32_t U, uint32_t K, uint32_t &pa
     }
 }
 
-/* Phase (ii) of one batch of up to MAXR source chunks of the unit: the event
- * wavefronts sum the chunks' block counts, one chunk at a time each. */
-template <int NB, int WR, int S_>
-__device__ void deliver_batch(const Shared &S, const bsim_dev &d, const bsim_unit &un, int32_t r0, int32_t nrb,
-                              int32_t list, uint32_t U, uint32_t K, uint32_t &par, const bsim_syn *syn,
-                              uint32_t &events, uint32_t &rows, Acc<S_> &acc)
+/* Event wavefronts: where the batch's source chunks lie and how many active
+ * rows each of their blocks has, one chunk at a time each.  The first
+ * BSIM_UNIT_CHUNKS of a unit are in its record. */
+__device__ __forceinline__ void prepare_batch(const Shared &S, const bsim_dev &d, const bsim_unit *un, int32_t rb,
+                                              int32_t nrb, int32_t list, uint32_t buf)
 {
     const uint32_t lane = threadIdx.x & (WAVE - 1);
-    const uint32_t w = wave_index();
     const uint32_t *cnt = d.seg_count + (int64_t)list * d.nwords;
-    if (w < NEV) {
-        for (int32_t c = (int32_t)w; c < nrb; c += NEV) {
-            const bsim_range r = d.rng[r0 + c];
-            const uint32_t blk = (uint32_t)r.lo / WAVE, nblk = (uint32_t)(r.hi - r.lo) / WAVE;
-            const uint32_t incl = wave_incl_scan(lane < nblk ? cnt[blk + lane] : 0u);
-            S.blk_end[c * BLKS + lane] = incl;
-            if (lane == WAVE - 1) {
-                const uint64_t ob = (uint64_t)r.off_base + (uint64_t)un.part;
-                S.ctot[c] = incl;
-                S.chunk[c] = Chunk{(uint32_t)ob, (uint32_t)(ob >> 32), blk, r.stride};
-            }
+    for (int32_t c = (int32_t)wave_index(); c < nrb; c += NEV) {
+        uint64_t ob;
+        uint32_t blk, nblk, st;
+        if (rb + c < BSIM_UNIT_CHUNKS) {
+            const bsim_chunk h = un->chunk[rb + c];
+            ob = (uint64_t)h.off_base;
+            blk = h.blk;
+            nblk = h.nblk;
+            st = h.stride;
+        } else {
+            const bsim_range r = d.rng[un->rng0 + rb + c];
+            ob = (uint64_t)r.off_base + (uint64_t)un->part;
+            blk = (uint32_t)r.lo / WAVE;
+            nblk = (uint32_t)(r.hi - r.lo) / WAVE;
+            st = r.stride;
+        }
+        const uint32_t incl = wave_incl_scan(lane < nblk ? cnt[blk + lane] : 0u);
+        S.blk_end[c * BLKS + lane] = incl;
+        if (lane == WAVE - 1) {
+            S.ctot[buf * MAXR + c] = incl;
+            S.chunk[c] = Chunk{(uint32_t)ob, (uint32_t)(ob >> 32), blk, st};
         }
     }
-    wg_barrier();
-    Rows R;
-    R.nrb = nrb;
-    R.at = 0;
-    R.end = wave_incl_scan((int32_t)lane < nrb ? S.ctot[lane] : 0u);
-    const uint32_t nrows = readlane(R.end, WAVE - 1);
-    rows += nrows;
-    if (nrows > 0) {                                          /* uniform */
-        if (w < NEV)
-            event_wave<NB, WR>(S, d, un, R, nrows, d.seg + (int64_t)list * d.nwords * (WAVE * d.dmax), U, K, par, syn,
-                           events);
-        else
-            owner_wave<S_>(S, U, K, par, acc);
-    }
-    wg_barrier();               /* the next batch writes the chunks */
 }
 
 /* The state of an owner thread's neurons that phase (i) reads, loaded
@@ -675,6 +673,7 @@ struct NState {
     int32_t refrac[S_];
     float v[S_], ie[S_], ii[S_], vtmp[S_];
     uint64_t hist[S_];
+    bsim_lifc c[S_];
 };
 
 template <int S_>
@@ -694,6 +693,15 @@ __device__ __forceinline__ void load_nstate(const bsim_dev &d, int32_t base, con
         ns.vtmp[j] = d.v_tmp[x];
         ns.hist[j] = hist_in[x];
     }
+}
+
+/* The neurons' parameter sets, once their classes have arrived. */
+template <int S_>
+__device__ __forceinline__ void load_params(const bsim_dev &d, NState<S_> &ns)
+{
+#pragma unroll
+    for (int j = 0; j < S_; j++)
+        ns.c[j] = d.lifc[ns.cls[j] >> 30 == BSIM_KIND_LIF ? ns.cls[j] & BSIM_CLS_SET_MASK : 0u];
 }
 
 /* This workgroup of a clocked launch has ended (see device_cycle). */
@@ -757,6 +765,212 @@ __device__ void rank_units(const bsim_dev &d, uint64_t *load, int32_t *perm, uin
     }
 }
 
+/* The kernel's first argument, read again from its segment: the compiler keeps
+ * what it loads from here in registers only while it is used, and not, as the
+ * argument's own fields, from the kernel's start to its end (some sixty pointers
+ * and sizes: 77 to 82 scalar registers went to spills with units of 384; a sweep
+ * of 96 chains 28.5 us per cycle so, 27.7 with this). */
+__device__ __forceinline__ const bsim_dev &args_again()
+{
+    typedef const __attribute__((address_space(4))) char *kptr;
+    kptr p = (kptr)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const bsim_dev *)p;
+}
+
+/* Phase (i) of cycle t: an owner thread updates its targets of unit id, with
+ * the input that phase (ii) left in acc. */
+template <int S_, bool PRE>
+__device__ __forceinline__ void update_unit(int32_t id, int32_t t, uint32_t U, const Acc<S_> &acc,
+                                            const NState<PRE ? S_ : 1> &ns)
+{
+    const uint32_t lane = threadIdx.x & (WAVE - 1), w = wave_index();
+    const bsim_dev &d = args_again();
+    const int32_t D = d.dmax;
+    const uint64_t dmask = (D >= 63) ? (~0ull >> 1) : ((1ull << D) - 1ull);
+    const int32_t base = id * (int32_t)U;
+    const uint64_t *hist_in = d.hist + (int64_t)((t - 1) & 1) * d.n;
+    uint64_t *hist_out = d.hist + (int64_t)(t & 1) * d.n;
+    uint32_t *cnt_out = d.seg_count + (int64_t)(t & 1) * d.nwords;
+    uint16_t *seg_out = d.seg + (int64_t)(t & 1) * d.nwords * (WAVE * D);
+    const bool rec = d.raster != nullptr && t >= d.rec_t0 && t < d.rec_t0 + d.rec_steps;
+#pragma unroll
+    for (int j = 0; j < S_; j++) {
+        const uint32_t i0 = (w - NEV) * WAVE + j * (NOWN * WAVE);
+        if (i0 >= U) continue;                            /* uniform */
+        const int32_t n0 = base + (int32_t)i0;
+        const int32_t nid = n0 + (int32_t)lane;
+        const bool valid = nid < d.n;
+        bool fired = false;
+        uint64_t h = 0;
+        if (valid) {
+            uint32_t cls;
+            int32_t rs;
+            float v, ie, ii, vtmp;
+            uint64_t hin;
+            if constexpr (PRE) {
+                cls = ns.cls[j]; rs = ns.refrac[j]; v = ns.v[j]; ie = ns.ie[j]; ii = ns.ii[j];
+                vtmp = ns.vtmp[j]; hin = ns.hist[j];
+            } else {
+                cls = d.ncls[nid]; rs = d.refrac[nid]; v = d.v[nid]; ie = d.ie[nid]; ii = d.ii[nid];
+                vtmp = d.v_tmp[nid]; hin = hist_in[nid];
+            }
+            const uint32_t kind = cls >> 30;
+            if (kind == BSIM_KIND_LIF) {
+                const float inE = acc.e[j];
+                const float inI = acc.i[j];
+                if (rs > 0) {
+                    d.refrac[nid] = rs - 1;
+                } else {
+                    bsim_lifc c;
+                    if constexpr (PRE) c = ns.c[j]; else c = d.lifc[cls & BSIM_CLS_SET_MASK];
+                    v = c.Cm * v + vtmp + ie * c.C_E + ii * c.C_I;
+                    ie = c.CE * ie;
+                    ii = c.CI * ii;
+                    if (v >= c.v_thresh) {
+                        fired = true;
+                        d.refrac[nid] = c.refrac_time - 1;
+                        v = c.v_reset;
+                    } else {
+                        if (d.in_sum) d.in_sum[nid] = d.in_sum[nid] + (inE + inI);
+                        ie += inE;
+                        ii += inI;
+                    }
+                    d.v[nid] = v;
+                    d.ie[nid] = ie;
+                    d.ii[nid] = ii;
+                }
+            } else if (kind == BSIM_KIND_ARRAY) {
+                const int32_t c = d.arr_cur[nid];
+                if (c < d.arr_end[nid] && d.arr_t[c] <= t) {
+                    fired = true;
+                    d.arr_cur[nid] = c + 1;
+                }
+            } else if (kind == BSIM_KIND_POISSON) {
+                /* PoissonNeuron::update (src/neuron/poisson/PoissonNeuron.cpp:52-63):
+                 * fire at the drawn cycle before the end cycle, then draw
+                 * the next one 1 + X cycles later */
+                const int32_t nx = d.arr_cur[nid];
+                if (t == nx && nx < d.arr_end[nid]) {
+                    fired = true;
+                    const uint32_t x = poisson_pick(d.pois_tab + d.bern_p[nid],
+                                                    bern_hash(d.bern_seed[nid], d.bern_key[nid], (uint32_t)t));
+                    d.arr_cur[nid] = (int32_t)min((int64_t)nx + 1 + x, (int64_t)0x7FFFFFFF);
+                }
+            } else {
+                fired = bern_hash(d.bern_seed[nid], d.bern_key[nid], (uint32_t)t) < d.bern_p[nid];
+            }
+            h = (hin << 1) | (fired ? 1ull : 0ull);
+            hist_out[nid] = h;
+            if (d.slot_count) d.slot_count[nid] += __popcll((h >> 1) & dmask);
+            if (fired) d.fire_count[nid] += 1;
+            if (rec && d.rec_index) {
+                const int32_t ri = d.rec_index[nid];
+                if (ri >= 0) {
+                    const int64_t o = (int64_t)(t - d.rec_t0) * d.n_rec + ri;
+                    d.rec_v[o] = kind == BSIM_KIND_LIF ? v : 0.0f;
+                    if (d.rec_ie) {
+                        d.rec_ie[o] = kind == BSIM_KIND_LIF ? ie : 0.0f;
+                        d.rec_ii[o] = kind == BSIM_KIND_LIF ? ii : 0.0f;
+                        d.rec_in_e[o] = kind == BSIM_KIND_LIF ? acc.e[j] : 0.0f;
+                        d.rec_in_i[o] = kind == BSIM_KIND_LIF ? acc.i[j] : 0.0f;
+                    }
+                }
+            }
+        }
+        const uint64_t fm = ballot64(fired);
+        /* the block's list of active rows: each neuron's delays that
+         * deliver in phase (ii) of this cycle, in order */
+        uint64_t m = valid ? (h >> 1) & dmask : 0ull;
+        const uint32_t c = (uint32_t)__popcll(m), incl = wave_incl_scan(c);
+        if (n0 < d.n) {                                   /* uniform */
+            uint16_t *out = seg_out + (int64_t)(n0 / 64) * (WAVE * D) + (incl - c);
+            for (; m; m &= m - 1) *out++ = (uint16_t)(lane << 6 | (uint32_t)__builtin_ctzll(m));
+            if (lane == WAVE - 1) cnt_out[n0 / 64] = incl;
+            if (lane == 0 && rec) d.raster[(int64_t)(t - d.rec_t0) * d.nwords + n0 / 64] = fm;
+        }
+    }
+}
+
+/* The batch's rows, once every chunk has been summed; how many there are. */
+__device__ __forceinline__ uint32_t batch_rows(const Shared &S, int32_t nrb, uint32_t buf, Rows &R)
+{
+    const uint32_t lane = threadIdx.x & (WAVE - 1);
+    R.nrb = nrb;
+    R.at = 0;
+    R.end = wave_incl_scan((int32_t)lane < nrb ? S.ctot[buf * MAXR + lane] : 0u);
+    return readlane(R.end, WAVE - 1);
+}
+
+/* Event wavefronts: the unit of record k (below 0: none). */
+template <int NB, int WR>
+__device__ __forceinline__ void event_unit(const Shared &S, int32_t k, int32_t t, bool deliver, bool clocked,
+                                           uint32_t U, uint32_t K)
+{
+    const bsim_dev &d = args_again();
+    const bsim_unit *un = d.unit + (k < 0 ? 0 : k);
+    const int32_t id = k < 0 ? -1 : un->id, list = (t - 1) & 1;
+    const int32_t nrng = deliver && id >= 0 ? un->nrng : 0;
+    uint32_t par = 0, nb = 0;                   /* passes and batches so far, modulo 2 */
+    uint32_t events = 0, rows = 0;
+    for (int32_t rb = 0; rb < nrng; rb += MAXR) {
+        const int32_t nrb = min(MAXR, nrng - rb);
+        prepare_batch(S, d, un, rb, nrb, list, nb);
+        wg_barrier();
+        Rows R;
+        const uint32_t nrows = batch_rows(S, nrb, nb, R);
+        nb ^= 1u;
+        rows += nrows;
+        if (nrows > 0)                          /* uniform */
+            event_wave<NB, WR>(S, d, (uint32_t)un->part * U, un->nsyn, R, nrows,
+                               d.seg + (int64_t)list * d.nwords * (WAVE * d.dmax), U, K, par, d.syn + un->base,
+                               events);
+    }
+    /* the unit's work in this launch, when the next one ranks the units: its
+     * deliveries plus a fixed cost of two deliveries per active row, x 16 */
+    if (threadIdx.x == 0 && rows > 0) {
+        atomicAdd((unsigned long long *)&d.ev_count[id], (unsigned long long)events);
+        const int32_t re = d.rank_every;
+        if (clocked && re > 0 && (t + 1) % re == 0)
+            d.tile_load[(int64_t)(t & 1) * d.ntiles + id] = (uint64_t)events * 16ull + (uint64_t)rows * 32ull;
+    }
+}
+
+/* Owner wavefronts: the same unit's sums and update. */
+template <int S_>
+__device__ __forceinline__ void owner_unit(const Shared &S, int32_t k, int32_t t, bool deliver, bool update,
+                                           uint32_t U, uint32_t K)
+{
+    constexpr bool PRE = S_ <= PREFETCH_MAX_S;
+    const bsim_dev &d = args_again();
+    const bsim_unit *un = d.unit + (k < 0 ? 0 : k);
+    const int32_t id = k < 0 ? -1 : un->id;
+    const int32_t nrng = deliver && id >= 0 ? un->nrng : 0;
+    const bool upd = update && id >= 0;
+    Acc<S_> acc;
+#pragma unroll
+    for (int j = 0; j < S_; j++) {
+        acc.e[j] = 0.0f;
+        acc.i[j] = 0.0f;
+    }
+    NState<PRE ? S_ : 1> ns;
+    if constexpr (PRE) {
+        if (upd) {
+            load_nstate<S_>(d, id * (int32_t)U, d.hist + (int64_t)((t - 1) & 1) * d.n, ns);
+            load_params<S_>(d, ns);
+        }
+    }
+    uint32_t par = 0, nb = 0;                   /* passes and batches so far, modulo 2 */
+    for (int32_t rb = 0; rb < nrng; rb += MAXR) {
+        wg_barrier();
+        Rows R;
+        const uint32_t nrows = batch_rows(S, min(MAXR, nrng - rb), nb, R);
+        nb ^= 1u;
+        if (nrows > 0) owner_wave<S_>(S, U, K, par, acc);     /* uniform */
+    }
+    if (upd) update_unit<S_, PRE>(id, t, U, acc, ns);
+}
+
 template <int NB, int WR, int S_>
 __global__ __launch_bounds__(NTHREAD, STEP_EU) void bsim_step_kernel(bsim_dev d, int32_t t, int32_t flags)
 {
@@ -780,12 +994,10 @@ __global__ __launch_bounds__(NTHREAD, STEP_EU) void bsim_step_kernel(bsim_dev d,
         return;
     }
     const uint32_t U = (uint32_t)d.tile, K = slots_of(U);
-    /* the unit, -1: an empty slot; which order: the last ranking's */
-    const int32_t order = re > 0 && t > 0 ? ((t - 1) / re) & 1 : 0;
-    const int32_t k = d.perm[(int64_t)order * d.nslots + blockIdx.x - d.rank_wgs];
-    const uint32_t tid = threadIdx.x;
-    const uint32_t lane = tid & (WAVE - 1);
-    const uint32_t w = wave_index();
+    /* the workgroup's unit record: the slot's own, or in the order of the last ranking */
+    int32_t k = (int32_t)blockIdx.x - d.rank_wgs;
+    if (d.rank_wgs > 0) k = d.perm[(re > 0 && t > 0 ? (int64_t)(((t - 1) / re) & 1) * d.nslots : 0) + k];
+    const uint32_t tid = threadIdx.x, w = wave_index();
 
     Shared S;
     {
@@ -797,154 +1009,22 @@ __global__ __launch_bounds__(NTHREAD, STEP_EU) void bsim_step_kernel(bsim_dev d,
         S.blk_mark = S.blk_end + MAXR * BLKS;
         S.btot = S.blk_mark + NEV * WAVE;
         S.ctot = S.btot + 2 * NEV;
-        S.most = S.ctot + MAXR;
+        S.most = S.ctot + 2 * MAXR;
         S.last = S.most + 2;
     }
 
-    Acc<S_> acc;
-#pragma unroll
-    for (int j = 0; j < S_; j++) {
-        acc.e[j] = 0.0f;
-        acc.i[j] = 0.0f;
-    }
-
-    constexpr bool PRE = S_ <= PREFETCH_MAX_S;
-    NState<PRE ? S_ : 1> ns;
-    if constexpr (PRE) {
-        if ((flags & 2) && w >= NEV && k >= 0)
-            load_nstate<S_>(d, k * (int32_t)U, d.hist + (int64_t)((t - 1) & 1) * d.n, ns);
-    }
-
-    /* ---- phase (ii) of cycle t-1 ---------------------------------------- */
-    if ((flags & 1) && k >= 0) {
-        const bsim_unit un = d.unit[k];
+    const bool deliver = (flags & 1) != 0, update = (flags & 2) != 0;
+    if (deliver) {
         for (uint32_t i = tid; i < 2 * U; i += NTHREAD)
             reinterpret_cast<uint4 *>(S.hist)[i] = make_uint4(0u, 0u, 0u, 0u);
         for (uint32_t i = tid; i < 2 * PASS; i += NTHREAD) S.mark[i] = NO_MARK;
         if (w < NEV) S.blk_mark[tid] = NO_MARK;
         if (tid < 4) S.most[tid] = 0u;          /* most and last */
-        const bsim_syn *syn = d.syn + un.base;
-        uint32_t events = 0, rows = 0, par = 0;
-        for (int32_t rb = 0; rb < un.nrng; rb += MAXR)
-            deliver_batch<NB, WR, S_>(S, d, un, un.rng0 + rb, min(MAXR, un.nrng - rb), (t - 1) & 1, U, K, par,
-                                  syn, events,
-                                  rows, acc);
-        /* the unit's work in this launch, when the next one ranks the units:
-         * its deliveries plus a fixed cost of two deliveries per active row,
-         * x 16 */
-        if (tid == 0 && rows > 0) {
-            d.ev_count[k] += (int64_t)events;   /* one workgroup per unit and launch */
-            if (clocked && re > 0 && (t + 1) % re == 0)
-                d.tile_load[(int64_t)(t & 1) * d.ntiles + k] = (uint64_t)events * 16ull + (uint64_t)rows * 32ull;
-        }
     }
-
-    /* ---- phase (i) of cycle t: each owner thread updates its targets -------- */
-    if ((flags & 2) && w >= NEV && k >= 0) {
-        const int32_t D = d.dmax;
-        const uint64_t dmask = (D >= 63) ? (~0ull >> 1) : ((1ull << D) - 1ull);
-        const int32_t base = k * (int32_t)U;
-        const uint64_t *hist_in = d.hist + (int64_t)((t - 1) & 1) * d.n;
-        uint64_t *hist_out = d.hist + (int64_t)(t & 1) * d.n;
-        uint32_t *cnt_out = d.seg_count + (int64_t)(t & 1) * d.nwords;
-        uint16_t *seg_out = d.seg + (int64_t)(t & 1) * d.nwords * (WAVE * D);
-        const bool rec = d.raster != nullptr && t >= d.rec_t0 && t < d.rec_t0 + d.rec_steps;
-#pragma unroll
-        for (int j = 0; j < S_; j++) {
-            const uint32_t i0 = (w - NEV) * WAVE + j * (NOWN * WAVE);
-            if (i0 >= U) continue;                            /* uniform */
-            const int32_t n0 = base + (int32_t)i0;
-            const int32_t nid = n0 + (int32_t)lane;
-            const bool valid = nid < d.n;
-            bool fired = false;
-            uint64_t h = 0;
-            if (valid) {
-                uint32_t cls;
-                int32_t rs;
-                float v, ie, ii, vtmp;
-                uint64_t hin;
-                if constexpr (PRE) {
-                    cls = ns.cls[j]; rs = ns.refrac[j]; v = ns.v[j]; ie = ns.ie[j]; ii = ns.ii[j];
-                    vtmp = ns.vtmp[j]; hin = ns.hist[j];
-                } else {
-                    cls = d.ncls[nid]; rs = d.refrac[nid]; v = d.v[nid]; ie = d.ie[nid]; ii = d.ii[nid];
-                    vtmp = d.v_tmp[nid]; hin = hist_in[nid];
-                }
-                const uint32_t kind = cls >> 30;
-                if (kind == BSIM_KIND_LIF) {
-                    const float inE = acc.e[j];
-                    const float inI = acc.i[j];
-                    if (rs > 0) {
-                        d.refrac[nid] = rs - 1;
-                    } else {
-                        const bsim_lifc c = d.lifc[cls & BSIM_CLS_SET_MASK];
-                        v = c.Cm * v + vtmp + ie * c.C_E + ii * c.C_I;
-                        ie = c.CE * ie;
-                        ii = c.CI * ii;
-                        if (v >= c.v_thresh) {
-                            fired = true;
-                            d.refrac[nid] = c.refrac_time - 1;
-                            v = c.v_reset;
-                        } else {
-                            if (d.in_sum) d.in_sum[nid] = d.in_sum[nid] + (inE + inI);
-                            ie += inE;
-                            ii += inI;
-                        }
-                        d.v[nid] = v;
-                        d.ie[nid] = ie;
-                        d.ii[nid] = ii;
-                    }
-                } else if (kind == BSIM_KIND_ARRAY) {
-                    const int32_t c = d.arr_cur[nid];
-                    if (c < d.arr_end[nid] && d.arr_t[c] <= t) {
-                        fired = true;
-                        d.arr_cur[nid] = c + 1;
-                    }
-                } else if (kind == BSIM_KIND_POISSON) {
-                    /* PoissonNeuron::update (src/neuron/poisson/PoissonNeuron.cpp:52-63):
-                     * fire at the drawn cycle before the end cycle, then draw
-                     * the next one 1 + X cycles later */
-                    const int32_t nx = d.arr_cur[nid];
-                    if (t == nx && nx < d.arr_end[nid]) {
-                        fired = true;
-                        const uint32_t x = poisson_pick(d.pois_tab + d.bern_p[nid],
-                                                        bern_hash(d.bern_seed[nid], d.bern_key[nid], (uint32_t)t));
-                        d.arr_cur[nid] = (int32_t)min((int64_t)nx + 1 + x, (int64_t)0x7FFFFFFF);
-                    }
-                } else {
-                    fired = bern_hash(d.bern_seed[nid], d.bern_key[nid], (uint32_t)t) < d.bern_p[nid];
-                }
-                h = (hin << 1) | (fired ? 1ull : 0ull);
-                hist_out[nid] = h;
-                if (d.slot_count) d.slot_count[nid] += __popcll((h >> 1) & dmask);
-                if (fired) d.fire_count[nid] += 1;
-                if (rec && d.rec_index) {
-                    const int32_t ri = d.rec_index[nid];
-                    if (ri >= 0) {
-                        const int64_t o = (int64_t)(t - d.rec_t0) * d.n_rec + ri;
-                        d.rec_v[o] = kind == BSIM_KIND_LIF ? v : 0.0f;
-                        if (d.rec_ie) {
-                            d.rec_ie[o] = kind == BSIM_KIND_LIF ? ie : 0.0f;
-                            d.rec_ii[o] = kind == BSIM_KIND_LIF ? ii : 0.0f;
-                            d.rec_in_e[o] = kind == BSIM_KIND_LIF ? acc.e[j] : 0.0f;
-                            d.rec_in_i[o] = kind == BSIM_KIND_LIF ? acc.i[j] : 0.0f;
-                        }
-                    }
-                }
-            }
-            const uint64_t fm = ballot64(fired);
-            /* the block's list of active rows: each neuron's delays that
-             * deliver in phase (ii) of this cycle, in order */
-            uint64_t m = valid ? (h >> 1) & dmask : 0ull;
-            const uint32_t c = (uint32_t)__popcll(m), incl = wave_incl_scan(c);
-            if (n0 < d.n) {                                   /* uniform */
-                uint16_t *out = seg_out + (int64_t)(n0 / 64) * (WAVE * D) + (incl - c);
-                for (; m; m &= m - 1) *out++ = (uint16_t)(lane << 6 | (uint32_t)__builtin_ctzll(m));
-                if (lane == WAVE - 1) cnt_out[n0 / 64] = incl;
-                if (lane == 0 && rec) d.raster[(int64_t)(t - d.rec_t0) * d.nwords + n0 / 64] = fm;
-            }
-        }
-    }
+    if (w < NEV)
+        event_unit<NB, WR>(S, k, t, deliver, clocked, U, K);
+    else
+        owner_unit<S_>(S, k, t, deliver, update, U, K);
     if (clocked) wg_barrier();      /* every wavefront has read the cycle */
     if (clocked && tid == 0) count_done(d);
 }
@@ -959,12 +1039,12 @@ extern "C" hipError_t bsim_launch_step(const bsim_dev *d, int32_t t, int32_t fla
     const size_t lds = lds_bytes(U);
     (void)hipGetLastError();       /* the check below then reports this launch alone */
 #define OWN(X) (((X) + NOWN * WAVE - 1) / (NOWN * WAVE))
-#define STEP(NB, X)                                                                                             \
-    do {                                                                                                        \
-        if (d->wrows == 2)                                                                                      \
-            hipLaunchKernelGGL((bsim_step_kernel<NB, 2, OWN(X)>), grid, block, lds, stream, *d, t, flags);      \
-        else                                                                                                    \
-            hipLaunchKernelGGL((bsim_step_kernel<NB, 1, OWN(X)>), grid, block, lds, stream, *d, t, flags);      \
+#define STEP(NB, X)                                                                                       \
+    do {                                                                                                  \
+        if (d->wrows == 2)                                                                                \
+            hipLaunchKernelGGL((bsim_step_kernel<NB, 2, OWN(X)>), grid, block, lds, stream, *d, t, flags); \
+        else                                                                                              \
+            hipLaunchKernelGGL((bsim_step_kernel<NB, 1, OWN(X)>), grid, block, lds, stream, *d, t, flags); \
     } while (0)
     if (U <= 64) STEP(6, 64);
     else if (U <= 128) STEP(7, 128);
