@@ -714,10 +714,20 @@ __device__ __forceinline__ void count_done(const bsim_dev &d)
 /* Orders the units by their work in the launch before, heaviest first, so that
  * the hardware dispatches the heavy units of the coming launches before the
  * light ones (results do not depend on the order; the firing volleys move
- * slowly against two cycles).  Counting sort over half-octave classes; within
- * a class the order is arbitrary.  Runs in one workgroup, beside the others of
- * the launch, and clears the loads that it has read.  The classes of the units
- * are kept in LDS where they fit. */
+ * slowly against two cycles).  Units of one group share lines of the row
+ * table and stay on one XCD while these have about the same work.  Where one
+ * has more than SPREAD_MIN times the mean, the units are dealt out to the XCDs
+ * in turn, unless the table has an entry per synapse or more (rows taken two
+ * at a time): lines that every XCD reads then cost more than the imbalance.
+ * us per cycle by group / dealt out: 330,000 neurons at ~100 Hz 59.9 / 54.4,
+ * 650,000 108.2 / 101.2, where volleys pass through the populations at
+ * different times; a balanced sweep of 96 chains 27.6 / 27.9, 110,000 neurons
+ * with delays up to 50 steps 941 / 1,002 to 1,046.
+ * Counting sort over half-octave classes; within a class the order is
+ * arbitrary.  Runs in one workgroup, beside the others of the launch, and
+ * clears the loads that it has read.  The classes of the units are kept in LDS
+ * where they fit. */
+#define SPREAD_MIN 1.125f
 #define RANK_CLASSES 64
 
 __device__ __forceinline__ uint32_t load_class(uint64_t x)
@@ -728,13 +738,22 @@ __device__ __forceinline__ uint32_t load_class(uint64_t x)
     return min(2u * (e - 4u) + h + 1u, (uint32_t)RANK_CLASSES - 1u);
 }
 
+/* a class's work, as a multiple of the lightest's */
+__device__ __forceinline__ float class_work(uint32_t c)
+{
+    return c == 0 ? 0.5f : ldexpf((c - 1u) & 1u ? 1.5f : 1.0f, (int)((c - 1u) / 2u));
+}
+
 __device__ void rank_units(const bsim_dev &d, uint64_t *load, int32_t *perm, uint32_t *lds, uint32_t lds_size)
 {
     uint32_t *cnt = lds, *fill = cnt + NRES * RANK_CLASSES, *rtot = fill + NRES * RANK_CLASSES;
-    uint8_t *cls = (uint32_t)d.ntiles <= lds_size - 4u * (2 * NRES * RANK_CLASSES + NRES)
-                       ? reinterpret_cast<uint8_t *>(rtot + NRES) : d.tile_cls;
-    const uint32_t tid = threadIdx.x;
-    for (uint32_t i = tid; i < NRES * RANK_CLASSES; i += NTHREAD) cnt[i] = 0u;
+    float *work = reinterpret_cast<float *>(rtot + NRES);
+    uint8_t *cls = (uint32_t)d.ntiles <= lds_size - 4u * (2 * NRES * RANK_CLASSES + 2 * NRES)
+                       ? reinterpret_cast<uint8_t *>(work + NRES) : d.tile_cls;
+    static_assert(RANK_CLASSES == WAVE && NRES * RANK_CLASSES <= NTHREAD, "a wavefront per residue, a lane per class");
+    const uint32_t tid = threadIdx.x, x = tid / RANK_CLASSES, c = RANK_CLASSES - 1u - tid % RANK_CLASSES;
+    const bool counts = tid < NRES * RANK_CLASSES;
+    if (counts) cnt[tid] = 0u;
     __syncthreads();
     for (int32_t k = tid; k < d.ntiles; k += NTHREAD) {
         const uint32_t c = load_class(load[k]);
@@ -743,10 +762,27 @@ __device__ void rank_units(const bsim_dev &d, uint64_t *load, int32_t *perm, uin
         atomicAdd(&cnt[d.tile_res[k] * RANK_CLASSES + c], 1u);
     }
     __syncthreads();
+    if (counts) {
+        float s = (float)cnt[x * RANK_CLASSES + c] * class_work(c);
+        for (int m = 1; m < WAVE; m *= 2) s += __shfl_xor(s, m);
+        if (c == 0) work[x] = s;
+    }
+    __syncthreads();
+    float all = 0.0f, most = 0.0f;
+    for (int i = 0; i < NRES; i++) {
+        all += work[i];
+        most = fmaxf(most, work[i]);
+    }
+    const bool spread = d.wrows == 1 && most * NRES > all * SPREAD_MIN;
+    if (spread) {                                   /* count again, by the residues dealt out */
+        if (counts) cnt[tid] = 0u;
+        __syncthreads();
+        for (int32_t k = tid; k < d.ntiles; k += NTHREAD)
+            atomicAdd(&cnt[(uint32_t)k % NRES * RANK_CLASSES + cls[k]], 1u);
+        __syncthreads();
+    }
     /* exclusive prefix of each residue's class counts, heaviest class first */
-    static_assert(RANK_CLASSES == WAVE && NRES * RANK_CLASSES <= NTHREAD, "a wavefront per residue");
-    if (tid < NRES * RANK_CLASSES) {
-        const uint32_t x = tid / RANK_CLASSES, c = RANK_CLASSES - 1u - tid % RANK_CLASSES;
+    if (counts) {
         const uint32_t v = cnt[x * RANK_CLASSES + c], incl = wave_incl_scan(v);
         fill[x * RANK_CLASSES + c] = incl - v;
         if (c == 0) rtot[x] = incl;
@@ -754,14 +790,13 @@ __device__ void rank_units(const bsim_dev &d, uint64_t *load, int32_t *perm, uin
     __syncthreads();
     /* unit of residue x at rank i goes to slot NRES * i + x */
     for (int32_t k = tid; k < d.ntiles; k += NTHREAD) {
-        const uint32_t x = d.tile_res[k];
+        const uint32_t x = spread ? (uint32_t)k % NRES : d.tile_res[k];
         const uint32_t pos = atomicAdd(&fill[x * RANK_CLASSES + cls[k]], 1u);
         perm[NRES * pos + x] = k;
     }
     /* the remaining slots of each residue are empty */
-    const int32_t per = d.nslots / NRES;
     for (int32_t i = tid; i < d.nslots; i += NTHREAD) {
-        if (i / NRES >= (int32_t)rtot[i % NRES] && i / NRES < per) perm[i] = -1;
+        if (i / NRES >= (int32_t)rtot[i % NRES]) perm[i] = -1;
     }
 }
 

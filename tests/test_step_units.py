@@ -1,8 +1,8 @@
 """The step kernel at the sizes where its passes, slots and units change:
 whole tiles and tiles in parts, a target with more events in a pass than it has
 slots, a sub-row longer than a pass, more source ranges than one batch holds,
-blocks of rows without a synapse into the unit.  Bit for bit against the
-oracle, as everything the step computes is.
+blocks of rows without a synapse into the unit, units that change XCD.  Bit for
+bit against the oracle, as everything the step computes is.
 """
 import numpy as np
 import pytest
@@ -94,3 +94,24 @@ def test_whole_tiles(npop, tile):
     o = oracle.run(spec, DT, steps, rec_ids=rec, mode="csr", tile=256, threads=8)
     assert o.events > 10_000
     assert_same(r, o, "whole tiles")
+
+
+@pytest.mark.parametrize("active", [1, 11])
+def test_ranked_units(active):
+    """More units than run at a time, ranked every other cycle: populations of
+    which one is active (its units are dealt out to all XCDs) or every one."""
+    npop, n, s, steps = 11, 9408, 300, 40
+    rng = np.random.Generator(np.random.PCG64(active))
+    b = netspec.Builder()
+    for p in range(npop):
+        base = p * (s + n)
+        sources(b, s, steps, rng, 0.3 if p < active else 0.01)
+        lif(b, n, rng)
+        connect(b, base + np.repeat(np.arange(s), 400), base + s + rng.integers(0, n, 400 * s), rng, 2, 0.05)
+    spec = b.build()
+    rec = [s, s + n - 1, spec.n - 1]
+    say(f"[gpu] ranked units active={active} n={spec.n} s={spec.s}")
+    r = run_gpu(spec, steps, rec, 192)
+    o = oracle.run(spec, DT, steps, rec_ids=rec, mode="csr", tile=256, threads=8)
+    assert o.events > 10_000
+    assert_same(r, o, "ranked units")
