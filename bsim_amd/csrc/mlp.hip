@@ -14,22 +14,22 @@
  *   loss       dZ = bf16(2 (out - Y) / (B * out_dim)); loss and bias-gradient
  *              partials
  *   backward   dZ_{l-1} = bf16(dZ_l W_l) where H_{l-1} > 0, with its
- *              bias-gradient partials; dW_l = dZ_l^T H_{l-1} (split over the
- *              batch, fp32 partials)
- *   adam       sums every gradient's partials in a fixed order, then Adam
- *              (Kingma & Ba, 2015) on the fp32 master, writes the bf16 copy
- *              and its transpose
- * The input, hidden activations and activation gradients of a training step
- * are also written transposed ([unit][row]), so that the weight-gradient
- * GEMM reads both of its operands with the batch (its reduction index)
- * contiguous; likewise the transposed bf16 copy of every weight matrix lets
- * the activation-gradient products read W^T with their reduction index
- * contiguous.
- * Launches per step: one GEMM per layer forward (the first gathers its
- * minibatch rows from the resident set, the last forms the loss and dZ of the
- * output in its epilogue), one GEMM per activation gradient, every weight
- * gradient in one launch (mlp_gemm_partials) and Adam with the transposes in
- * one (mlp_adam_tiles).
+ *              bias-gradient partials
+ *   update     dW_l = dZ_l^T H_{l-1} in four sums over quarters of the batch,
+ *              added in order; Adam (Kingma & Ba, 2015) on the fp32 master;
+ *              the bf16 copies of W_l and its transpose
+ * Launches per step: with layers of up to 512 units two, everything up to the
+ * backward products (mlp_chain) and the update (mlp_update); with wider ones a
+ * GEMM per layer forward and per activation gradient (mlp_gemm) before the
+ * update.
+ *
+ * Operands that are read along a reduction index from memory lie in fragments
+ * (frag_index): the bf16 copies of the weights and, for the weight gradients,
+ * the transposed copies of the inputs, activations and activation gradients.  A
+ * wavefront loads or stores a fragment as one contiguous KB, straight to and
+ * from the registers that the MFMA reads and writes.  In rows, the same loads
+ * fetched 64 bytes from each of 16 rows: mlp_chain's launch of 4,096 rows
+ * through 4 x 512 units took 73 us that way and 28 in fragments (predict).
  * Every reduction has a fixed order, so results repeat bit for bit.
  *
  * There is no counterpart in the reference; the algorithm is the textbook
@@ -59,8 +59,8 @@ constexpr int BM = 64, BN = 64, BK = 64;   /* workgroup tile and k step */
 constexpr int LDS_STRIDE = BK + 8;         /* bf16 per LDS tile row (144 B) */
 constexpr int GEMM_THREADS = 256;          /* 2 x 2 wavefronts of 32 x 32 */
 constexpr int KSPLIT = 4;                  /* batch split of the weight gradients */
-constexpr int TRAIN_BATCH_ALIGN = KSPLIT * BK;   /* training batches: whole k steps per split */
-constexpr int ROWS_PER_PART = 64;          /* bias-gradient partial: rows per partial */
+constexpr int TRAIN_BATCH_ALIGN = KSPLIT * BK;   /* training batches: whole pairs of 32 rows per split */
+constexpr int ROWS_PER_PART = 32;          /* bias-gradient partial: rows per partial */
 constexpr int MAX_LAYERS = 10;             /* linear layers (hidden + 1) */
 
 __host__ __device__ inline uint16_t f2bf(float x)
@@ -71,6 +71,13 @@ __host__ __device__ inline uint16_t f2bf(float x)
     return (uint16_t)(u >> 16);
 }
 
+/* Two at once on the device, v_cvt_pk_bf16_f32: lo in the low half. */
+__device__ inline uint32_t pack_bf(float lo, float hi)
+{
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, bf16x2{(__bf16)lo, (__bf16)hi});
+}
+
 __host__ __device__ inline float bf2f(uint16_t h)
 {
     const uint32_t u = (uint32_t)h << 16;
@@ -79,31 +86,37 @@ __host__ __device__ inline float bf2f(uint16_t h)
     return x;
 }
 
-enum Epi { EPI_RELU_BF16 = 0, EPI_LINEAR_F32 = 1, EPI_DRELU_BF16 = 2, EPI_PARTIAL_F32 = 3, EPI_LOSS = 4 };
+/* Where element (n, k) of a matrix [N][K] with reduction index k lies in
+ * fragments: the 16 x 32 operand of one MFMA, as the wavefront's lanes hold it,
+ * is 1 KB; those of 32 k for all n follow one another. */
+__host__ __device__ inline int64_t frag_index(int32_t n, int32_t k, int32_t N)
+{
+    return ((int64_t)(k / 32) * (N / 16) + n / 16) * 512 + (k % 32 / 8 * 16 + n % 16) * 8 + k % 8;
+}
 
-/* C[m][n] = sum_k A[m * lda + k] B[n * ldb + k] over this workgroup's k
- * range (both operands k-contiguous). */
+enum Epi { EPI_RELU_BF16 = 0, EPI_LINEAR_F32 = 1, EPI_DRELU_BF16 = 2, EPI_LOSS = 3 };
+
+/* C[m][n] = sum_k A[m * lda + k] B(n, k), B in fragments. */
 struct GemmArgs {
     const uint16_t *A;
     const uint16_t *B;
-    int64_t lda, ldb;
-    int32_t M, N, K;        /* K: length of one split (blockIdx.z) */
+    int64_t lda;
+    int32_t M, N, K;
     int32_t pad;
     const float *bias;      /* EPI_RELU_BF16, EPI_LINEAR_F32: [N] */
     uint16_t *out_bf;       /* EPI_RELU_BF16, EPI_DRELU_BF16: [M][ldo] */
-    float *out_f;           /* EPI_LINEAR_F32: [M][ldo]; EPI_PARTIAL_F32: [split][M][ldo] */
+    float *out_f;           /* EPI_LINEAR_F32: [M][ldo] */
     int64_t ldo;
     const uint16_t *mask;   /* EPI_DRELU_BF16: keep where mask[m * ldo + n] > 0 */
-    float *bpart;           /* EPI_DRELU_BF16: bias-gradient partials [M / 64][N] */
-    uint16_t *out_t;        /* EPI_RELU_BF16, EPI_DRELU_BF16, EPI_LOSS: transposed copy [N][ldt] or null */
-    int64_t ldt;
+    float *bpart;           /* EPI_DRELU_BF16, EPI_LOSS: bias-gradient partials [M / 32][N] */
+    uint16_t *out_t;        /* EPI_RELU_BF16, EPI_DRELU_BF16, EPI_LOSS: transposed copy [N][M] in fragments, or null */
     const int32_t *arow;    /* row m of A is row arow[m] of the array A (null: row m) */
-    uint16_t *a_t;          /* with K == BK: workgroups of column tile 0 write A^T [K][ldt] */
+    uint16_t *a_t;          /* with K == BK: workgroups of column tile 0 write A^T [K][M] in fragments */
     const float *y;         /* EPI_LOSS: targets, row m at y[(yrow ? yrow[m] : m) * ny] */
     const int32_t *yrow;
     int32_t ny;             /* EPI_LOSS: valid output columns */
     float scale;            /* EPI_LOSS: dZ = bf16(scale * (C + bias - y)) */
-    float *lpart;           /* EPI_LOSS: squared-error sum of each 64 x 64 tile [M / 64][N / 64] */
+    float *lpart;           /* EPI_LOSS: squared-error sums, of the quadrants of each 64 x 64 tile [M / 64][N / 64][4] */
 };
 
 /* One k step of a 64-row operand: thread tid holds rows tid / 8 and
@@ -131,20 +144,36 @@ __device__ inline void store_tile(uint16_t *T, const Tile &t, uint32_t tid)
     *(uint4 *)(T + (r + 32) * LDS_STRIDE + kc) = t.v[1];
 }
 
-/* Output tile (bx, by) of split bz: C[by * 64 .. + 63][bx * 64 .. + 63]. */
+/* The same of an operand in fragments: of each 32 k, the tile's four are
+ * contiguous, and a wavefront takes one. */
+__device__ inline Tile load_frag_tile(const uint16_t *P, int32_t N, int32_t r0, int32_t k0, uint32_t tid)
+{
+    const uint16_t *p = P + ((int64_t)(k0 / 32) * (N / 16) + r0 / 16) * 512;
+    Tile t;
+    t.v[0] = *(const uint4 *)(p + tid * 8u);
+    t.v[1] = *(const uint4 *)(p + (uint32_t)N * 32u + tid * 8u);
+    return t;
+}
+
+__device__ inline void store_frag_tile(uint16_t *T, const Tile &t, uint32_t tid)
+{
+    const uint32_t r = tid / 64 * 16 + tid % 16, k = tid % 64 / 16 * 8;
+    *(uint4 *)(T + r * LDS_STRIDE + k) = t.v[0];
+    *(uint4 *)(T + r * LDS_STRIDE + k + 32) = t.v[1];
+}
+
+/* Output tile (bx, by): C[by * 64 .. + 63][bx * 64 .. + 63]. */
 template <int EPI>
-__device__ inline void gemm_tile(const GemmArgs &g, int32_t bx, int32_t by, int32_t bz)
+__device__ inline void gemm_tile(const GemmArgs &g, int32_t bx, int32_t by)
 {
     __shared__ __attribute__((aligned(16))) uint16_t As[2][BM * LDS_STRIDE];
     __shared__ __attribute__((aligned(16))) uint16_t Bs[2][BN * LDS_STRIDE];
     __shared__ float bsum[2][BN];
-    __shared__ float lwave[GEMM_THREADS / WAVE];
 
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & (WAVE - 1), w = tid / WAVE;
     const uint32_t wm = w >> 1, wn = w & 1u;     /* wavefront's 32 x 32 quadrant */
     const int32_t n0 = bx * BN, m0 = by * BM;
-    const int32_t kbeg = bz * g.K;
     const int32_t nk = g.K / BK;
 
     f32x4 acc[2][2];
@@ -159,14 +188,14 @@ __device__ inline void gemm_tile(const GemmArgs &g, int32_t bx, int32_t by, int3
      * whole step */
     Tile ra, rb;
     {
-        const Tile a0 = load_tile(g.A, g.lda, m0, kbeg, tid, g.arow);
-        const Tile b0 = load_tile(g.B, g.ldb, n0, kbeg, tid);
+        const Tile a0 = load_tile(g.A, g.lda, m0, 0, tid, g.arow);
+        const Tile b0 = load_frag_tile(g.B, g.N, n0, 0, tid);
         if (nk > 1) {
-            ra = load_tile(g.A, g.lda, m0, kbeg + BK, tid, g.arow);
-            rb = load_tile(g.B, g.ldb, n0, kbeg + BK, tid);
+            ra = load_tile(g.A, g.lda, m0, BK, tid, g.arow);
+            rb = load_frag_tile(g.B, g.N, n0, BK, tid);
         }
         store_tile(As[0], a0, tid);
-        store_tile(Bs[0], b0, tid);
+        store_frag_tile(Bs[0], b0, tid);
     }
     /* the epilogue's other operands for this lane's 16 outputs (rows m0 +
      * 32 wm + 16 i + 4 (lane / 16) + r, column n0 + 32 wn + 16 j + lane %
@@ -206,7 +235,7 @@ __device__ inline void gemm_tile(const GemmArgs &g, int32_t bx, int32_t by, int3
     if (g.a_t && bx == 0 && nk == 1) {
         for (uint32_t x = tid; x < (uint32_t)(BM * BK); x += GEMM_THREADS) {
             const uint32_t k = x / BM, r = x % BM;
-            g.a_t[(int64_t)(kbeg + (int32_t)k) * g.ldt + m0 + (int32_t)r] = As[0][r * LDS_STRIDE + k];
+            g.a_t[frag_index((int32_t)k, m0 + (int32_t)r, g.K)] = As[0][r * LDS_STRIDE + k];
         }
     }
 
@@ -215,10 +244,10 @@ __device__ inline void gemm_tile(const GemmArgs &g, int32_t bx, int32_t by, int3
         const int cur = s & 1;
         if (s + 1 < nk) {
             store_tile(As[cur ^ 1], ra, tid);
-            store_tile(Bs[cur ^ 1], rb, tid);
+            store_frag_tile(Bs[cur ^ 1], rb, tid);
             if (s + 2 < nk) {
-                ra = load_tile(g.A, g.lda, m0, kbeg + (s + 2) * BK, tid, g.arow);
-                rb = load_tile(g.B, g.ldb, n0, kbeg + (s + 2) * BK, tid);
+                ra = load_tile(g.A, g.lda, m0, (s + 2) * BK, tid, g.arow);
+                rb = load_frag_tile(g.B, g.N, n0, (s + 2) * BK, tid);
             }
         }
 #pragma unroll
@@ -287,20 +316,18 @@ __device__ inline void gemm_tile(const GemmArgs &g, int32_t bx, int32_t by, int3
                     }
                     g.out_bf[(int64_t)row * g.ldo + col] = h[r];
                     csum[j] += bf2f(h[r]);
-                } else {
-                    g.out_f[((int64_t)bz * g.M + row) * g.ldo + col] = v;
                 }
             }
             if ((EPI == EPI_RELU_BF16 || EPI == EPI_DRELU_BF16 || EPI == EPI_LOSS) && g.out_t) {
                 /* 4 consecutive rows of one column: one 8-byte store */
                 const uint2 q = {(uint32_t)h[0] | ((uint32_t)h[1] << 16),
                                  (uint32_t)h[2] | ((uint32_t)h[3] << 16)};
-                *(uint2 *)(g.out_t + (int64_t)col * g.ldt + row0) = q;
+                *(uint2 *)(g.out_t + frag_index(col, row0, g.N)) = q;
             }
         }
     }
     if (EPI == EPI_DRELU_BF16 || EPI == EPI_LOSS) {
-        /* column sums over the workgroup's 64 rows, in a fixed order */
+        /* column sums over 32 rows each, in a fixed order */
 #pragma unroll
         for (int j = 0; j < 2; j++) {
             float x = csum[j];
@@ -309,235 +336,560 @@ __device__ inline void gemm_tile(const GemmArgs &g, int32_t bx, int32_t by, int3
             if (lane < 16) bsum[wm][wn * 32 + j * 16 + lane] = x;
         }
         if (EPI == EPI_LOSS) {
-            /* the tile's squared error: lane, wavefront, then the four
-             * wavefronts, in a fixed order */
+            /* the quadrant's squared error, in a fixed order */
 #pragma unroll
             for (int o = 1; o < WAVE; o <<= 1) lsum += __shfl_xor(lsum, o);
-            if (lane == 0) lwave[w] = lsum;
+            if (lane == 0) g.lpart[((int64_t)by * (g.N / BN) + bx) * 4 + w] = lsum;
         }
         __syncthreads();
-        if (tid < BN) g.bpart[(int64_t)by * g.N + n0 + tid] = bsum[0][tid] + bsum[1][tid];
-        if (EPI == EPI_LOSS && tid == 0)
-            g.lpart[(int64_t)by * (g.N / BN) + bx] = ((lwave[0] + lwave[1]) + lwave[2]) + lwave[3];
+        if (tid < 2 * BN) g.bpart[(2 * (int64_t)by + tid / BN) * g.N + n0 + tid % BN] = bsum[tid / BN][tid % BN];
     }
 }
 
 template <int EPI>
 __global__ __launch_bounds__(GEMM_THREADS) void mlp_gemm(GemmArgs g)
 {
-    gemm_tile<EPI>(g, blockIdx.x, blockIdx.y, blockIdx.z);
+    /* an XCD takes consecutive tiles, row by row: it reads an eighth of A, and
+     * the rows that it wrote itself in the layer before */
+    const int32_t nx = g.N / BN, nt = (int32_t)gridDim.x, x = (int32_t)blockIdx.x % 8;
+    const int32_t t = x * (nt / 8) + min(x, nt % 8) + (int32_t)blockIdx.x / 8;
+    gemm_tile<EPI>(g, t % nx, t / nx);
 }
 
-/* The weight-gradient GEMMs of every layer in one launch: workgroups
- * first[l] .. first[l + 1] - 1 take layer l's tiles, split by split. */
-struct GemmGroup {
-    GemmArgs g[MAX_LAYERS];
-    int32_t first[MAX_LAYERS + 1];
-    int32_t n;
+/* ---- every layer in one launch ---------------------------------------------
+ *
+ * A row of the batch depends on no other row until the weight gradients, so a
+ * workgroup can take CH_ROWS rows through all layers, forward and back, with
+ * the activations in LDS.  A stage is one product with a weight matrix: the
+ * forward layers in order, then (training) the activation gradients from the
+ * last layer to the second.
+ *
+ * What bounds it: every workgroup reads every weight, 512 KB per stage of 512 x
+ * 512 from its XCD's L2 at the 64 bytes per cycle that a compute unit takes in,
+ * 3.4 us, against 1.7 of MFMA; measured 4.7 us per such stage (the rest is the
+ * epilogue, between two barriers), and 8 to launch, load the input and start
+ * the stream.  A launch per layer took 9 to 10 us for the same stage, of which
+ * the kernel's start, a pass of loads that nothing hides and the end of the
+ * grid were most.  The weights are loaded 128 rows of the reduction index ahead,
+ * through the ends of the stages, as they depend on nothing; 16 rows per
+ * workgroup would read the weights twice as often in the same time, 64 would
+ * leave more compute units idle.  Sixteen wavefronts of 32 columns each against
+ * eight of 64: 51 / 54 us.  Training step of 4,096 rows through 4 x 512 units,
+ * 200 outputs: 83 us in nine launches, 51 chained; 256 rows through 2 x 192: 33
+ * / 12; predict 4,096 rows: 47 / 25.
+ *
+ * Layers wider than CH_MAX run in a launch each: 1,024 units would take 14 us
+ * per stage here whatever the rows, as many as 2,048 rows take in a launch of
+ * their own, and two of them exceed a wavefront's registers.
+ */
+constexpr int CH_ROWS = 32;                /* rows of a workgroup: two MFMA tiles, one bias-gradient partial */
+constexpr int CH_MAX = 512;                /* widest layer */
+static_assert(CH_ROWS == ROWS_PER_PART, "a workgroup writes its rows' bias-gradient partial");
+
+struct ChainArgs {
+    int32_t nlin, ld;                      /* ld: LDS row stride, widest layer + 8 */
+    int32_t kdim[MAX_LAYERS + 1];
+    int32_t din;
+    int64_t woff[MAX_LAYERS], boff[MAX_LAYERS];
+    const uint16_t *w, *wt;                /* W_l and W_l^T at woff[l], in fragments (frag_index) */
+    const float *p;                        /* biases at boff[l] */
+    const uint16_t *xb;                    /* input rows, bf16 [.][kdim[0]], or null: */
+    const float *xf;                       /* f32 [n][din] */
+    const int32_t *rows;                   /* row m of the batch is row rows[m] of xb and y (null: row m) */
+    int64_t n;                             /* rows of xf; the batch's others are 0 */
+    float *out;                            /* predict: [batch][kdim[nlin]] */
+    uint16_t *act_t[MAX_LAYERS], *dzt[MAX_LAYERS];   /* training: transposed, [unit][batch] in fragments */
+    float *bpart[MAX_LAYERS], *lpart;
+    const float *y;
+    int32_t ny;
+    float scale;
 };
 
-__global__ __launch_bounds__(GEMM_THREADS) void mlp_gemm_partials(GemmGroup a)
+/* The product of a stage: W [N][K]. */
+struct ChainStage {
+    const uint16_t *w;
+    int32_t K, N;
+};
+
+__device__ inline ChainStage chain_stage(const ChainArgs &a, int32_t s)
 {
-    int l = 0;
-    while (l + 1 < a.n && (int32_t)blockIdx.x >= a.first[l + 1]) l++;
-    const GemmArgs &g = a.g[l];
-    const int32_t t = (int32_t)blockIdx.x - a.first[l];
-    const int32_t tn = g.N / BN, tmn = tn * (g.M / BM);
-    const int32_t r = t % tmn;
-    gemm_tile<EPI_PARTIAL_F32>(g, r % tn, r / tn, t / tmn);
+    if (s < a.nlin) return ChainStage{a.w + a.woff[s], a.kdim[s], a.kdim[s + 1]};
+    const int32_t l = 2 * a.nlin - 1 - s;
+    return ChainStage{a.wt + a.woff[l], a.kdim[l + 1], a.kdim[l]};
 }
 
-struct AdamSeg {
-    int64_t off, count;   /* into the flat parameter arrays */
-    const float *parts;   /* gradient partials, [nparts][count] */
-    int32_t nparts;
-    int32_t pad;
-};
+/* 0xFFFF in each half of x that is not 0; no half has its top bit set. */
+__device__ inline uint32_t nonzero_halves(uint32_t x)
+{
+    const uint32_t t = (x + 0x7FFF7FFFu) & 0x80008000u;
+    return (t - (t >> 15)) | t;
+}
 
-struct AdamArgs {
-    AdamSeg seg[2 * MAX_LAYERS];
-    int32_t nseg;
-    int32_t update;       /* 0: only write the summed gradient */
-    float lr, b1, b2, eps, c1, c2;   /* c1 = 1 - b1^t, c2 = 1 - b2^t */
+/* W wavefronts; wavefront w has the columns 32 w .. 32 w + 31 of every stage. */
+template <int W, bool TRAIN>
+__global__ __launch_bounds__(W * WAVE) void mlp_chain(ChainArgs a)
+{
+    constexpr int T = 2;                                        /* tiles of 16 columns */
+    extern __shared__ __align__(16) uint16_t ch_lds[];
+    const int32_t LD = a.ld, L = a.nlin;
+    int32_t *rowid = reinterpret_cast<int32_t *>(ch_lds + 2 * CH_ROWS * LD);      /* [CH_ROWS] rows of y */
+    const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1), w = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const uint32_t r16 = lane & 15u, kg = (lane >> 4) * 8u, rq = (lane >> 4) * 4u;
+    /* an XCD takes consecutive row tiles: two of them share the lines of the transposed copies */
+    const int32_t nt = (int32_t)gridDim.x, x = (int32_t)blockIdx.x % 8, q = (int32_t)blockIdx.x / 8;
+    const int32_t mt = x * (nt / 8) + min(x, nt % 8) + q;
+    const int32_t m0 = mt * CH_ROWS;
+    const int32_t S = TRAIN ? 2 * L - 1 : L;
+    /* rows rq .. rq + 3 of unit r16 in a fragment (rows 16 on: 256 further) */
+    const uint32_t fl = (rq / 8 * 16 + r16) * 8 + rq % 8;
+
+    /* the weights stream: two steps of 64 of the reduction index in registers,
+     * through the stages' ends.  Stages with an odd number of steps take one more,
+     * which is loaded (the last again) and not multiplied. */
+    bf16x8 B[2][T][2];
+    int32_t ls = 0, lc = 0, lnk = 0, lst = 0;
+    const uint16_t *lp[T];
+    auto enter = [&]() {
+        const ChainStage g = chain_stage(a, ls);
+        lnk = g.K / BK;
+        lst = g.N * 32;
+#pragma unroll
+        for (int j = 0; j < T; j++) {
+            /* columns past the stage's: any others of it */
+            const int32_t c = (int32_t)w * 32, col = (c < g.N ? c : 0) + j * 16;
+            lp[j] = g.w + col * 32;
+        }
+    };
+    auto issue = [&](bf16x8 (&b)[T][2]) {
+        const int32_t k = min(lc, lnk - 1) * 2 * lst;
+#pragma unroll
+        for (int j = 0; j < T; j++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) b[j][h] = *(const bf16x8 *)(lp[j] + k + h * lst + lane * 8u);
+        if (++lc >= ((lnk + 1) & ~1) && ls + 1 < S) {
+            ls++;
+            lc = 0;
+            enter();
+        }
+    };
+    enter();
+    issue(B[0]);
+    issue(B[1]);
+
+    /* the input rows: thread tid has four columns of row tid / 16 */
+    if (tid < CH_ROWS * 16) {
+        const int32_t r = (int32_t)tid / 16, c = (int32_t)(tid % 16) * 4;
+        uint2 v = {0u, 0u};
+        const int64_t row = a.rows ? (int64_t)a.rows[m0 + r] : (int64_t)(m0 + r);
+        if (a.xb) {
+            v = *(const uint2 *)(a.xb + row * BK + c);
+        } else if (row < a.n) {
+            uint16_t h[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) h[i] = c + i < a.din ? f2bf(a.xf[row * a.din + c + i]) : (uint16_t)0;
+            v = {(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16)};
+        }
+        *(uint2 *)(ch_lds + r * LD + c) = v;
+        if (c == 0) rowid[r] = (int32_t)row;
+    }
+    __syncthreads();
+    if (TRAIN && tid < CH_ROWS * 16) {
+        const int32_t k = (int32_t)tid / 8, r = (int32_t)(tid % 8) * 4;
+        const uint16_t *c = ch_lds + r * LD + k;
+        const uint2 v = {(uint32_t)c[0] | ((uint32_t)c[LD] << 16),
+                         (uint32_t)c[2 * LD] | ((uint32_t)c[3 * LD] << 16)};
+        *(uint2 *)(a.act_t[0] + frag_index(k, m0 + r, BK)) = v;
+    }
+
+    for (int32_t s = 0; s < S; s++) {
+        const ChainStage g = chain_stage(a, s);
+        const int32_t nk = g.K / BK;
+        const uint16_t *in = ch_lds + (s & 1) * CH_ROWS * LD;
+        uint16_t *nx = ch_lds + ((s + 1) & 1) * CH_ROWS * LD;
+        const bool fwd = !TRAIN || s < L;
+        float bias[T];
+        int32_t col[T];
+        int64_t fr[T];                                          /* this lane's rows of a transposed copy */
+        const int32_t c0 = (int32_t)w * 32;
+        const bool on = c0 < g.N;                               /* uniform */
+#pragma unroll
+        for (int j = 0; j < T; j++) {
+            col[j] = (on ? c0 : 0) + j * 16 + (int32_t)r16;
+            fr[j] = ((int64_t)mt * (g.N / 16) + (on ? c0 : 0) / 16 + j) * 512;
+            bias[j] = fwd ? a.p[a.boff[s] + col[j]] : 0.f;
+        }
+        f32x4 acc[2][T];
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < T; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        auto mul = [&](bf16x8 (&b)[T][2], int32_t k0) {
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                bf16x8 av[2];
+#pragma unroll
+                for (int i = 0; i < 2; i++) av[i] = *(const bf16x8 *)(in + (i * 16 + r16) * LD + k0 + h * 32 + kg);
+#pragma unroll
+                for (int j = 0; j < T; j++)
+#pragma unroll
+                    for (int i = 0; i < 2; i++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[i], b[j][h], acc[i][j], 0, 0, 0);
+            }
+        };
+        /* dZ of layer l's output is what a stage from the loss on forms */
+        const int32_t l = s < L ? s : 2 * L - 2 - s;
+        uint16_t *tr = !TRAIN ? nullptr : s < L - 1 ? a.act_t[s + 1] : a.dzt[l];
+        float yv[2][T][4];
+        uint2 act[2][T];
+        if (TRAIN && s == L - 1) {
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int64_t row = rowid[i * 16 + (int32_t)rq + r];
+#pragma unroll
+                    for (int j = 0; j < T; j++) yv[i][j][r] = a.y[row * a.ny + min(col[j], a.ny - 1)];
+                }
+        }
+        if (TRAIN && s >= L) {
+            /* this lane's own values, written in the forward stage */
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < T; j++)
+                    act[i][j] = *(const uint2 *)(a.act_t[l + 1] + fr[j] + i * 256 + fl);
+        }
+        int32_t c = 0;
+        do {
+            mul(B[0], c * BK);
+            issue(B[0]);
+            if (c + 1 < nk) mul(B[1], (c + 1) * BK);
+            issue(B[1]);
+            c += 2;
+        } while (c < nk);           /* at least once: the loads before it then have 16 after them */
+        /* lane holds rows 16 i + rq + r, columns col[j] */
+        if (!TRAIN && s == L - 1) {
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < T; j++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        if (on) a.out[(int64_t)(m0 + i * 16 + (int32_t)rq + r) * g.N + col[j]] = acc[i][j][r] + bias[j];
+            break;
+        }
+        uint2 h[2][T];                                          /* the stage's bf16 values */
+        if (s < L - 1) {
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < T; j++) {
+                    float z[4];
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        z[r] = acc[i][j][r] + bias[j];
+                        z[r] = z[r] > 0.f ? z[r] : 0.f;
+                    }
+                    h[i][j] = uint2{pack_bf(z[0], z[1]), pack_bf(z[2], z[3])};
+                }
+        } else if (TRAIN && s == L - 1) {
+            float lsum = 0.f;
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < T; j++) {
+                    float z[4];
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const float diff = col[j] < a.ny ? acc[i][j][r] + bias[j] - yv[i][j][r] : 0.f;
+                        lsum += diff * diff;
+                        z[r] = a.scale * diff;
+                    }
+                    h[i][j] = uint2{pack_bf(z[0], z[1]), pack_bf(z[2], z[3])};
+                }
+#pragma unroll
+            for (int o = 1; o < WAVE; o <<= 1) lsum += __shfl_xor(lsum, o);
+            /* a quadrant of a tile of 64 x 64 */
+            if (lane == 0 && on)
+                a.lpart[((int64_t)(mt / 2) * (g.N / BN) + w / 2) * 4 + (mt & 1) * 2 + (w & 1)] = lsum;
+        } else if (TRAIN) {
+            /* where the activation is not 0 (it is never below) */
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < T; j++) {
+                    h[i][j] = uint2{pack_bf(acc[i][j][0], acc[i][j][1]), pack_bf(acc[i][j][2], acc[i][j][3])};
+                    h[i][j].x &= nonzero_halves(act[i][j].x);
+                    h[i][j].y &= nonzero_halves(act[i][j].y);
+                }
+        }
+#pragma unroll
+        for (int j = 0; j < T; j++) {
+            if (!on) continue;                                  /* uniform */
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                uint16_t *c = nx + (i * 16 + rq) * LD + col[j];
+                c[0] = (uint16_t)h[i][j].x;
+                c[LD] = (uint16_t)(h[i][j].x >> 16);
+                c[2 * LD] = (uint16_t)h[i][j].y;
+                c[3 * LD] = (uint16_t)(h[i][j].y >> 16);
+                if (TRAIN) *(uint2 *)(tr + fr[j] + i * 256 + fl) = h[i][j];
+            }
+            if (TRAIN && s >= L - 1) {
+                float v = 0.f;
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    v += __uint_as_float(h[i][j].x << 16);
+                    v += __uint_as_float(h[i][j].x & 0xFFFF0000u);
+                    v += __uint_as_float(h[i][j].y << 16);
+                    v += __uint_as_float(h[i][j].y & 0xFFFF0000u);
+                }
+                v += __shfl_xor(v, 16);
+                v += __shfl_xor(v, 32);
+                if (lane < 16) a.bpart[l][(int64_t)mt * g.N + col[j]] = v;
+            }
+        }
+        __syncthreads();
+    }
+}
+
+/* ---- weight gradients and Adam ---------------------------------------------- */
+
+struct UpdateArgs {
+    int32_t nlin, batch;
+    int32_t n[MAX_LAYERS], k[MAX_LAYERS];   /* W_l is [n][k] */
+    int32_t tfirst[MAX_LAYERS + 1];         /* first 64 x 64 tile of W_l */
+    int32_t bfirst[MAX_LAYERS + 1];         /* first bias workgroup of layer l; those before the tiles': */
+    int32_t nbias;                          /*   a multiple of 8, the last ones idle */
+    int32_t update;                         /* 0: only write the gradient */
+    int64_t woff[MAX_LAYERS], boff[MAX_LAYERS];
+    const uint16_t *dzt[MAX_LAYERS], *act_t[MAX_LAYERS];    /* [unit][batch], in fragments */
+    const float *bpart[MAX_LAYERS];         /* bias-gradient partials [batch / 32][n] */
+    float lr, b1, b2, eps, c1, c2;          /* c1 = 1 - b1^t, c2 = 1 - b2^t */
     float *p, *m, *v, *grad;
-    uint16_t *pbf;
-    const float *lpart;   /* loss partials of the step, summed by wavefront 0 of workgroup 0 */
+    uint16_t *w, *wt;                       /* bf16 W_l and W_l^T at woff[l], in fragments */
+    const float4 *lpart;                    /* loss partials of the step */
     int32_t nlpart;
     float lscale;
     float *loss;
 };
 
-/* Adam (Kingma & Ba, 2015) for the j-th parameter of segment sg: sums its
- * gradient partials in a fixed order, updates the fp32 master (m, v in fp32)
- * and writes the bf16 copy; returns the new bf16 value (0 when only the
- * gradient is written). */
-__device__ inline uint16_t adam_elem(const AdamArgs &a, const AdamSeg &sg, int64_t j)
+/* Adam (Kingma & Ba, 2015) for one parameter: its state before, gradient g;
+ * the parameter after. */
+__device__ inline float adam(const UpdateArgs &a, int64_t i, float g, float p, float m, float v)
 {
-    const int64_t i = sg.off + j;
-    float gsum = 0.f;
-#pragma unroll 8
-    for (int32_t k = 0; k < sg.nparts; k++) gsum += sg.parts[(int64_t)k * sg.count + j];
-    if (a.grad) a.grad[i] = gsum;
-    if (!a.update) return 0;
-    const float m = a.b1 * a.m[i] + (1.f - a.b1) * gsum;
-    const float v = a.b2 * a.v[i] + (1.f - a.b2) * (gsum * gsum);
+    m = a.b1 * m + (1.f - a.b1) * g;
+    v = a.b2 * v + (1.f - a.b2) * (g * g);
     a.m[i] = m;
     a.v[i] = v;
     const float mhat = m / a.c1, vhat = v / a.c2;
-    const float p = a.p[i] - a.lr * (mhat / (sqrtf(vhat) + a.eps));
+    p -= a.lr * (mhat / (sqrtf(vhat) + a.eps));
     a.p[i] = p;
-    const uint16_t h = f2bf(p);
-    a.pbf[i] = h;
-    return h;
+    return p;
 }
 
-/* adam_elem for E parameters j[0..E-1] of one segment at once: every load
- * of the E is issued before the first store (the same arithmetic, element by
- * element). */
-template <int E>
-__device__ inline void adam_elems(const AdamArgs &a, const AdamSeg &sg, const int64_t (&j)[E], uint16_t (&h)[E])
+typedef uint16_t WTile[64][66];
+
+/* A 64 x 64 tile (row r0, column c0) of W [N][K] to the bf16 copies of W and
+ * its transpose: a lane's eight elements of a fragment at a time. */
+__device__ inline void put_weights(const WTile &tile, uint16_t *w, uint16_t *wt, int32_t N, int32_t K, int32_t r0,
+                                   int32_t c0)
 {
-    float g[E], mo[E], vo[E], po[E];
+    for (int32_t x = (int32_t)threadIdx.x; x < 512; x += (int32_t)blockDim.x) {
+        const int32_t f = x / 64, l = x % 64;
+        const int32_t n = f / 2 * 16 + l % 16, k = f % 2 * 32 + l / 16 * 8;
+        uint32_t q[4], t[4];
 #pragma unroll
-    for (int e = 0; e < E; e++) g[e] = 0.f;
-    for (int32_t k = 0; k < sg.nparts; k++)
+        for (int i = 0; i < 4; i++) {
+            q[i] = (uint32_t)tile[n][k + 2 * i] | ((uint32_t)tile[n][k + 2 * i + 1] << 16);
+            t[i] = (uint32_t)tile[k + 2 * i][n] | ((uint32_t)tile[k + 2 * i + 1][n] << 16);
+        }
+        *(uint4 *)(w + frag_index(r0 + n, c0 + k, N)) = uint4{q[0], q[1], q[2], q[3]};
+        *(uint4 *)(wt + frag_index(c0 + n, r0 + k, K)) = uint4{t[0], t[1], t[2], t[3]};
+    }
+}
+
+/* One workgroup per 64 x 64 tile of a weight matrix: dW_l = dZ_l^T H_l, a
+ * quarter of the batch per wavefront, the quarters' sums added in order, then
+ * Adam on the tile and its bf16 copies.
+ *
+ * What bounds it: a tile reads 1 MB of fragments at 4,096 rows, 6.8 us at the 64
+ * bytes per cycle of a compute unit, of which a few are waits for what other
+ * XCDs wrote; 8 us go to the launch, the exchange of the sums and Adam's divides
+ * and square roots.  Without LDS for the operands: each wavefront multiplies 64 x
+ * 64 outputs from registers (8 KB of loads per 16 MFMAs).  In two launches, with
+ * the four sums written out and read back, this took 25 + 10 us where it takes
+ * 22 now (950,000 parameters, 4,096 rows), and 27 + 10 / 22 (2,600,000, 2,048
+ * rows).  Four steps in flight instead of two need the registers of a second
+ * workgroup per compute unit: 28 us for the latter.
+ * The workgroups before them take 256 biases each, the first also the step's loss. */
+constexpr int UP_THREADS = KSPLIT * WAVE;
+constexpr int UP_DEPTH = 2;                /* steps of 32 rows in flight; a quarter of a batch has whole pairs */
+constexpr int UP_JS = 80, UP_IR = 4 * UP_JS;     /* LDS strides (floats) of a sum's 16 columns and 4 x 16 */
+
+__global__ __launch_bounds__(UP_THREADS) void mlp_update(UpdateArgs a)
+{
+    __shared__ __align__(16) float sums[KSPLIT][16 * UP_IR];
+    const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1), w = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    if ((int32_t)blockIdx.x < a.nbias) {
+        if (blockIdx.x == 0 && w == 0 && a.loss) {
+            /* lane l adds partials l, l + 64, ... in order, then a fixed
+             * butterfly combines the lanes */
+            float s = 0.f;
+#pragma unroll 4
+            for (int32_t k = (int32_t)lane; k < a.nlpart; k += WAVE) {
+                const float4 q = a.lpart[k];
+                s += ((q.x + q.y) + q.z) + q.w;
+            }
 #pragma unroll
-        for (int e = 0; e < E; e++) g[e] += sg.parts[(int64_t)k * sg.count + j[e]];
-    if (a.grad)
-#pragma unroll
-        for (int e = 0; e < E; e++) a.grad[sg.off + j[e]] = g[e];
-    if (!a.update) {
-#pragma unroll
-        for (int e = 0; e < E; e++) h[e] = 0;
+            for (int o = 1; o < WAVE; o <<= 1) s += __shfl_xor(s, o);
+            if (lane == 0) *a.loss = s * a.lscale;
+        }
+        const int32_t b = (int32_t)blockIdx.x;
+        if (b >= a.bfirst[a.nlin]) return;
+        int l = 0;
+        while (l + 1 < a.nlin && b >= a.bfirst[l + 1]) l++;
+        const int32_t n = a.n[l], j = (b - a.bfirst[l]) * UP_THREADS + (int32_t)tid;
+        if (j >= n) return;
+        /* the partials in order, the two of every 64 rows first */
+        const float *parts = a.bpart[l] + j;
+        float g = 0.f;
+#pragma unroll 32
+        for (int32_t k = 0; k < a.batch / ROWS_PER_PART; k += 2)
+            g += parts[(int64_t)k * n] + parts[(int64_t)(k + 1) * n];
+        const int64_t i = a.boff[l] + j;
+        if (a.grad) a.grad[i] = g;
+        if (a.update) (void)adam(a, i, g, a.p[i], a.m[i], a.v[i]);
         return;
     }
+    /* an XCD takes consecutive tiles: they share rows of dZ */
+    const int32_t nt = a.tfirst[a.nlin], b = (int32_t)blockIdx.x - a.nbias, x = b % 8;
+    const int32_t t = x * (nt / 8) + min(x, nt % 8) + b / 8;
+    int l = 0;
+    while (l + 1 < a.nlin && t >= a.tfirst[l + 1]) l++;
+    const int32_t N = a.n[l], K = a.k[l], tk = K / 64, ti = t - a.tfirst[l];
+    const int32_t r0 = (ti / tk) * 64, c0 = (ti % tk) * 64;
+    const int32_t ns = a.batch / 32 / KSPLIT;
+    const uint16_t *pa = a.dzt[l] + ((int64_t)w * ns * N + r0) * 32;
+    const uint16_t *pb = a.act_t[l] + ((int64_t)w * ns * K + c0) * 32;
+    constexpr int D = UP_DEPTH;
+    bf16x8 fa[D][4], fb[D][4];
+    f32x4 acc[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto issue = [&](int d, int32_t s) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            fa[d][i] = *(const bf16x8 *)(pa + (int64_t)s * N * 32 + i * 512 + lane * 8u);
+            fb[d][i] = *(const bf16x8 *)(pb + (int64_t)s * K * 32 + i * 512 + lane * 8u);
+        }
+    };
+    auto mul = [&](int d) {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[d][i], fb[d][j], acc[i][j], 0, 0, 0);
+    };
+    /* Adam's operands, which so arrive during the products.  Thread: column lane of
+     * rows w, w + 4, ... of the tile */
+    constexpr int E = 64 / KSPLIT;
+    float g[E], po[E], mo[E], vo[E];
+    const int64_t i0 = a.woff[l] + (int64_t)(r0 + (int32_t)w) * K + c0 + lane;
+    if (a.update) {
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const int64_t i = i0 + (int64_t)e * KSPLIT * K;
+            po[e] = a.p[i];
+            mo[e] = a.m[i];
+            vo[e] = a.v[i];
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < D; d++) issue(d, d);
+    for (int32_t s = D; s < ns; s += D) {
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            mul(d);
+            issue(d, s + d);
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < D; d++) mul(d);
+    /* lane holds rows 16 i + 4 (lane / 16) + r, column 16 j + lane % 16 */
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) sums[w][(i * 4 + r) * UP_IR + j * UP_JS + lane] = acc[i][j][r];
+    __syncthreads();
 #pragma unroll
     for (int e = 0; e < E; e++) {
-        mo[e] = a.m[sg.off + j[e]];
-        vo[e] = a.v[sg.off + j[e]];
-        po[e] = a.p[sg.off + j[e]];
-    }
+        const uint32_t row = w + e * KSPLIT;
+        const uint32_t o = (row / 16 * 4 + row % 4) * UP_IR + lane / 16 * UP_JS + row % 16 / 4 * 16 + lane % 16;
+        g[e] = 0.f;
 #pragma unroll
-    for (int e = 0; e < E; e++) {
-        const int64_t i = sg.off + j[e];
-        const float m = a.b1 * mo[e] + (1.f - a.b1) * g[e];
-        const float v = a.b2 * vo[e] + (1.f - a.b2) * (g[e] * g[e]);
-        a.m[i] = m;
-        a.v[i] = v;
-        const float mhat = m / a.c1, vhat = v / a.c2;
-        const float p = po[e] - a.lr * (mhat / (sqrtf(vhat) + a.eps));
-        a.p[i] = p;
-        h[e] = f2bf(p);
-        a.pbf[i] = h[e];
+        for (int z = 0; z < KSPLIT; z++) g[e] += sums[z][o];
     }
+    if (a.grad)
+#pragma unroll
+        for (int e = 0; e < E; e++) a.grad[i0 + (int64_t)e * KSPLIT * K] = g[e];
+    if (!a.update) return;                                      /* uniform */
+    __syncthreads();                                            /* the sums are read */
+    WTile &tile = *reinterpret_cast<WTile *>(&sums[0][0]);
+#pragma unroll
+    for (int e = 0; e < E; e++)
+        tile[w + e * KSPLIT][lane] = f2bf(adam(a, i0 + (int64_t)e * KSPLIT * K, g[e], po[e], mo[e], vo[e]));
+    __syncthreads();
+    put_weights(tile, a.w + a.woff[l], a.wt + a.woff[l], N, K, r0, c0);
 }
 
-/* Adam over every parameter, with the transposed bf16 weights written
- * alongside (the copy the activation-gradient products read): workgroups 0 .. wfirst[nlin] - 1 take
- * one 64 x 64 tile of a weight matrix each and transpose its new bf16 values
- * through LDS, the others 256 bias entries each. */
-struct AdamTileArgs {
-    AdamArgs a;
-    int32_t n[MAX_LAYERS], k[MAX_LAYERS];   /* W_l is [n][k] */
-    int32_t wfirst[MAX_LAYERS + 1];         /* first tile workgroup of W_l */
-    int32_t bfirst[MAX_LAYERS + 1];         /* first bias workgroup of layer l, after the tiles */
-    int32_t nlin;
-    uint16_t *pbf_t;                        /* W_l^T [k][n] at the offset of W_l */
-};
-
-constexpr int ADAM_THREADS = 1024;                   /* 4 parameters of a tile per thread */
-constexpr int ADAM_ROWS_STEP = ADAM_THREADS / 64;
-
-__global__ __launch_bounds__(ADAM_THREADS) void mlp_adam_tiles(AdamTileArgs t)
-{
-    __shared__ uint16_t tile[64][66];
-    const AdamArgs &a = t.a;
-    if (blockIdx.x == 0 && threadIdx.x < WAVE && a.loss) {
-        /* the step's loss from the output tiles' partials: lane l adds
-         * partials l, l + 64, ... in order (their loads issued together),
-         * then a fixed butterfly combines the lanes; lane 0's total is
-         * written (one thread adding them one by one waited for each load
-         * in turn, which made this workgroup the last of the launch) */
-        float s = 0.f;
-#pragma unroll 4
-        for (int32_t k = (int32_t)threadIdx.x; k < a.nlpart; k += WAVE) s += a.lpart[k];
-#pragma unroll
-        for (int o = 1; o < WAVE; o <<= 1) s += __shfl_xor(s, o);
-        if (threadIdx.x == 0) *a.loss = s * a.lscale;
-    }
-    const int32_t b = (int32_t)blockIdx.x;
-    if (b < t.wfirst[t.nlin]) {
-        int l = 0;
-        while (l + 1 < t.nlin && b >= t.wfirst[l + 1]) l++;
-        const int32_t ti = b - t.wfirst[l], tk = t.k[l] / 64;
-        const int32_t r0 = (ti / tk) * 64, c0 = (ti % tk) * 64;
-        const AdamSeg &sg = a.seg[2 * l];
-        const uint32_t x = threadIdx.x & 63u, y = threadIdx.x >> 6;
-        constexpr int E = 64 / ADAM_ROWS_STEP;
-        int64_t j[E];
-        uint16_t h[E];
-#pragma unroll
-        for (int e = 0; e < E; e++) j[e] = (int64_t)(r0 + (int32_t)y + e * ADAM_ROWS_STEP) * t.k[l] + c0 + x;
-        adam_elems<E>(a, sg, j, h);
-#pragma unroll
-        for (int e = 0; e < E; e++) tile[y + e * ADAM_ROWS_STEP][x] = h[e];
-        if (!a.update) return;                    /* uniform */
-        __syncthreads();
-        uint16_t *wt = t.pbf_t + sg.off;
-        for (uint32_t c = y; c < 64; c += ADAM_ROWS_STEP) wt[(int64_t)(c0 + c) * t.n[l] + r0 + x] = tile[x][c];
-    } else {
-        const int32_t bb = b - t.wfirst[t.nlin];
-        int l = 0;
-        while (l + 1 < t.nlin && bb >= t.bfirst[l + 1]) l++;
-        const AdamSeg &sg = a.seg[2 * l + 1];
-        const int64_t j = (int64_t)(bb - t.bfirst[l]) * ADAM_THREADS + threadIdx.x;
-        if (j < sg.count) (void)adam_elem(a, sg, j);
-    }
-}
-
-/* Input conversion: f32 [n][in_dim] -> bf16 [n][kin] (zero padded). */
+/* Input conversion: f32 [rows][in_dim] -> bf16 [n][kin] (zero padded). */
 __global__ __launch_bounds__(256) void mlp_convert_x(const float *x, uint16_t *xb, uint16_t *xb_t,
-                                                     int64_t n, int32_t in_dim, int32_t kin)
+                                                     int64_t n, int64_t rows, int32_t in_dim, int32_t kin)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n * kin) return;
     const int64_t r = i / kin;
     const int32_t c = (int32_t)(i % kin);
-    const uint16_t v = c < in_dim ? f2bf(x[r * in_dim + c]) : (uint16_t)0;
+    const uint16_t v = c < in_dim && r < rows ? f2bf(x[r * in_dim + c]) : (uint16_t)0;
     xb[i] = v;
-    if (xb_t) xb_t[(int64_t)c * n + r] = v;
+    if (xb_t) xb_t[frag_index(c, (int32_t)r, kin)] = v;
 }
 
-struct TransArgs {
-    int64_t off[MAX_LAYERS];    /* weight matrix l at off[l] in both copies */
+struct PackArgs {
+    int64_t off[MAX_LAYERS];    /* weight matrix l at off[l] in all copies */
     int32_t n[MAX_LAYERS], k[MAX_LAYERS];
     int32_t first[MAX_LAYERS + 1];   /* first 64 x 64 tile of matrix l */
     int32_t nlin;
-    const uint16_t *w;           /* W_l [n][k] */
-    uint16_t *wt;                /* W_l^T [k][n] */
+    const float *p;              /* W_l [n][k] */
+    uint16_t *w, *wt;            /* bf16 W_l and W_l^T, in fragments */
 };
 
-/* bf16 weight copies transposed through LDS, one 64 x 64 tile per workgroup. */
-__global__ __launch_bounds__(256) void mlp_transpose_w(TransArgs a)
+/* The bf16 weights and their transpose from the master, one 64 x 64 tile per
+ * workgroup. */
+__global__ __launch_bounds__(256) void mlp_pack(PackArgs a)
 {
-    __shared__ uint16_t t[64][66];
+    __shared__ WTile t;
     int l = 0;
     while (l + 1 < a.nlin && (int32_t)blockIdx.x >= a.first[l + 1]) l++;
     const int32_t tile = blockIdx.x - a.first[l];
     const int32_t tk = a.k[l] / 64;
     const int32_t r0 = (tile / tk) * 64, c0 = (tile % tk) * 64;
-    const uint16_t *w = a.w + a.off[l];
-    uint16_t *wt = a.wt + a.off[l];
-    const uint32_t x = threadIdx.x & 63u, y = threadIdx.x >> 6;
-    for (uint32_t r = y; r < 64; r += 4) t[r][x] = w[(int64_t)(r0 + r) * a.k[l] + c0 + x];
+    const uint32_t x = threadIdx.x & 63u;
+    for (uint32_t y = threadIdx.x >> 6; y < 64; y += 4)
+        t[y][x] = f2bf(a.p[a.off[l] + (int64_t)(r0 + y) * a.k[l] + c0 + x]);
     __syncthreads();
-    for (uint32_t c = y; c < 64; c += 4) wt[(int64_t)(c0 + c) * a.n[l] + r0 + x] = t[x][c];
+    put_weights(t, a.w + a.off[l], a.wt + a.off[l], a.n[l], a.k[l], r0, c0);
 }
 
 template <int EPI>
-hipError_t gemm(const GemmArgs &g, int32_t splits, hipStream_t st)
+hipError_t gemm(const GemmArgs &g, hipStream_t st)
 {
-    const dim3 grid(g.N / BN, g.M / BM, splits);
+    const dim3 grid((uint32_t)(g.N / BN) * (uint32_t)(g.M / BM));
     (void)hipGetLastError();   /* the check after the launch reports it alone */
     hipLaunchKernelGGL((mlp_gemm<EPI>), grid, dim3(GEMM_THREADS), 0, st, g);
     return hipGetLastError();
@@ -557,19 +909,18 @@ struct bsim_mlp {
     hipStream_t stream = nullptr;
     std::vector<void *> allocs;
     float *p = nullptr, *m = nullptr, *v = nullptr, *grad = nullptr;
-    uint16_t *pbf = nullptr;
-    uint16_t *pbf_t = nullptr;        /* weights transposed (W_l^T [k][n] at woff[l]) */
+    uint16_t *pbf = nullptr, *pbf_t = nullptr;   /* bf16 W_l and W_l^T at woff[l], in fragments */
     uint16_t *act[MAX_LAYERS + 1]{};  /* act[0] input, act[l] hidden l (bf16) */
     float *out = nullptr, *ybat = nullptr;
     uint16_t *dz[2]{};                /* activation gradients (ping-pong) */
-    uint16_t *act_t[MAX_LAYERS]{};    /* act[l] transposed, [kdim[l]][batch] */
-    float *wpart[MAX_LAYERS]{}, *bpart[MAX_LAYERS]{};
+    uint16_t *act_t[MAX_LAYERS]{};    /* act[l] transposed, [kdim[l]][batch] in fragments */
+    float *bpart[MAX_LAYERS]{};
     float *lpart = nullptr, *loss = nullptr;
     uint16_t *xall = nullptr;
     float *yall = nullptr;
     int64_t ndata = 0;
     float *xstage = nullptr;          /* predict input staging (f32) */
-    uint16_t *dzt[MAX_LAYERS]{};      /* dZ of layer l's output, transposed [kdim[l+1]][batch] */
+    uint16_t *dzt[MAX_LAYERS]{};      /* dZ of layer l's output, transposed [kdim[l+1]][batch] in fragments */
 };
 
 namespace {
@@ -610,6 +961,60 @@ double hash_uniform(uint64_t seed, uint64_t i)
     return (double)(z >> 11) * (2.0 / 9007199254740992.0) - 1.0;
 }
 
+bool chained(const bsim_mlp *m)
+{
+    return *std::max_element(m->kdim, m->kdim + m->nlin + 1) <= CH_MAX;
+}
+
+/* The chain's launch: predict (xf f32 input of n rows, output in m->out), or
+ * training (as forward and the activation gradients of backward), from the
+ * resident rows or, with rows null, from xstage and ybat. */
+int chain(bsim_mlp *m, int32_t batch, bool train, const int32_t *rows, int64_t n)
+{
+    const int L = m->nlin;
+    ChainArgs a{};
+    a.nlin = L;
+    int32_t wide = 0;
+    for (int l = 0; l <= L; l++) {
+        a.kdim[l] = m->kdim[l];
+        wide = std::max(wide, m->kdim[l]);
+    }
+    a.ld = wide + 8;
+    a.din = m->cfg.in_dim;
+    for (int l = 0; l < L; l++) {
+        a.woff[l] = m->woff[l];
+        a.boff[l] = m->boff[l];
+        a.act_t[l] = m->act_t[l];
+        a.dzt[l] = m->dzt[l];
+        a.bpart[l] = m->bpart[l];
+    }
+    a.w = m->pbf;
+    a.wt = m->pbf_t;
+    a.p = m->p;
+    a.xb = rows ? m->xall : nullptr;
+    a.xf = m->xstage;
+    a.rows = rows;
+    a.n = n;
+    a.out = m->out;
+    a.lpart = m->lpart;
+    a.y = rows ? m->yall : m->ybat;
+    a.ny = m->cfg.out_dim;
+    a.scale = 2.0f / ((float)batch * (float)m->cfg.out_dim);
+    const dim3 grid((uint32_t)(batch / CH_ROWS));
+    const size_t lds = (size_t)2 * CH_ROWS * a.ld * 2 + CH_ROWS * 4;
+    (void)hipGetLastError();   /* the check after the launch reports it alone */
+#define CHAIN(W, TRAIN) hipLaunchKernelGGL((mlp_chain<W, TRAIN>), grid, dim3((W) * WAVE), lds, m->stream, a)
+    if (wide <= CH_MAX / 2) {
+        if (train) CHAIN(8, true);
+        else CHAIN(8, false);
+    } else {
+        if (train) CHAIN(16, true);
+        else CHAIN(16, false);
+    }
+#undef CHAIN
+    return hip_check(hipGetLastError(), "chain launch");
+}
+
 /* Forward pass of a batch.  predict (train false): from act[0], fp32 output
  * in m->out.  train: the hidden activations also written transposed, and the
  * output layer forms the loss partials, dZ of the output (row-major and
@@ -627,21 +1032,19 @@ int forward(bsim_mlp *m, int32_t batch, bool train, const int32_t *rows = nullpt
         g.a_t = (l == 0 && rows) ? m->act_t[0] : nullptr;
         g.lda = m->kdim[l];
         g.B = m->pbf + m->woff[l];
-        g.ldb = m->kdim[l];
         g.M = batch;
         g.N = m->kdim[l + 1];
         g.K = m->kdim[l];
         g.bias = m->p + m->boff[l];
         g.ldo = m->kdim[l + 1];
-        g.ldt = batch;
         hipError_t e;
         if (l + 1 < L) {
             g.out_bf = m->act[l + 1];
             g.out_t = train ? m->act_t[l + 1] : nullptr;
-            e = gemm<EPI_RELU_BF16>(g, 1, m->stream);
+            e = gemm<EPI_RELU_BF16>(g, m->stream);
         } else if (!train) {
             g.out_f = m->out;
-            e = gemm<EPI_LINEAR_F32>(g, 1, m->stream);
+            e = gemm<EPI_LINEAR_F32>(g, m->stream);
         } else {
             g.out_bf = m->dz[0];
             g.out_t = m->dzt[L - 1];
@@ -651,17 +1054,16 @@ int forward(bsim_mlp *m, int32_t batch, bool train, const int32_t *rows = nullpt
             g.yrow = rows;
             g.ny = m->cfg.out_dim;
             g.scale = 2.0f / ((float)batch * (float)m->cfg.out_dim);
-            e = gemm<EPI_LOSS>(g, 1, m->stream);
+            e = gemm<EPI_LOSS>(g, m->stream);
         }
         if (e != hipSuccess) return hip_check(e, "forward launch");
     }
     return BSIM_OK;
 }
 
-/* Backward pass of a batch after a training forward pass (which formed dZ
- * of the output): gradient partials left in wpart / bpart.  The activation
- * gradients go down the layers one GEMM each, their transposed copies kept
- * per layer, and then every weight gradient is formed in one launch. */
+/* The activation gradients after a training forward pass (which formed dZ of
+ * the output), one GEMM each down the layers: transposed copies in dzt, bias
+ * partials in bpart. */
 int backward(bsim_mlp *m, int32_t batch)
 {
     const int L = m->nlin;
@@ -674,7 +1076,6 @@ int backward(bsim_mlp *m, int32_t batch)
         gx.A = m->dz[cur];
         gx.lda = m->kdim[l + 1];
         gx.B = m->pbf_t + m->woff[l];
-        gx.ldb = m->kdim[l + 1];
         gx.M = batch;
         gx.N = m->kdim[l];
         gx.K = m->kdim[l + 1];
@@ -683,80 +1084,60 @@ int backward(bsim_mlp *m, int32_t batch)
         gx.mask = m->act[l];
         gx.bpart = m->bpart[l - 1];
         gx.out_t = m->dzt[l - 1];
-        gx.ldt = batch;
-        e = gemm<EPI_DRELU_BF16>(gx, 1, m->stream);
+        e = gemm<EPI_DRELU_BF16>(gx, m->stream);
         if (e != hipSuccess) return hip_check(e, "activation-gradient launch");
         cur ^= 1;
     }
-    /* dW_l [kdim[l+1]][kdim[l]] = dZ_l^T H_l: A(m = out unit, k = row) = dzt[l][m][k],
-     * B(n = in unit, k = row) = act_t[l][n][k]; every layer in one launch */
-    GemmGroup g{};
-    g.n = L;
-    for (int l = 0; l < L; l++) {
-        GemmArgs &x = g.g[l];
-        x.A = m->dzt[l];
-        x.lda = batch;
-        x.B = m->act_t[l];
-        x.ldb = batch;
-        x.M = m->kdim[l + 1];
-        x.N = m->kdim[l];
-        x.K = batch / KSPLIT;
-        x.out_f = m->wpart[l];
-        x.ldo = m->kdim[l];
-        g.first[l + 1] = g.first[l] + (x.M / BM) * (x.N / BN) * KSPLIT;
-    }
-    (void)hipGetLastError();   /* the check after the launch reports it alone */
-    hipLaunchKernelGGL(mlp_gemm_partials, dim3(g.first[L]), dim3(GEMM_THREADS), 0, m->stream, g);
-    return hip_check(hipGetLastError(), "weight-gradient launch");
+    return BSIM_OK;
 }
 
-int adam(bsim_mlp *m, int32_t batch, bool update, float lr, float *grad_out, float *loss_dev)
+/* Weight and bias gradients of a batch, and with update Adam's step. */
+int update(bsim_mlp *m, int32_t batch, bool upd, float lr, float *grad_out, float *loss_dev)
 {
-    AdamArgs a{};
-    a.nseg = 2 * m->nlin;
-    for (int l = 0; l < m->nlin; l++) {
-        a.seg[2 * l] = AdamSeg{m->woff[l], (int64_t)m->kdim[l + 1] * m->kdim[l], m->wpart[l], KSPLIT, 0};
-        a.seg[2 * l + 1] = AdamSeg{m->boff[l], m->kdim[l + 1], m->bpart[l], batch / ROWS_PER_PART, 0};
+    const int L = m->nlin, t = m->step + 1;
+    UpdateArgs a{};
+    a.nlin = L;
+    a.batch = batch;
+    for (int l = 0; l < L; l++) {
+        a.n[l] = m->kdim[l + 1];
+        a.k[l] = m->kdim[l];
+        a.tfirst[l + 1] = a.tfirst[l] + (a.n[l] / 64) * (a.k[l] / 64);
+        a.bfirst[l + 1] = a.bfirst[l] + (a.n[l] + UP_THREADS - 1) / UP_THREADS;
+        a.woff[l] = m->woff[l];
+        a.boff[l] = m->boff[l];
+        a.dzt[l] = m->dzt[l];
+        a.act_t[l] = m->act_t[l];
+        a.bpart[l] = m->bpart[l];
     }
-    a.update = update ? 1 : 0;
+    a.nbias = (int32_t)round_up(a.bfirst[L], 8);
+    a.update = upd ? 1 : 0;
     a.lr = lr;
     a.b1 = m->cfg.beta1;
     a.b2 = m->cfg.beta2;
     a.eps = m->cfg.eps;
-    const int t = m->step + 1;
     a.c1 = (float)(1.0 - std::pow((double)m->cfg.beta1, t));
     a.c2 = (float)(1.0 - std::pow((double)m->cfg.beta2, t));
     a.p = m->p;
     a.m = m->m;
     a.v = m->v;
     a.grad = grad_out;
-    a.pbf = m->pbf;
-    a.lpart = m->lpart;
-    a.nlpart = batch / ROWS_PER_PART * (m->kdim[m->nlin] / 64);
+    a.w = m->pbf;
+    a.wt = m->pbf_t;
+    a.lpart = (const float4 *)m->lpart;
+    a.nlpart = batch / BM * (m->kdim[L] / BN);
     a.lscale = 1.0f / ((float)batch * (float)m->cfg.out_dim);
     a.loss = loss_dev;
-    AdamTileArgs ta{};
-    ta.a = a;
-    ta.nlin = m->nlin;
-    ta.pbf_t = m->pbf_t;
-    for (int l = 0; l < m->nlin; l++) {
-        ta.n[l] = m->kdim[l + 1];
-        ta.k[l] = m->kdim[l];
-        ta.wfirst[l + 1] = ta.wfirst[l] + (ta.n[l] / 64) * (ta.k[l] / 64);
-        ta.bfirst[l + 1] = ta.bfirst[l] + (ta.n[l] + ADAM_THREADS - 1) / ADAM_THREADS;
-    }
     (void)hipGetLastError();   /* the check after the launch reports it alone */
-    hipLaunchKernelGGL(mlp_adam_tiles, dim3((uint32_t)(ta.wfirst[m->nlin] + ta.bfirst[m->nlin])),
-                       dim3(ADAM_THREADS), 0, m->stream, ta);
+    hipLaunchKernelGGL(mlp_update, dim3((uint32_t)(a.nbias + a.tfirst[L])), dim3(UP_THREADS), 0, m->stream, a);
     const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return hip_check(e, "adam launch");
-    if (update) m->step++;
+    if (e != hipSuccess) return hip_check(e, "update launch");
+    if (upd) m->step++;
     return BSIM_OK;
 }
 
-int transpose_weights(bsim_mlp *m)
+int pack_weights(bsim_mlp *m)
 {
-    TransArgs a{};
+    PackArgs a{};
     a.nlin = m->nlin;
     a.first[0] = 0;
     for (int l = 0; l < m->nlin; l++) {
@@ -765,11 +1146,12 @@ int transpose_weights(bsim_mlp *m)
         a.k[l] = m->kdim[l];
         a.first[l + 1] = a.first[l] + (a.n[l] / 64) * (a.k[l] / 64);
     }
+    a.p = m->p;
     a.w = m->pbf;
     a.wt = m->pbf_t;
     (void)hipGetLastError();   /* the check after the launch reports it alone */
-    hipLaunchKernelGGL(mlp_transpose_w, dim3(a.first[m->nlin]), dim3(256), 0, m->stream, a);
-    return hip_check(hipGetLastError(), "transpose launch");
+    hipLaunchKernelGGL(mlp_pack, dim3(a.first[m->nlin]), dim3(256), 0, m->stream, a);
+    return hip_check(hipGetLastError(), "pack launch");
 }
 
 int check_batch(const bsim_mlp *m, int32_t batch)
@@ -834,20 +1216,19 @@ bsim_mlp *bsim_mlp_create(const bsim_mlp_config *cfg)
     if (!rc) rc = dalloc(m, &m->grad, m->nparam);
     if (!rc) rc = dalloc(m, &m->pbf, m->nparam);
     if (!rc) rc = dalloc(m, &m->pbf_t, m->nparam);
-    for (int l = 0; l < m->nlin && !rc; l++) rc = dalloc(m, &m->act[l], B * m->kdim[l]);
+    for (int l = 0; l < m->nlin && !rc && !chained(m); l++) rc = dalloc(m, &m->act[l], B * m->kdim[l]);
     if (!rc) rc = dalloc(m, &m->out, B * m->kdim[m->nlin]);
     if (!rc) rc = dalloc(m, &m->ybat, B * c.out_dim);
     int32_t wmax = 0;
     for (int l = 0; l <= m->nlin; l++) wmax = std::max(wmax, m->kdim[l]);
-    if (!rc) rc = dalloc(m, &m->dz[0], B * wmax);
-    if (!rc) rc = dalloc(m, &m->dz[1], B * wmax);
+    if (!rc && !chained(m)) rc = dalloc(m, &m->dz[0], B * wmax);
+    if (!rc && !chained(m)) rc = dalloc(m, &m->dz[1], B * wmax);
     for (int l = 0; l < m->nlin && !rc; l++) rc = dalloc(m, &m->act_t[l], B * m->kdim[l]);
     for (int l = 0; l < m->nlin && !rc; l++) {
-        rc = dalloc(m, &m->wpart[l], (int64_t)KSPLIT * m->kdim[l + 1] * m->kdim[l]);
-        if (!rc) rc = dalloc(m, &m->bpart[l], B / ROWS_PER_PART * m->kdim[l + 1]);
+        rc = dalloc(m, &m->bpart[l], B / ROWS_PER_PART * m->kdim[l + 1]);
         if (!rc) rc = dalloc(m, &m->dzt[l], B * m->kdim[l + 1]);
     }
-    if (!rc) rc = dalloc(m, &m->lpart, B / ROWS_PER_PART * (m->kdim[m->nlin] / 64));
+    if (!rc) rc = dalloc(m, &m->lpart, B / BM * (m->kdim[m->nlin] / BN) * 4);
     if (!rc) rc = dalloc(m, &m->loss, 1);
     if (!rc) rc = dalloc(m, &m->xstage, B * c.in_dim);
     if (rc != BSIM_OK) return bad(0);
@@ -909,11 +1290,8 @@ int bsim_mlp_set_params(bsim_mlp *m, const float *in)
             if (r >= nrow) p[m->boff[l] + r] = 0.f;
         }
     }
-    std::vector<uint16_t> pb(m->nparam);
-    for (int64_t i = 0; i < m->nparam; i++) pb[i] = f2bf(p[i]);
     int rc = hip_check(hipMemcpy(m->p, p.data(), m->nparam * 4, hipMemcpyHostToDevice), "hipMemcpy");
-    if (!rc) rc = hip_check(hipMemcpy(m->pbf, pb.data(), m->nparam * 2, hipMemcpyHostToDevice), "hipMemcpy");
-    if (!rc) rc = transpose_weights(m);
+    if (!rc) rc = pack_weights(m);
     if (!rc) rc = hip_check(hipStreamSynchronize(m->stream), "sync");
     if (!rc) rc = hip_check(hipMemset(m->m, 0, m->nparam * 4), "hipMemset");
     if (!rc) rc = hip_check(hipMemset(m->v, 0, m->nparam * 4), "hipMemset");
@@ -971,9 +1349,10 @@ int train_steps(bsim_mlp *m, const int32_t *rdev, float *ldev, int32_t steps, in
     int rc = BSIM_OK;
     for (int32_t s = 0; s < steps && !rc; s++) {
         /* the minibatch is gathered by the first layer's GEMM and the loss */
-        rc = forward(m, batch, true, rdev + (int64_t)s * batch);
-        if (!rc) rc = backward(m, batch);
-        if (!rc) rc = adam(m, batch, true, lr, nullptr, ldev + s);   /* writes W^T too */
+        const int32_t *rows = rdev + (int64_t)s * batch;
+        rc = chained(m) ? chain(m, batch, true, rows, 0) : forward(m, batch, true, rows);
+        if (!rc && !chained(m)) rc = backward(m, batch);
+        if (!rc) rc = update(m, batch, true, lr, nullptr, ldev + s);
     }
     const int src = hip_check(hipStreamSynchronize(m->stream), "sync");
     return rc ? rc : src;
@@ -1069,14 +1448,18 @@ int bsim_mlp_gradients(bsim_mlp *m, const float *x, const float *y, int32_t batc
     if (!rc) rc = hip_check(hipMemcpyAsync(m->ybat, y, (size_t)batch * m->cfg.out_dim * 4,
                                            hipMemcpyHostToDevice, m->stream), "hipMemcpyAsync");
     if (rc) return rc;
-    const int64_t tot = (int64_t)batch * kin;
-    (void)hipGetLastError();   /* the check after the launch reports it alone */
-    hipLaunchKernelGGL(mlp_convert_x, dim3((uint32_t)((tot + 255) / 256)), dim3(256), 0, m->stream,
-                       m->xstage, m->act[0], m->act_t[0], (int64_t)batch, din, kin);
-    rc = hip_check(hipGetLastError(), "convert launch");
-    if (!rc) rc = forward(m, batch, true);
-    if (!rc) rc = backward(m, batch);
-    if (!rc) rc = adam(m, batch, false, 0.f, m->grad, m->loss);
+    if (chained(m)) {
+        rc = chain(m, batch, true, nullptr, batch);
+    } else {
+        const int64_t tot = (int64_t)batch * kin;
+        (void)hipGetLastError();   /* the check after the launch reports it alone */
+        hipLaunchKernelGGL(mlp_convert_x, dim3((uint32_t)((tot + 255) / 256)), dim3(256), 0, m->stream,
+                           m->xstage, m->act[0], m->act_t[0], (int64_t)batch, (int64_t)batch, din, kin);
+        rc = hip_check(hipGetLastError(), "convert launch");
+        if (!rc) rc = forward(m, batch, true);
+        if (!rc) rc = backward(m, batch);
+    }
+    if (!rc) rc = update(m, batch, false, 0.f, m->grad, m->loss);
     if (!rc) rc = hip_check(hipStreamSynchronize(m->stream), "sync");
     if (!rc) rc = hip_check(hipMemcpy(grad, m->grad, m->nparam * 4, hipMemcpyDeviceToHost), "hipMemcpy");
     if (!rc) rc = hip_check(hipMemcpy(loss, m->loss, 4, hipMemcpyDeviceToHost), "hipMemcpy");
@@ -1094,17 +1477,20 @@ int bsim_mlp_predict(bsim_mlp *m, const float *x, int64_t n, float *y)
     for (int64_t r0 = 0; r0 < n && !rc; r0 += B) {
         const int64_t rows = std::min<int64_t>(B, n - r0);
         const int32_t batch = (int32_t)round_up(rows, 64);
-        rc = hip_check(hipMemsetAsync(m->xstage, 0, (size_t)batch * din * 4, m->stream), "memset");
-        if (!rc) rc = hip_check(hipMemcpyAsync(m->xstage, x + r0 * din, (size_t)rows * din * 4,
-                                               hipMemcpyHostToDevice, m->stream), "hipMemcpyAsync");
+        rc = hip_check(hipMemcpyAsync(m->xstage, x + r0 * din, (size_t)rows * din * 4,
+                                      hipMemcpyHostToDevice, m->stream), "hipMemcpyAsync");
         if (rc) break;
-        const int64_t tot = (int64_t)batch * kin;
-        (void)hipGetLastError();   /* the check after the launch reports it alone */
-        hipLaunchKernelGGL(mlp_convert_x, dim3((uint32_t)((tot + 255) / 256)), dim3(256), 0,
-                           m->stream, m->xstage, m->act[0], (uint16_t *)nullptr, (int64_t)batch,
-                           din, kin);
-        rc = hip_check(hipGetLastError(), "convert launch");
-        if (!rc) rc = forward(m, batch, false);
+        if (chained(m)) {
+            rc = chain(m, (int32_t)round_up(rows, CH_ROWS), false, nullptr, rows);
+        } else {
+            const int64_t tot = (int64_t)batch * kin;
+            (void)hipGetLastError();   /* the check after the launch reports it alone */
+            hipLaunchKernelGGL(mlp_convert_x, dim3((uint32_t)((tot + 255) / 256)), dim3(256), 0,
+                               m->stream, m->xstage, m->act[0], (uint16_t *)nullptr, (int64_t)batch, rows,
+                               din, kin);
+            rc = hip_check(hipGetLastError(), "convert launch");
+            if (!rc) rc = forward(m, batch, false);
+        }
         if (rc) break;
         tmp.resize((size_t)rows * nout);
         rc = hip_check(hipMemcpyAsync(tmp.data(), m->out, (size_t)rows * nout * 4,
