@@ -49,7 +49,7 @@ def test_chained_equals_layered(in_dim, hidden, layers, out_dim, batch):
     m.set_params(p)
     p = m.get_params()                          # with the padding cleared
     v.set_params(widen(p, narrow, wide, total))
-    for rows in (1, 31, 32, 33, batch, 2 * batch + 65):
+    for rows in (0, 1, 31, 32, 33, batch, 2 * batch + 65, 4000):
         x = rng.normal(size=(rows, in_dim)).astype(np.float32)
         np.testing.assert_array_equal(m.predict(x), v.predict(x))
     x = rng.normal(size=(batch, in_dim)).astype(np.float32)
