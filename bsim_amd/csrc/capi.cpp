@@ -331,9 +331,10 @@ extern "C" {
  * slowly against 2 cycles); bsim_sim_set_schedule changes it. */
 static const int32_t kRankEvery = 2;
 
-/* Step workgroups that run at a time: two per compute unit.  Up to as many
- * units start at once, and their order is nothing. */
-static const int32_t kResident = 512;
+/* Units from which on their order counts: with more than one to a compute unit,
+ * heavy ones should start first and not share one.  us per cycle of 396 units,
+ * 110,000 neurons with delays up to 50 steps: in order 1,010, ranked 877. */
+static const int32_t kRanked = 256;
 
 static int32_t check_config(const bsim_sim_config &c, int32_t N, const char *who)
 {
@@ -497,19 +498,17 @@ static bsim_sim *sim_from_layout(bsim::Layout &L, const bsim_sim_config &c, bsim
     UP(bern_seed, L.bern_seed);
     UP(bern_key, L.bern_key);
     UP(pois_tab, L.pois_tab);
-    d.nslots = L.nslots * L.parts;
-    d.rank_wgs = d.nslots > kResident ? 8 : 0;
+    /* slot s runs on XCD s % 8: an eighth of the units each, in order */
+    d.nslots = (d.ntiles + 7) / 8 * 8;
+    d.rank_wgs = d.ntiles > kRanked ? 8 : 0;
     {
-        /* the units of each residue in order (until the first ranking) */
         std::vector<bsim_unit> unit((size_t)(d.rank_wgs ? d.ntiles : d.nslots));
-        std::vector<uint8_t> res((size_t)d.ntiles);
         std::vector<int32_t> used(8, 0);
         for (auto &x : unit) x.id = -1;
         perm.assign((size_t)std::max(d.nslots, 1), -1);
         for (int32_t u = 0; u < d.ntiles; u++) {
-            const int32_t t = u / L.parts;
-            res[u] = L.tile_res[t];
-            const int32_t slot = 8 * used[res[u]]++ + res[u];
+            const int32_t t = u / L.parts, x8 = (int32_t)(8ll * u / d.ntiles);
+            const int32_t slot = 8 * used[x8]++ + x8;
             perm[(size_t)slot] = u;
             bsim_unit &x = unit[(size_t)(d.rank_wgs ? u : slot)];
             x.base = L.tile_base[t];
@@ -525,7 +524,6 @@ static bsim_sim *sim_from_layout(bsim::Layout &L, const bsim_sim_config &c, bsim
             }
         }
         UP(unit, unit);
-        UP(tile_res, res);
     }
     {
         /* an event thread takes two rows at a time where a unit has many rows

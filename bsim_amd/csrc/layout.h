@@ -145,10 +145,9 @@ typedef struct bsim_dev {
     int32_t *fire_count;
     uint64_t *hist;             /* [2][n] by cycle parity */
     /* synapses */
-    int32_t nslots;             /* step workgroups (units placed by XCD residue) */
+    int32_t nslots;             /* step workgroups: the units, and empty slots to a multiple of 8 */
     int32_t wrows;              /* rows that an event thread takes at a time, 1 or 2 */
-    const bsim_unit *unit;      /* [ntiles], or [nslots] in slot order where every unit has a workgroup */
-    const uint8_t *tile_res;    /* [ntiles] XCD residue of the unit's group */
+    const bsim_unit *unit;      /* [ntiles], or without ranking [nslots] in slot order */
     const bsim_syn *syn;        /* [S] target and weight of each synapse, group-major */
     const bsim_range *rng;
     const uint32_t *off_tab;    /* group row tables */
@@ -168,8 +167,8 @@ typedef struct bsim_dev {
     uint64_t *tile_load;        /* [2][ntiles] work of a launch before a ranking (x 16), by cycle parity */
     int32_t rank_every;         /* units ranked heaviest first every this many cycles (0: never,
                                    the units stay in their initial order) */
-    int32_t rank_wgs;           /* workgroups before the others (the first ranks): 8, or 0 where every
-                                   unit has a workgroup and order is nothing */
+    int32_t rank_wgs;           /* workgroups before the slots' (the first ranks): 8, or 0 where the
+                                   units run in their initial order */
     uint8_t *tile_cls;          /* [ntiles] half-octave class of a unit's work */
     uint64_t *raster;           /* [rec_steps][nwords] fired bitmaps, or NULL */
     int32_t rec_steps;

@@ -14,9 +14,9 @@
  *        ballot) and active (pre, delay) rows, the list that the next launch's
  *        units read.
  *
- * One more workgroup orders the units for the launches to come, heaviest
- * first, by the work that the launch before recorded, where they are more than
- * run at a time.
+ * Where a compute unit has more than one unit, one more workgroup orders them
+ * for the launches to come, by the work that the launch before recorded
+ * (rank_units).
  *
  * A unit finds its active rows from the lists of the blocks of 64 pres that its
  * source chunks cover.  A second launch per cycle, which merged them into one
@@ -711,24 +711,25 @@ __device__ __forceinline__ void count_done(const bsim_dev &d)
                                  __HIP_MEMORY_SCOPE_AGENT);
 }
 
-/* Orders the units by their work in the launch before, heaviest first, so that
- * the hardware dispatches the heavy units of the coming launches before the
- * light ones (results do not depend on the order; the firing volleys move
- * slowly against two cycles).  Units of one group share lines of the row
- * table and stay on one XCD while these have about the same work.  Where one
- * has more than SPREAD_MIN times the mean, the units are dealt out to the XCDs
- * in turn, unless the table has an entry per synapse or more (rows taken two
- * at a time): lines that every XCD reads then cost more than the imbalance.
- * us per cycle by group / dealt out: 330,000 neurons at ~100 Hz 59.9 / 54.4,
- * 650,000 108.2 / 101.2, where volleys pass through the populations at
- * different times; a balanced sweep of 96 chains 27.6 / 27.9, 110,000 neurons
- * with delays up to 50 steps 941 / 1,002 to 1,046.
- * Counting sort over half-octave classes; within a class the order is
- * arbitrary.  Runs in one workgroup, beside the others of the launch, and
- * clears the loads that it has read.  The classes of the units are kept in LDS
- * where they fit. */
-#define SPREAD_MIN 1.125f
+/* Orders the units for the coming launches by their work in the launch before
+ * (results do not depend on the order; the firing volleys move slowly against
+ * two cycles).  The hardware deals the workgroups out to the XCDs in turn, slot s
+ * to XCD s % 8, and starts an XCD's in order.  The units are cut, in index order,
+ * into eight runs of equal cost, one per XCD: units of a group, which read the
+ * same rows at the same time, so share an L2.  Within an XCD the heavy units come
+ * first, by half-octave classes (counting sort; within a class the order is
+ * arbitrary).  An XCD has slots for an eighth of the units; the lightest of a
+ * longer run fill what others leave free, so that no XCD starts more workgroups
+ * than another.  us per cycle with whole groups on XCDs / with the units dealt
+ * out in turn where those were uneven / with runs: 330,000 neurons at ~100 Hz
+ * 59.9 / 54.5 / 55.0, 650,000 108 / 101 / 98.9, 110,000 with delays up to 50
+ * steps 950 / 1,046 / 877, a sweep of 96 chains 27.6 / 27.9 / 27.1, the same in
+ * units of half the size 21.7 / 21.9 / 21.2.  Twice the slots, so that runs stay
+ * whole: 59.5, 110, 875, 26.9, 22.9 (XCDs with few heavy units start more).
+ * Runs in one workgroup, beside the others of the launch, and clears the loads
+ * that it has read.  The classes of the units are kept in LDS where they fit. */
 #define RANK_CLASSES 64
+#define RANK_FIXED 8192ull
 
 __device__ __forceinline__ uint32_t load_class(uint64_t x)
 {
@@ -738,65 +739,84 @@ __device__ __forceinline__ uint32_t load_class(uint64_t x)
     return min(2u * (e - 4u) + h + 1u, (uint32_t)RANK_CLASSES - 1u);
 }
 
-/* a class's work, as a multiple of the lightest's */
-__device__ __forceinline__ float class_work(uint32_t c)
+/* The cost of a unit of class c: its work, and that of a workgroup that finds
+ * next to nothing to deliver. */
+__device__ __forceinline__ uint64_t class_cost(uint32_t c)
 {
-    return c == 0 ? 0.5f : ldexpf((c - 1u) & 1u ? 1.5f : 1.0f, (int)((c - 1u) / 2u));
+    return RANK_FIXED + (c == 0 ? 0ull : (2ull + ((c - 1u) & 1u)) << ((c - 1u) / 2u + 3u));
 }
 
 __device__ void rank_units(const bsim_dev &d, uint64_t *load, int32_t *perm, uint32_t *lds, uint32_t lds_size)
 {
-    uint32_t *cnt = lds, *fill = cnt + NRES * RANK_CLASSES, *rtot = fill + NRES * RANK_CLASSES;
-    float *work = reinterpret_cast<float *>(rtot + NRES);
-    uint8_t *cls = (uint32_t)d.ntiles <= lds_size - 4u * (2 * NRES * RANK_CLASSES + 2 * NRES)
-                       ? reinterpret_cast<uint8_t *>(work + NRES) : d.tile_cls;
+    uint64_t *sum = reinterpret_cast<uint64_t *>(lds);              /* [NTHREAD] */
+    uint32_t *cnt = reinterpret_cast<uint32_t *>(sum + NTHREAD), *fill = cnt + NRES * RANK_CLASSES;
+    uint32_t *rtot = fill + NRES * RANK_CLASSES;                    /* [NRES] */
+    uint8_t *cls = (uint32_t)d.ntiles <= lds_size - (8u * NTHREAD + 4u * (2 * NRES * RANK_CLASSES + NRES))
+                       ? reinterpret_cast<uint8_t *>(rtot + NRES) : d.tile_cls;
     static_assert(RANK_CLASSES == WAVE && NRES * RANK_CLASSES <= NTHREAD, "a wavefront per residue, a lane per class");
-    const uint32_t tid = threadIdx.x, x = tid / RANK_CLASSES, c = RANK_CLASSES - 1u - tid % RANK_CLASSES;
+    const uint32_t tid = threadIdx.x;
     const bool counts = tid < NRES * RANK_CLASSES;
     if (counts) cnt[tid] = 0u;
-    __syncthreads();
-    for (int32_t k = tid; k < d.ntiles; k += NTHREAD) {
+    /* thread: units k0 .. k1 - 1 */
+    const int32_t per = (d.ntiles + NTHREAD - 1) / NTHREAD;
+    const int32_t k0 = min((int32_t)tid * per, d.ntiles), k1 = min(k0 + per, d.ntiles);
+    uint64_t mine = 0;
+    for (int32_t k = k0; k < k1; k++) {
         const uint32_t c = load_class(load[k]);
         load[k] = 0ull;
         cls[k] = (uint8_t)c;
-        atomicAdd(&cnt[d.tile_res[k] * RANK_CLASSES + c], 1u);
+        mine += class_cost(c);
     }
-    __syncthreads();
-    if (counts) {
-        float s = (float)cnt[x * RANK_CLASSES + c] * class_work(c);
-        for (int m = 1; m < WAVE; m *= 2) s += __shfl_xor(s, m);
-        if (c == 0) work[x] = s;
-    }
-    __syncthreads();
-    float all = 0.0f, most = 0.0f;
-    for (int i = 0; i < NRES; i++) {
-        all += work[i];
-        most = fmaxf(most, work[i]);
-    }
-    const bool spread = d.wrows == 1 && most * NRES > all * SPREAD_MIN;
-    if (spread) {                                   /* count again, by the residues dealt out */
-        if (counts) cnt[tid] = 0u;
+    uint64_t upto = mine;
+    for (uint32_t o = 1; o < NTHREAD; o <<= 1) {
+        sum[tid] = upto;
         __syncthreads();
-        for (int32_t k = tid; k < d.ntiles; k += NTHREAD)
-            atomicAdd(&cnt[(uint32_t)k % NRES * RANK_CLASSES + cls[k]], 1u);
+        if (tid >= o) upto += sum[tid - o];
         __syncthreads();
     }
+    sum[tid] = upto;
+    __syncthreads();
+    const double part = (double)NRES / (double)sum[NTHREAD - 1];
+    auto residue = [&](uint64_t before) { return min((uint32_t)((double)before * part), (uint32_t)NRES - 1u); };
+    uint64_t at = upto - mine;
+    for (int32_t k = k0; k < k1; k++) {
+        const uint32_t c = cls[k];
+        atomicAdd(&cnt[residue(at) * RANK_CLASSES + c], 1u);
+        at += class_cost(c);
+    }
+    __syncthreads();
     /* exclusive prefix of each residue's class counts, heaviest class first */
     if (counts) {
+        const uint32_t x = tid / RANK_CLASSES, c = RANK_CLASSES - 1u - tid % RANK_CLASSES;
         const uint32_t v = cnt[x * RANK_CLASSES + c], incl = wave_incl_scan(v);
         fill[x * RANK_CLASSES + c] = incl - v;
         if (c == 0) rtot[x] = incl;
     }
     __syncthreads();
     /* unit of residue x at rank i goes to slot NRES * i + x */
-    for (int32_t k = tid; k < d.ntiles; k += NTHREAD) {
-        const uint32_t x = spread ? (uint32_t)k % NRES : d.tile_res[k];
-        const uint32_t pos = atomicAdd(&fill[x * RANK_CLASSES + cls[k]], 1u);
+    const uint32_t cap = (uint32_t)d.nslots / NRES;
+    at = upto - mine;
+    for (int32_t k = k0; k < k1; k++) {
+        const uint32_t c = cls[k];
+        uint32_t x = residue(at), pos = atomicAdd(&fill[x * RANK_CLASSES + c], 1u);
+        at += class_cost(c);
+        if (pos >= cap) {                           /* the n-th unit without a slot */
+            uint32_t n = pos - cap;
+            for (uint32_t y = 0; y < x; y++) n += max(rtot[y], cap) - cap;
+            for (x = 0; n >= cap - min(rtot[x], cap); x++) n -= cap - min(rtot[x], cap);
+            pos = rtot[x] + n;
+        }
         perm[NRES * pos + x] = k;
     }
-    /* the remaining slots of each residue are empty */
+    /* the remaining slots are empty */
+    uint32_t over = 0;
+    for (uint32_t y = 0; y < NRES; y++) over += max(rtot[y], cap) - cap;
     for (int32_t i = tid; i < d.nslots; i += NTHREAD) {
-        if (i / NRES >= (int32_t)rtot[i % NRES]) perm[i] = -1;
+        const uint32_t x = (uint32_t)i % NRES, pos = (uint32_t)i / NRES;
+        if (pos < rtot[x]) continue;
+        uint32_t n = pos - rtot[x];                 /* free slots before this one */
+        for (uint32_t y = 0; y < x; y++) n += cap - min(rtot[y], cap);
+        if (n >= over) perm[i] = -1;
     }
 }
 
