@@ -17,7 +17,7 @@
 #include "internal.h"
 #include "network.h"
 
-extern "C" hipError_t bsim_launch_step(const bsim_dev *d, int32_t t, int32_t flags,
+extern "C" hipError_t bsim_launch_step(const bsim_dev *d, int32_t t, int32_t flags, int32_t cycles,
                                        hipStream_t stream);
 
 thread_local std::string g_bsim_err;
@@ -478,7 +478,7 @@ static bsim_sim *sim_from_layout(bsim::Layout &L, const bsim_sim_config &c, bsim
     sim->tile = L.tile;
     sim->ntiles = L.ntiles;
     d.tile = L.tile / L.parts;
-    d.ntiles = L.ntiles * L.parts;
+    d.ntiles = (int32_t)(((int64_t)L.n + d.tile - 1) / d.tile);     /* those that have neurons */
     d.dmax = L.dmax;
     d.nwords = (L.n + 63) / 64;
     sim->s = L.s;
@@ -638,7 +638,7 @@ static hipError_t build_graph(bsim_sim *sim)
     if (e != hipSuccess) return e;
     hipError_t le = hipSuccess;
     for (int32_t i = 0; i < kGraphCycles && le == hipSuccess; i++) {
-        le = bsim_launch_step(&sim->d, -1, 0, sim->stream);
+        le = bsim_launch_step(&sim->d, -1, 0, 1, sim->stream);
     }
     hipGraph_t g = nullptr;
     e = hipStreamEndCapture(sim->stream, &g);
@@ -666,6 +666,14 @@ int32_t bsim_sim_step(bsim_sim *sim, int32_t n)
     if ((int64_t)sim->cycle + n > 0x7FFFFFFF) return fail(BSIM_E_ARG, "bsim_sim_step: cycle overflow");
     if (int32_t rc = use_device(sim)) return rc;
     hipError_t e = hipSuccess;
+    while (sim->d.ntiles == 1 && n > 0) {
+        /* one workgroup: many cycles per launch */
+        const int32_t c = std::min(n, kGraphCycles);
+        e = bsim_launch_step(&sim->d, -1, 0, c, sim->stream);
+        if (e != hipSuccess) return fail(BSIM_E_HIP, std::string("step launch: ") + hipGetErrorString(e));
+        sim->cycle += c;
+        n -= c;
+    }
     if (n >= kGraphCycles && !sim->gexec) {
         e = build_graph(sim);
         if (e != hipSuccess) return fail(BSIM_E_HIP, std::string("step graph: ") + hipGetErrorString(e));
@@ -677,7 +685,7 @@ int32_t bsim_sim_step(bsim_sim *sim, int32_t n)
         n -= kGraphCycles;
     }
     for (; n > 0; n--) {
-        e = bsim_launch_step(&sim->d, -1, 0, sim->stream);
+        e = bsim_launch_step(&sim->d, -1, 0, 1, sim->stream);
         if (e != hipSuccess) return fail(BSIM_E_HIP, std::string("step launch: ") + hipGetErrorString(e));
         sim->cycle++;
     }
@@ -693,7 +701,7 @@ int32_t bsim_sim_time_steps(bsim_sim *sim, int32_t n, double *step_us, double *r
     for (size_t i = 0; i < ev.size() && e == hipSuccess; i++) e = hipEventCreate(&ev[i]);
     for (int32_t i = 0; i < n && e == hipSuccess; i++) {
         e = hipEventRecord(ev[2 * i], sim->stream);
-        if (e == hipSuccess) e = bsim_launch_step(&sim->d, -1, 0, sim->stream);
+        if (e == hipSuccess) e = bsim_launch_step(&sim->d, -1, 0, 1, sim->stream);
         if (e == hipSuccess) e = hipEventRecord(ev[2 * i + 1], sim->stream);
         if (e == hipSuccess) sim->cycle++;
     }
@@ -721,7 +729,7 @@ int32_t bsim_sim_finish(bsim_sim *sim)
     d.ev_count = sim->ev_fin;
     hipError_t e = hipMemsetAsync(sim->ev_fin, 0, (size_t)(d.ntiles > 0 ? d.ntiles : 1) * 8, sim->stream);
     if (e != hipSuccess) return fail(BSIM_E_HIP, std::string("finish: ") + hipGetErrorString(e));
-    e = bsim_launch_step(&d, sim->cycle, 1, sim->stream);
+    e = bsim_launch_step(&d, sim->cycle, 1, 1, sim->stream);
     if (e != hipSuccess) return fail(BSIM_E_HIP, std::string("finish launch: ") + hipGetErrorString(e));
     sim->finished_at = sim->cycle;
     return 0;

@@ -145,8 +145,13 @@ int32_t default_parts(int64_t n, int32_t tile)
      * 1950 tiles 52 / 84; TILE 192, 78 tiles 13.8 / 12.0, 169 tiles 16.1 / 19.9.
      * So: always from TILE 576 up (a whole tile is three or more targets per
      * owner thread), below that while the parts leave no more than about one
-     * workgroup per compute unit and 192 targets of the tile. */
+     * workgroup per compute unit and 192 targets of the tile.  A network that is one
+     * unit runs many cycles per launch, so a single tile stays whole where it
+     * is at most a target per owner thread: 180 neurons in runs 4.6 / 2.8, in
+     * launches of one cycle 7.2 / 7.7; of 384 targets (370 neurons) 5.9 / 5.2 and
+     * 8.3 / 10.4, so not there. */
     const int64_t tiles = (n + tile - 1) / tile;
+    if (n <= tile && tile <= 256 && BSIM_NWAVE * n > tile) return 1;
     return tile >= 3 * BSIM_TILE_ALIGN || BSIM_NWAVE * tiles <= 256 * (tile / BSIM_TILE_ALIGN) ? BSIM_NWAVE : 1;
 }
 

@@ -704,10 +704,10 @@ __device__ __forceinline__ void load_params(const bsim_dev &d, NState<S_> &ns)
         ns.c[j] = d.lifc[ns.cls[j] >> 30 == BSIM_KIND_LIF ? ns.cls[j] & BSIM_CLS_SET_MASK : 0u];
 }
 
-/* This workgroup of a clocked launch has ended (see device_cycle). */
-__device__ __forceinline__ void count_done(const bsim_dev &d)
+/* This workgroup of a clocked launch has ended its cycles (see device_cycle). */
+__device__ __forceinline__ void count_done(const bsim_dev &d, uint64_t cycles)
 {
-    (void)__hip_atomic_fetch_add(d.done + BSIM_DONE_STRIDE * (blockIdx.x % 8u), (uint64_t)1, __ATOMIC_RELAXED,
+    (void)__hip_atomic_fetch_add(d.done + BSIM_DONE_STRIDE * (blockIdx.x % 8u), cycles, __ATOMIC_RELAXED,
                                  __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -960,13 +960,12 @@ __device__ __forceinline__ uint32_t batch_rows(const Shared &S, int32_t nrb, uin
 /* Event wavefronts: the unit of record k (below 0: none). */
 template <int NB, int WR>
 __device__ __forceinline__ void event_unit(const Shared &S, int32_t k, int32_t t, bool deliver, bool clocked,
-                                           uint32_t U, uint32_t K)
+                                           uint32_t U, uint32_t K, uint32_t &par, uint32_t &nb)
 {
     const bsim_dev &d = args_again();
     const bsim_unit *un = d.unit + (k < 0 ? 0 : k);
     const int32_t id = k < 0 ? -1 : un->id, list = (t - 1) & 1;
     const int32_t nrng = deliver && id >= 0 ? un->nrng : 0;
-    uint32_t par = 0, nb = 0;                   /* passes and batches so far, modulo 2 */
     uint32_t events = 0, rows = 0;
     for (int32_t rb = 0; rb < nrng; rb += MAXR) {
         const int32_t nrb = min(MAXR, nrng - rb);
@@ -994,7 +993,7 @@ __device__ __forceinline__ void event_unit(const Shared &S, int32_t k, int32_t t
 /* Owner wavefronts: the same unit's sums and update. */
 template <int S_>
 __device__ __forceinline__ void owner_unit(const Shared &S, int32_t k, int32_t t, bool deliver, bool update,
-                                           uint32_t U, uint32_t K)
+                                           uint32_t U, uint32_t K, uint32_t &par, uint32_t &nb)
 {
     constexpr bool PRE = S_ <= PREFETCH_MAX_S;
     const bsim_dev &d = args_again();
@@ -1015,7 +1014,6 @@ __device__ __forceinline__ void owner_unit(const Shared &S, int32_t k, int32_t t
             load_params<S_>(d, ns);
         }
     }
-    uint32_t par = 0, nb = 0;                   /* passes and batches so far, modulo 2 */
     for (int32_t rb = 0; rb < nrng; rb += MAXR) {
         wg_barrier();
         Rows R;
@@ -1026,8 +1024,10 @@ __device__ __forceinline__ void owner_unit(const Shared &S, int32_t k, int32_t t
     if (upd) update_unit<S_, PRE>(id, t, U, acc, ns);
 }
 
-template <int NB, int WR, int S_>
-__global__ __launch_bounds__(NTHREAD, STEP_EU) void bsim_step_kernel(bsim_dev d, int32_t t, int32_t flags)
+/* ONE: the grid's one unit, cycles cycles from the clock's on; otherwise one cycle. */
+template <int NB, int WR, int S_, bool ONE>
+__global__ __launch_bounds__(NTHREAD, STEP_EU) void bsim_step_kernel(bsim_dev d, int32_t t, int32_t flags,
+                                                                     int32_t cycles)
 {
     extern __shared__ __align__(16) uint32_t lds[];
     const bool clocked = t < 0;
@@ -1044,7 +1044,7 @@ __global__ __launch_bounds__(NTHREAD, STEP_EU) void bsim_step_kernel(bsim_dev d,
                 rank_units(d, d.tile_load + (int64_t)((t - 1) & 1) * d.ntiles,
                            d.perm + (int64_t)((t / re) & 1) * d.nslots, lds, (uint32_t)lds_bytes((uint32_t)d.tile));
             wg_barrier();
-            if (threadIdx.x == 0) count_done(d);
+            if (threadIdx.x == 0) count_done(d, 1u);
         }
         return;
     }
@@ -1069,43 +1069,69 @@ __global__ __launch_bounds__(NTHREAD, STEP_EU) void bsim_step_kernel(bsim_dev d,
     }
 
     const bool deliver = (flags & 1) != 0, update = (flags & 2) != 0;
-    if (deliver) {
+    if (deliver || ONE) {
         for (uint32_t i = tid; i < 2 * U; i += NTHREAD)
             reinterpret_cast<uint4 *>(S.hist)[i] = make_uint4(0u, 0u, 0u, 0u);
         for (uint32_t i = tid; i < 2 * PASS; i += NTHREAD) S.mark[i] = NO_MARK;
         if (w < NEV) S.blk_mark[tid] = NO_MARK;
         if (tid < 4) S.most[tid] = 0u;          /* most and last */
     }
+    uint32_t par = 0, nb = 0;       /* passes and batches so far, modulo 2 */
+    if (ONE && clocked) {
+        /* what the owner wavefronts write in a cycle, this workgroup's event
+         * wavefronts read in the next: a barrier in between orders that */
+        if (w < NEV) {
+            for (int32_t c = 0; c < cycles; c++, t++) {
+                event_unit<NB, WR>(S, k, t, t > 0, true, U, K, par, nb);
+                wg_barrier();
+            }
+        } else {
+            for (int32_t c = 0; c < cycles; c++, t++) {
+                owner_unit<S_>(S, k, t, t > 0, true, U, K, par, nb);
+                wg_barrier();
+            }
+        }
+        if (tid == 0) count_done(d, (uint64_t)cycles);
+        return;
+    }
     if (w < NEV)
-        event_unit<NB, WR>(S, k, t, deliver, clocked, U, K);
+        event_unit<NB, WR>(S, k, t, deliver, clocked, U, K, par, nb);
     else
-        owner_unit<S_>(S, k, t, deliver, update, U, K);
+        owner_unit<S_>(S, k, t, deliver, update, U, K, par, nb);
     if (clocked) wg_barrier();      /* every wavefront has read the cycle */
-    if (clocked && tid == 0) count_done(d);
+    if (clocked && tid == 0) count_done(d, 1u);
 }
 
-extern "C" hipError_t bsim_launch_step(const bsim_dev *d, int32_t t, int32_t flags,
+/* One cycle, or with one unit (d.nslots 8, the others empty) and clocked as many
+ * as cycles says: the launch and what a workgroup reads at its start are over
+ * half of a small network's cycle.  us per cycle in runs, a launch each / 64 cycles a
+ * launch: 48 neurons 5.1 / 3.0, 180 4.6 / 2.8, 250 with delays up to 30 steps 6.3
+ * / 4.1. */
+extern "C" hipError_t bsim_launch_step(const bsim_dev *d, int32_t t, int32_t flags, int32_t cycles,
                                        hipStream_t stream)
 {
     if (d->ntiles <= 0) return hipSuccess;
     const uint32_t U = (uint32_t)d->tile;
     if (U == 0 || U % WAVE != 0 || U > BSIM_MAX_UNIT) return hipErrorInvalidValue;
+    if (cycles != 1 && (t >= 0 || d->ntiles != 1)) return hipErrorInvalidValue;
     const dim3 grid(d->nslots + d->rank_wgs), block(NTHREAD);
     const size_t lds = lds_bytes(U);
     (void)hipGetLastError();       /* the check below then reports this launch alone */
 #define OWN(X) (((X) + NOWN * WAVE - 1) / (NOWN * WAVE))
-#define STEP(NB, X)                                                                                       \
-    do {                                                                                                  \
-        if (d->wrows == 2)                                                                                \
-            hipLaunchKernelGGL((bsim_step_kernel<NB, 2, OWN(X)>), grid, block, lds, stream, *d, t, flags); \
-        else                                                                                              \
-            hipLaunchKernelGGL((bsim_step_kernel<NB, 1, OWN(X)>), grid, block, lds, stream, *d, t, flags); \
+#define LAUNCH(NB, WR, X, ONE) \
+    hipLaunchKernelGGL((bsim_step_kernel<NB, WR, OWN(X), ONE>), grid, block, lds, stream, *d, t, flags, cycles)
+#define STEP(NB, X)                                    \
+    do {                                               \
+        if (d->ntiles == 1) LAUNCH(NB, 1, X, true);    \
+        else if (d->wrows == 2) LAUNCH(NB, 2, X, false); \
+        else LAUNCH(NB, 1, X, false);                  \
     } while (0)
     if (U <= 64) STEP(6, 64);
     else if (U <= 128) STEP(7, 128);
     else if (U <= 256) STEP(8, 256);
     else STEP(9, 512);
 #undef OWN
+#undef LAUNCH
 #undef STEP
     return hipGetLastError();
 }

@@ -1,14 +1,14 @@
 """The step kernel at the sizes where its passes, slots and units change:
 whole tiles and tiles in parts, a target with more events in a pass than it has
 slots, a sub-row longer than a pass, more source ranges than one batch holds,
-blocks of rows without a synapse into the unit, units that change XCD.  Bit for
-bit against the oracle, as everything the step computes is.
+blocks of rows without a synapse into the unit, units that change XCD, networks of one
+unit and many cycles per launch.  Bit for bit against the oracle, as everything the step computes is.
 """
 import numpy as np
 import pytest
 
 import oracle
-from bsim_amd import netspec
+from bsim_amd import api, netspec
 
 from test_gpu_parity import DT, assert_same, run_gpu, say
 
@@ -115,3 +115,35 @@ def test_ranked_units(active):
     o = oracle.run(spec, DT, steps, rec_ids=rec, mode="csr", tile=256, threads=8)
     assert o.events > 10_000
     assert_same(r, o, "ranked units")
+
+
+@pytest.mark.parametrize("tile,dmax,n", [(192, 3, 1), (192, 3, 64), (192, 3, 65), (192, 7, 192), (192, 2, 193),
+                                         (384, 12, 128), (384, 12, 129), (768, 40, 256), (768, 63, 257)])
+def test_one_unit(tile, dmax, n):
+    """Networks of one unit take up to 64 cycles per launch, in the last case of
+    each pair one more neuron makes two."""
+    steps, s = 150, max(n // 4, 1) if n > 1 else 0
+    rng = np.random.Generator(np.random.PCG64(n))
+    b = netspec.Builder()
+    if s:
+        sources(b, s, steps, rng)
+    lif(b, n - s, rng)
+    if s:
+        connect(b, rng.integers(0, n, 12 * n), s + rng.integers(0, n - s, 12 * n), rng, dmax, 0.2)
+    else:
+        connect(b, np.zeros(3, int), np.zeros(3, int), rng, dmax, 0.2)
+    spec = b.build()
+    rec = sorted({0, n // 2, n - 1})
+    say(f"[gpu] one unit tile={tile} n={n}")
+    r = run_gpu(spec, steps, rec, tile)
+    assert_same(r, oracle.run(spec, DT, steps, rec_ids=rec, mode="csr", tile=256, threads=8), "one unit")
+    sim = api.Simulation(api.Network.from_spec(spec), DT, tile=tile)
+    for k in (1, 2, 64, 1, 65, 17):             # cycles in other portions
+        sim.step(k)
+    sim.finish()
+    sim.sync()
+    st = sim.state()
+    for k in ("v", "ie", "ii", "refrac"):
+        assert np.array_equal(st[k], r[k]), k
+    assert sim.events() == r["events"]
+    sim.close()
