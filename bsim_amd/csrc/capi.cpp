@@ -537,6 +537,7 @@ static bsim_sim *sim_from_layout(bsim::Layout &L, const bsim_sim_config &c, bsim
         int64_t rows = 0;
         for (const auto &r : L.rng) rows += (int64_t)(r.hi - r.lo) * L.dmax;
         d.wrows = (double)L.s < 1.25 * (double)L.off_tab.size() && rows >= (int64_t)32768 * L.ntiles ? 2 : 1;
+        d.many = d.ntiles >= BSIM_MANY_UNITS && d.tile <= 256 && d.wrows == 1;
     }
     if (dev_syn) {
         d.syn = dev_syn;

@@ -118,6 +118,10 @@ typedef struct __attribute__((aligned(16))) bsim_lifc {
 #define BSIM_CLS_SET_MASK 0x3FFFFFFFu   /* ncls: kind << 30 | parameter set */
 #define BSIM_DONE_STRIDE 16              /* uint64 per completion counter: one 128-byte line each */
 
+/* Units from which on the step kernel runs in workgroups of eight wavefronts,
+ * four per compute unit instead of two of twelve (step_many.hip). */
+#define BSIM_MANY_UNITS 2560
+
 /* Kernel arguments (passed by value). */
 typedef struct bsim_dev {
     int32_t n;           /* neurons */
@@ -125,7 +129,7 @@ typedef struct bsim_dev {
     int32_t ntiles;      /* units */
     int32_t dmax;        /* D, 1..BSIM_MAX_DELAY */
     int32_t nwords;      /* (n + 63) / 64 */
-    int32_t pad0;
+    int32_t many;        /* workgroups of eight wavefronts (step_many.hip) */
     /* neuron constants: kind and LIF parameter set per neuron, the sets'
      * shared constants, v_tmp per neuron */
     const uint32_t *ncls;       /* kind << 30 | index into lifc (LIF neurons) */

@@ -69,7 +69,10 @@
 #include "layout.h"
 
 #define WAVE 64
+#ifndef NEV                           /* step_many.hip sets it and STEP_EU */
 #define NEV 8                         /* event wavefronts of a step workgroup */
+#define STEP_EU 6                     /* wavefronts per SIMD: two workgroups per compute unit */
+#endif
 #define NOWN 4                        /* owner wavefronts */
 #define NTHREAD (WAVE * (NEV + NOWN))
 #define NCOL 16                       /* groups of 64 events in a pass */
@@ -79,19 +82,18 @@
 #define MAXR 32                       /* source chunks per batch */
 #define BLKS (BSIM_CHUNK / WAVE)      /* blocks of 64 pres per source chunk */
 #define NRES 8                        /* XCDs: workgroup w runs on XCD (w + c) mod 8 */
-#define STEP_EU 6                     /* wavefronts per SIMD: two workgroups per compute unit */
 static_assert(BLKS == WAVE, "a lane per block of a source chunk");
 static_assert(NCOL == 16 && NCOL % NEV == 0, "a target's histogram row is one 16-byte vector");
 
 /* Slots per target: a pass puts PASS / U events on a target of a unit of U on
  * average, if full; three times that, at least 8. */
-__host__ __device__ constexpr uint32_t slots_of(uint32_t U)
+__host__ __device__ static constexpr uint32_t slots_of(uint32_t U)
 {
     return U >= 384 ? 8u : (3u * PASS / U) & ~3u;
 }
 
 /* LDS bytes of a workgroup: chunk | hist | mark | slot | blk_end | blk_mark | btot, ctot, most, last */
-__host__ __device__ constexpr size_t lds_bytes(uint32_t U)
+__host__ __device__ static constexpr size_t lds_bytes(uint32_t U)
 {
     return 16 * MAXR + 2 * U * NCOL + 8 * PASS + 4 * slots_of(U) * U + 4 * MAXR * BLKS + 4 * NEV * WAVE + 8 * NEV +
            8 * MAXR + 16;
@@ -1102,6 +1104,24 @@ __global__ __launch_bounds__(NTHREAD, STEP_EU) void bsim_step_kernel(bsim_dev d,
     if (clocked && tid == 0) count_done(d, 1u);
 }
 
+#ifdef STEP_MANY
+extern "C" hipError_t bsim_launch_step_many(const bsim_dev *d, int32_t t, int32_t flags, hipStream_t stream)
+{
+    const uint32_t U = (uint32_t)d->tile;
+    if (U == 0 || U % WAVE != 0 || U > NOWN * WAVE) return hipErrorInvalidValue;
+    const dim3 grid(d->nslots + d->rank_wgs), block(NTHREAD);
+    const size_t lds = lds_bytes(U);
+    (void)hipGetLastError();       /* the check below then reports this launch alone */
+#define STEP(NB) hipLaunchKernelGGL((bsim_step_kernel<NB, 1, 1, false>), grid, block, lds, stream, *d, t, flags, 1)
+    if (U <= 64) STEP(6);
+    else if (U <= 128) STEP(7);
+    else STEP(8);
+#undef STEP
+    return hipGetLastError();
+}
+#else
+extern "C" hipError_t bsim_launch_step_many(const bsim_dev *d, int32_t t, int32_t flags, hipStream_t stream);
+
 /* One cycle, or with one unit (d.nslots 8, the others empty) and clocked as many
  * as cycles says: the launch and what a workgroup reads at its start are over
  * half of a small network's cycle.  us per cycle in runs, a launch each / 64 cycles a
@@ -1114,6 +1134,7 @@ extern "C" hipError_t bsim_launch_step(const bsim_dev *d, int32_t t, int32_t fla
     const uint32_t U = (uint32_t)d->tile;
     if (U == 0 || U % WAVE != 0 || U > BSIM_MAX_UNIT) return hipErrorInvalidValue;
     if (cycles != 1 && (t >= 0 || d->ntiles != 1)) return hipErrorInvalidValue;
+    if (d->many) return bsim_launch_step_many(d, t, flags, stream);
     const dim3 grid(d->nslots + d->rank_wgs), block(NTHREAD);
     const size_t lds = lds_bytes(U);
     (void)hipGetLastError();       /* the check below then reports this launch alone */
@@ -1135,3 +1156,4 @@ extern "C" hipError_t bsim_launch_step(const bsim_dev *d, int32_t t, int32_t fla
 #undef STEP
     return hipGetLastError();
 }
+#endif

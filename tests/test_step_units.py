@@ -96,11 +96,12 @@ def test_whole_tiles(npop, tile):
     assert_same(r, o, "whole tiles")
 
 
-@pytest.mark.parametrize("active", [1, 11])
-def test_ranked_units(active):
+@pytest.mark.parametrize("npop,active", [(11, 1), (11, 11), (52, 9)])
+def test_ranked_units(npop, active):
     """More units than run at a time, ranked every other cycle: populations of
-    which one is active (its units are dealt out to all XCDs) or every one."""
-    npop, n, s, steps = 11, 9408, 300, 40
+    which one, some or every one is active; with 52 also in workgroups of eight
+    wavefronts."""
+    n, s, steps = 9408, 300, 40
     rng = np.random.Generator(np.random.PCG64(active))
     b = netspec.Builder()
     for p in range(npop):
@@ -110,7 +111,7 @@ def test_ranked_units(active):
         connect(b, base + np.repeat(np.arange(s), 400), base + s + rng.integers(0, n, 400 * s), rng, 2, 0.05)
     spec = b.build()
     rec = [s, s + n - 1, spec.n - 1]
-    say(f"[gpu] ranked units active={active} n={spec.n} s={spec.s}")
+    say(f"[gpu] ranked units npop={npop} active={active} n={spec.n} s={spec.s}")
     r = run_gpu(spec, steps, rec, 192)
     o = oracle.run(spec, DT, steps, rec_ids=rec, mode="csr", tile=256, threads=8)
     assert o.events > 10_000
