@@ -365,11 +365,13 @@ bsim_sim *bsim_sim_create(const bsim_network *net, float dt, const bsim_sim_conf
     if (cfg) c = *cfg;
     const int32_t N = net->net.n();
     if (check_config(c, N, "bsim_sim_create") != 0) return nullptr;
-    const int32_t tile = c.tile > 0 ? c.tile : bsim::default_tile(bsim::max_delay_steps(net->net, dt));
+    const int32_t dmax = bsim::max_delay_steps(net->net, dt);
+    const int32_t tile = c.tile > 0 ? c.tile : bsim::default_tile(dmax);
+    const int32_t lt = bsim::layout_tile(N, tile, dmax);
     bsim::Layout L;
     std::string err;
     try {
-        if (bsim::build_layout(net->net, dt, tile, L, err, 0, bsim::default_parts(N, tile)) != 0) {
+        if (bsim::build_layout(net->net, dt, lt, L, err, 0, bsim::default_parts(N, lt)) != 0) {
             fail(BSIM_E_NETWORK, err);
             return nullptr;
         }
@@ -377,7 +379,12 @@ bsim_sim *bsim_sim_create(const bsim_network *net, float dt, const bsim_sim_conf
         fail(BSIM_E_NOMEM, "out of host memory while building the layout");
         return nullptr;
     }
-    return sim_from_layout(L, c, nullptr, 0);
+    bsim_sim *sim = sim_from_layout(L, c, nullptr, 0);
+    if (sim) {
+        sim->tile = tile;
+        sim->ntiles = (N + tile - 1) / tile;
+    }
+    return sim;
 }
 
 bsim_sim *bsim_sim_create_chains(const bsim_chain_params *p, int32_t count, float dt,

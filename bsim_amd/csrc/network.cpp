@@ -155,6 +155,19 @@ int32_t default_parts(int64_t n, int32_t tile)
     return tile >= 3 * BSIM_TILE_ALIGN || BSIM_NWAVE * tiles <= 256 * (tile / BSIM_TILE_ALIGN) ? BSIM_NWAVE : 1;
 }
 
+int32_t layout_tile(int64_t n, int32_t tile, int32_t dmax)
+{
+    /* With deep delay rings most of a cycle's lines are row-table entries, one
+     * per active row and unit, and a unit's run into the next unit's on the same
+     * XCD only while both run: with more units than two rounds of workgroups,
+     * units of twice the targets read fewer.  ms per cycle of the stress network
+     * with delays up to 50 steps in tiles of 768 / 1,536 (units of 256 / 512): 150,000
+     * neurons 1.43 / 1.69, 210,000 1.49 / 1.50, 290,000 2.07 / 2.03, 410,000 3.15 /
+     * 2.38, 1,010,000 11.1 / 5.7. */
+    const int64_t units = BSIM_NWAVE * ((n + tile - 1) / tile);
+    return dmax > 24 && tile >= 3 * BSIM_TILE_ALIGN && tile <= 4 * BSIM_TILE_ALIGN && units > 1024 ? 2 * tile : tile;
+}
+
 int build_layout(const HostNet &net, float dt, int32_t tile, Layout &L, std::string &err,
                  int32_t dmax_min, int32_t parts)
 {
@@ -549,9 +562,9 @@ int build_layout(const HostNet &net, float dt, int32_t tile, Layout &L, std::str
     L.tile_base.resize(NT);
     L.tile_nsyn.resize(NT);
     L.tile_res.resize(NT);
-    /* XCD residue of each group (workgroups are dispatched to the 8 XCDs
-     * round-robin by workgroup id): groups are spread over the residues to
-     * balance tile counts, so that a group's tiles share one L2 */
+    /* whole groups spread over eight residues to balance tile counts: a
+     * property of the layout that its checks compare (the device cuts the
+     * units into eight runs itself) */
     {
         std::vector<int64_t> rcount(8, 0);
         for (int32_t g = 0; g < NG; g++) {

@@ -71,10 +71,10 @@ struct Layout {
     std::vector<int32_t> src_lo, src_hi;     /* distinct source ranges */
     std::vector<int64_t> src_list_base;      /* list capacity (hi - lo) * D each */
     int64_t src_list_len = 0;
-    int32_t ngroups = 0, nslots = 0;         /* target groups; step workgroups */
+    int32_t ngroups = 0, nslots = 0;         /* target groups; 8 x the tiles of the largest residue */
     std::vector<int64_t> tile_base;          /* per tile: first synapse of its group */
     std::vector<uint32_t> tile_nsyn;         /* per tile: synapses of its group */
-    std::vector<uint8_t> tile_res;           /* per tile: XCD residue of its group */
+    std::vector<uint8_t> tile_res;           /* per tile: residue of its group */
     std::vector<int64_t> chunk_tiles_off;    /* per chunk: the tiles reading it */
     std::vector<int32_t> chunk_tiles;
     std::vector<int32_t> chunk_rng;          /* range entry of each (chunk, tile) */
@@ -99,6 +99,10 @@ int32_t max_delay_steps(const HostNet &net, float dt);
 /* Step workgroups (units) per tile for a network of n neurons in tiles of
  * `tile`: 1, or BSIM_NWAVE, one per target part. */
 int32_t default_parts(int64_t n, int32_t tile);
+
+/* The tile that a simulation of n neurons lays its targets out in, when tile is
+ * the caller's. */
+int32_t layout_tile(int64_t n, int32_t tile, int32_t dmax);
 
 /* Returns 0 or a negative code with a message in err.  The delay ring is at
  * least dmax_min steps deep (a part of a larger layout uses the whole

@@ -73,7 +73,8 @@ int bsim_mlp_train(bsim_mlp *m, const int32_t *rows, int32_t steps, int32_t batc
  * results as bsim_mlp_train, but the per-call staging (the minibatch row
  * indices and the per-step losses) lives in a fixed device array of
  * BSIM_MLP_NOALLOC_WORDS 32-bit words per GPU, allocated with the library
- * and held until the process ends, instead of a hipMalloc per call:
+ * and held until the process ends, instead of the model's and its pinned
+ * buffers, so a call takes no event and no host thread of its own either:
  * round_up(steps, 64) + steps * batch must not exceed it (255 steps at batch
  * 4,096), or BSIM_E_ARG is returned.  Calls on one GPU share the array:
  * calls that overlap on one GPU (from several threads or handles) race. */

@@ -148,3 +148,25 @@ def test_one_unit(tile, dmax, n):
         assert np.array_equal(st[k], r[k]), k
     assert sim.events() == r["events"]
     sim.close()
+
+
+@pytest.mark.parametrize("npop", [26, 28])
+def test_deep_delays_of_many_units(npop):
+    """Delays past 24 steps with more than 341 tiles of 768 are laid out in tiles
+    of twice the size (28 populations); what the caller sees stays."""
+    n, s, steps, dmax, tile = 9600, 200, 60, 30, 768
+    rng = np.random.Generator(np.random.PCG64(npop))
+    b = netspec.Builder()
+    for p in range(npop):
+        base = p * (s + n)
+        sources(b, s, steps, rng, 0.1 if p % 3 else 0.4)
+        lif(b, n, rng)
+        connect(b, base + np.repeat(np.arange(s), 300), base + s + rng.integers(0, n, 300 * s), rng, dmax, 0.1)
+    spec = b.build()
+    rec = [s, s + n - 1, spec.n - 1]
+    say(f"[gpu] deep delays npop={npop} n={spec.n} s={spec.s}")
+    r = run_gpu(spec, steps, rec, tile)
+    assert r["info"]["tile"] == tile and r["info"]["ntiles"] == -(-spec.n // tile)
+    o = oracle.run(spec, DT, steps, rec_ids=rec, mode="csr", tile=256, threads=8)
+    assert o.events > 10_000
+    assert_same(r, o, "deep delays")
