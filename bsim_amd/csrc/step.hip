@@ -50,14 +50,15 @@
  * applied them by masks per 64 events took 3.8 us per 768 events; here the
  * expansion and the sort of 1,024 events are spread over eight wavefronts,
  * every row is expanded once and not once per part, and the sequential part,
- * the adds, is left to the owners: 2 us.  Whole step launch, before and after:
- * 330,000 neurons at ~100 Hz (3.1e6 events) 83 / 60 us, 110,000 at ~1,600 Hz
- * with delays up to 50 steps (3.2e7 events) 3,408 / 927, 96 chains of 100 to
- * 1,000 neurons (2.4e5 events) 46 / 30, 650,000 neurons at ~100 Hz (7e6
- * events) 106 / 106.  Measured and not used: 4 event wavefronts (71, 1,930, 33,
- * 121 us for the same, whole tiles), 16 (one workgroup per compute unit), LDS
- * masks by target instead of ballots (70 against 60 us for the first), four
- * wavefronts that each take the add of their own targets (71).
+ * the adds, is left to the owners: 2 us.  Whole step launch, before and now:
+ * 330,000 neurons at ~100 Hz (3.1e6 events) 83 / 54 us, 110,000 at ~1,600 Hz
+ * with delays up to 50 steps (3.2e7 events) 3,408 / 877, 96 chains of 100 to
+ * 1,000 neurons (2.4e5 events) 46 / 29, 650,000 neurons at ~100 Hz (7e6
+ * events, workgroups of eight wavefronts) 106 / 91.  Measured and not used: 4
+ * event wavefronts for all but the last (71, 1,930, 33 us when these took 60, 927
+ * and 30), 16 (one workgroup per compute unit), LDS masks by target instead of
+ * ballots (70 against 60 us for the first), four wavefronts that each take the
+ * add of their own targets (71).
  *
  * Arithmetic: compiled with -ffp-contract=off (no FMA contraction) and
  * without denormal flushing, so V = ((Cm*V + v_tmp) + iE*C_E) + iI*C_I rounds
@@ -719,8 +720,11 @@ __device__ __forceinline__ void count_done(const bsim_dev &d, uint64_t cycles)
  * to XCD s % 8, and starts an XCD's in order.  The units are cut, in index order,
  * into eight runs of equal cost, one per XCD: units of a group, which read the
  * same rows at the same time, so share an L2.  Within an XCD the heavy units come
- * first, by half-octave classes (counting sort; within a class the order is
- * arbitrary).  An XCD has slots for an eighth of the units; the lightest of a
+ * first, by half-octave classes (counting sort).  Within a class the order is
+ * arbitrary up to delays of RANK_ORDERED_DMAX steps, and while two workgroups per
+ * compute unit hold all units; past them, where most lines are row-table entries
+ * that a group's units share while they run together, units keep their order: 1,010,000 neurons with delays up to 50 steps 7.65 / 6.14
+ * ms, 410,000 2.51 / 2.36, but 330,000 with delays up to 6 56.5 / 57.9 us.  An XCD has slots for an eighth of the units; the lightest of a
  * longer run fill what others leave free, so that no XCD starts more workgroups
  * than another.  us per cycle with whole groups on XCDs / with the units dealt
  * out in turn where those were uneven / with runs: 330,000 neurons at ~100 Hz
@@ -732,6 +736,7 @@ __device__ __forceinline__ void count_done(const bsim_dev &d, uint64_t cycles)
  * that it has read.  The classes of the units are kept in LDS where they fit. */
 #define RANK_CLASSES 64
 #define RANK_FIXED 8192ull
+#define RANK_ORDERED_DMAX 24
 
 __device__ __forceinline__ uint32_t load_class(uint64_t x)
 {
@@ -788,20 +793,17 @@ __device__ void rank_units(const bsim_dev &d, uint64_t *load, int32_t *perm, uin
     }
     __syncthreads();
     /* exclusive prefix of each residue's class counts, heaviest class first */
+    const uint32_t x8 = tid / RANK_CLASSES;
     if (counts) {
-        const uint32_t x = tid / RANK_CLASSES, c = RANK_CLASSES - 1u - tid % RANK_CLASSES;
-        const uint32_t v = cnt[x * RANK_CLASSES + c], incl = wave_incl_scan(v);
-        fill[x * RANK_CLASSES + c] = incl - v;
-        if (c == 0) rtot[x] = incl;
+        const uint32_t c = RANK_CLASSES - 1u - tid % RANK_CLASSES;
+        const uint32_t v = cnt[x8 * RANK_CLASSES + c], incl = wave_incl_scan(v);
+        fill[x8 * RANK_CLASSES + c] = incl - v;
+        if (c == 0) rtot[x8] = incl;
     }
     __syncthreads();
     /* unit of residue x at rank i goes to slot NRES * i + x */
     const uint32_t cap = (uint32_t)d.nslots / NRES;
-    at = upto - mine;
-    for (int32_t k = k0; k < k1; k++) {
-        const uint32_t c = cls[k];
-        uint32_t x = residue(at), pos = atomicAdd(&fill[x * RANK_CLASSES + c], 1u);
-        at += class_cost(c);
+    auto place = [&](int32_t k, uint32_t x, uint32_t pos) {
         if (pos >= cap) {                           /* the n-th unit without a slot */
             uint32_t n = pos - cap;
             for (uint32_t y = 0; y < x; y++) n += max(rtot[y], cap) - cap;
@@ -809,6 +811,31 @@ __device__ void rank_units(const bsim_dev &d, uint64_t *load, int32_t *perm, uin
             pos = rtot[x] + n;
         }
         perm[NRES * pos + x] = k;
+    };
+    if (d.dmax <= RANK_ORDERED_DMAX || d.ntiles <= 512) {
+        at = upto - mine;
+        for (int32_t k = k0; k < k1; k++) {
+            const uint32_t c = cls[k], x = residue(at);
+            at += class_cost(c);
+            place(k, x, atomicAdd(&fill[x * RANK_CLASSES + c], 1u));
+        }
+    } else if (counts) {
+        /* a wavefront per run, 64 units at a time, so that the units of a class
+         * keep their order */
+        const uint32_t lane = tid & (WAVE - 1);
+        int32_t b = 0;
+        for (uint32_t y = 0; y < x8; y++) b += (int32_t)rtot[y];
+        for (const int32_t end = b + (int32_t)rtot[x8]; b < end; b += WAVE) {
+            const int32_t k = b + (int32_t)lane;
+            const uint32_t c = k < end ? cls[k] : 0u;
+            const uint64_t m = same_lanes<6>(c, ballot64(k < end));
+            const uint32_t before = (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+            const uint32_t pos = fill[x8 * RANK_CLASSES + c] + before;
+            wave_sync();
+            if (k < end && before == 0u) fill[x8 * RANK_CLASSES + c] += (uint32_t)__popcll(m);
+            wave_sync();
+            if (k < end) place(k, x8, pos);
+        }
     }
     /* the remaining slots are empty */
     uint32_t over = 0;
