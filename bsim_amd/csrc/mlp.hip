@@ -348,14 +348,28 @@ __device__ inline void gemm_tile(const GemmArgs &g, int32_t bx, int32_t by)
     }
 }
 
+/* Tile t of ny x nx: bands of `band` rows, in a band column by column.  The
+ * workgroups that an XCD runs at a time so form a block of tiles that shares rows
+ * and columns in its L2; row by row (a band of 1) they read one row of tiles and,
+ * in wide layers, more columns than it holds.  Training steps of 4,096 rows, us,
+ * products and weight gradients row by row / in bands: 3 x 1,024 units 185 / 179,
+ * 3 x 1,536 317 / 290, 2 x 4,096 and 4,096 outputs 2,020 / 1,560. */
+__device__ inline void band_tile(int32_t t, int32_t nx, int32_t ny, int32_t band, int32_t &bx, int32_t &by)
+{
+    const int32_t b = t / (band * nx) * band, h = min(band, ny - b), i = t - b * nx;
+    bx = i / h;
+    by = b + i % h;
+}
+
 template <int EPI>
 __global__ __launch_bounds__(GEMM_THREADS) void mlp_gemm(GemmArgs g)
 {
-    /* an XCD takes consecutive tiles, row by row: it reads an eighth of A, and
-     * the rows that it wrote itself in the layer before */
-    const int32_t nx = g.N / BN, nt = (int32_t)gridDim.x, x = (int32_t)blockIdx.x % 8;
-    const int32_t t = x * (nt / 8) + min(x, nt % 8) + (int32_t)blockIdx.x / 8;
-    gemm_tile<EPI>(g, t % nx, t / nx);
+    /* an XCD takes consecutive tiles: it reads an eighth of A, and the rows that
+     * it wrote itself in the layer before */
+    const int32_t nt = (int32_t)gridDim.x, x = (int32_t)blockIdx.x % 8;
+    int32_t bx, by;
+    band_tile(x * (nt / 8) + min(x, nt % 8) + (int32_t)blockIdx.x / 8, g.N / BN, g.M / BM, 8, bx, by);
+    gemm_tile<EPI>(g, bx, by);
 }
 
 /* ---- every layer in one launch ---------------------------------------------
@@ -661,7 +675,8 @@ __global__ __launch_bounds__(W * WAVE) void mlp_chain(ChainArgs a)
 struct UpdateArgs {
     int32_t nlin, batch;
     int32_t n[MAX_LAYERS], k[MAX_LAYERS];   /* W_l is [n][k] */
-    int32_t tfirst[MAX_LAYERS + 1];         /* first 64 x 64 tile of W_l */
+    int32_t tfirst[MAX_LAYERS + 1];         /* first workgroup of W_l's tiles */
+    int32_t wide[MAX_LAYERS];               /* tiles of 128 x 128, else 64 x 64 */
     int32_t bfirst[MAX_LAYERS + 1];         /* first bias workgroup of layer l; those before the tiles': */
     int32_t nbias;                          /*   a multiple of 8, the last ones idle */
     int32_t update;                         /* 0: only write the gradient */
@@ -725,14 +740,77 @@ __device__ inline void put_weights(const WTile &tile, uint16_t *w, uint16_t *wt,
  * 22 now (950,000 parameters, 4,096 rows), and 27 + 10 / 22 (2,600,000, 2,048
  * rows).  Four steps in flight instead of two need the registers of a second
  * workgroup per compute unit: 28 us for the latter.
+ *
+ * Layers of 2,048 x 2,048 and more whose operands exceed 192 MB (a quarter less
+ * than the 256 MB cache between the L2s and memory) go in tiles of 128 x 128, a
+ * 64 x 64 quadrant per wavefront in the whole batch, quarter by quarter: the four
+ * wavefronts walk one place of the batch instead of four, with half the bytes per
+ * product.  Two layers of 4,096 x 4,096, 16,384 rows: 158 million lines missed the
+ * L2s in tiles of 64, 2,900 us; the training step 6,950 us so, 5,850 in tiles of
+ * 128.  Below the line tiles of 64 are as good (3,072 x 3,072, 8,192 rows: 2,475 /
+ * 2,436; 2,048 x 2,048, 16,384 rows: 2,310 / 2,412), and with fewer than 256 tiles
+ * of 128 compute units stay idle (512 x 512, 65,536 rows: 740 / 1,270).
+ * Tiles of 64 of layers from 1,024 x 1,024 up are taken in bands of four (band_tile);
+ * smaller ones row by row (9 x 512 units, 16,384 rows: 490 / 502).
  * The workgroups before them take 256 biases each, the first also the step's loss. */
 constexpr int UP_THREADS = KSPLIT * WAVE;
+constexpr int64_t UP_WIDE_BYTES = 192ll << 20;   /* operands of a layer that goes in tiles of 128 x 128, */
+constexpr int UP_WIDE_TILES = 256;         /*   if it has as many */
+constexpr int UP_BAND_AREA = 1024 * 1024;  /* parameters of a layer whose tiles of 64 go in bands */
 constexpr int UP_DEPTH = 2;                /* steps of 32 rows in flight; a quarter of a batch has whole pairs */
 constexpr int UP_JS = 80, UP_IR = 4 * UP_JS;     /* LDS strides (floats) of a sum's 16 columns and 4 x 16 */
 
-__global__ __launch_bounds__(UP_THREADS) void mlp_update(UpdateArgs a)
+/* Adam's operands of a thread: column lane of rows w, w + 4, ... of a tile of W
+ * whose first is parameter i0. */
+constexpr int UP_E = 64 / KSPLIT;
+struct AdamState {
+    float p[UP_E], m[UP_E], v[UP_E];
+};
+
+__device__ inline void load_adam(const UpdateArgs &a, int64_t i0, int32_t K, AdamState &st)
 {
-    __shared__ __align__(16) float sums[KSPLIT][16 * UP_IR];
+#pragma unroll
+    for (int e = 0; e < UP_E; e++) {
+        const int64_t i = i0 + (int64_t)e * KSPLIT * K;
+        st.p[e] = a.p[i];
+        st.m[e] = a.m[i];
+        st.v[e] = a.v[i];
+    }
+}
+
+typedef float TileSum[16 * UP_IR];
+
+/* Where the sum of (row, column lane) of a tile lies. */
+__device__ inline uint32_t sum_at(uint32_t row, uint32_t lane)
+{
+    return (row / 16 * 4 + row % 4) * UP_IR + lane / 16 * UP_JS + row % 16 / 4 * 16 + lane % 16;
+}
+
+/* The gradient of a tile (row r0, column c0) of W_l in g: written out, and with
+ * update Adam's step and the bf16 copies, through LDS that nobody reads any more. */
+__device__ inline void finish_tile(const UpdateArgs &a, int l, int32_t r0, int32_t c0, int64_t i0,
+                                   const float (&g)[UP_E], const AdamState &st, TileSum &lds)
+{
+    const uint32_t lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+    const int32_t N = a.n[l], K = a.k[l];
+    if (a.grad)
+#pragma unroll
+        for (int e = 0; e < UP_E; e++) a.grad[i0 + (int64_t)e * KSPLIT * K] = g[e];
+    if (!a.update) return;                                      /* uniform */
+    __syncthreads();                                            /* the sums are read */
+    WTile &tile = *reinterpret_cast<WTile *>(&lds[0]);
+#pragma unroll
+    for (int e = 0; e < UP_E; e++)
+        tile[w + e * KSPLIT][lane] = f2bf(adam(a, i0 + (int64_t)e * KSPLIT * K, g[e], st.p[e], st.m[e], st.v[e]));
+    __syncthreads();
+    put_weights(tile, a.w + a.woff[l], a.wt + a.woff[l], N, K, r0, c0);
+}
+
+/* WIDE: some layers in tiles of 128 x 128 (UpdateArgs::wide). */
+template <bool WIDE>
+__global__ __launch_bounds__(UP_THREADS, 2) void mlp_update(UpdateArgs a)
+{
+    __shared__ __align__(16) TileSum sums[KSPLIT];
     const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1), w = __builtin_amdgcn_readfirstlane(tid / WAVE);
     if ((int32_t)blockIdx.x < a.nbias) {
         if (blockIdx.x == 0 && w == 0 && a.loss) {
@@ -765,23 +843,27 @@ __global__ __launch_bounds__(UP_THREADS) void mlp_update(UpdateArgs a)
         if (a.update) (void)adam(a, i, g, a.p[i], a.m[i], a.v[i]);
         return;
     }
-    /* an XCD takes consecutive tiles: they share rows of dZ */
+    /* an XCD takes consecutive tiles: they share rows of dZ and of the inputs */
     const int32_t nt = a.tfirst[a.nlin], b = (int32_t)blockIdx.x - a.nbias, x = b % 8;
     const int32_t t = x * (nt / 8) + min(x, nt % 8) + b / 8;
     int l = 0;
     while (l + 1 < a.nlin && t >= a.tfirst[l + 1]) l++;
-    const int32_t N = a.n[l], K = a.k[l], tk = K / 64, ti = t - a.tfirst[l];
-    const int32_t r0 = (ti / tk) * 64, c0 = (ti % tk) * 64;
-    const int32_t ns = a.batch / 32 / KSPLIT;
-    const uint16_t *pa = a.dzt[l] + ((int64_t)w * ns * N + r0) * 32;
-    const uint16_t *pb = a.act_t[l] + ((int64_t)w * ns * K + c0) * 32;
+    const bool wide = WIDE && a.wide[l] != 0;                   /* uniform */
+    const int32_t N = a.n[l], K = a.k[l], ti = t - a.tfirst[l], ns = a.batch / 32 / KSPLIT;
+    int32_t r0, c0;
+    const int32_t side = wide ? 128 : 64;
+    band_tile(ti, K / side, N / side, wide ? 8 : N * K >= UP_BAND_AREA ? 4 : 1, c0, r0);
+    r0 *= side;
+    c0 *= side;
+    /* this wavefront's 64 x 64: the tile in its quarter of the batch, or its
+     * quadrant of a wide tile in all of it */
+    const int32_t wr = wide ? r0 + (int32_t)w / 2 * 64 : r0, wc = wide ? c0 + (int32_t)w % 2 * 64 : c0;
+    const int32_t s0 = wide ? 0 : (int32_t)w * ns;
+    const uint16_t *pa = a.dzt[l] + ((int64_t)s0 * N + wr) * 32;
+    const uint16_t *pb = a.act_t[l] + ((int64_t)s0 * K + wc) * 32;
     constexpr int D = UP_DEPTH;
     bf16x8 fa[D][4], fb[D][4];
     f32x4 acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto issue = [&](int d, int32_t s) {
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -796,58 +878,57 @@ __global__ __launch_bounds__(UP_THREADS) void mlp_update(UpdateArgs a)
             for (int j = 0; j < 4; j++)
                 acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[d][i], fb[d][j], acc[i][j], 0, 0, 0);
     };
-    /* Adam's operands, which so arrive during the products.  Thread: column lane of
-     * rows w, w + 4, ... of the tile */
-    constexpr int E = 64 / KSPLIT;
-    float g[E], po[E], mo[E], vo[E];
     const int64_t i0 = a.woff[l] + (int64_t)(r0 + (int32_t)w) * K + c0 + lane;
-    if (a.update) {
+    AdamState st;
+    if (!WIDE && a.update) load_adam(a, i0, K, st);             /* arrives during the products */
+    const int32_t nq = wide ? KSPLIT : 1;
+    for (int32_t q = 0; q < nq; q++) {
 #pragma unroll
-        for (int e = 0; e < E; e++) {
-            const int64_t i = i0 + (int64_t)e * KSPLIT * K;
-            po[e] = a.p[i];
-            mo[e] = a.m[i];
-            vo[e] = a.v[i];
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int d = 0; d < D; d++) issue(d, d);
+        for (int32_t s = D; s < ns; s += D) {
+#pragma unroll
+            for (int d = 0; d < D; d++) {
+                mul(d);
+                issue(d, s + d);
+            }
         }
+#pragma unroll
+        for (int d = 0; d < D; d++) mul(d);
+        pa += (int64_t)ns * N * 32;
+        pb += (int64_t)ns * K * 32;
+        /* lane holds rows 16 i + 4 (lane / 16) + r, column 16 j + lane % 16 */
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    float &x = sums[w][(i * 4 + r) * UP_IR + j * UP_JS + lane];
+                    x = q == 0 ? acc[i][j][r] : x + acc[i][j][r];
+                }
     }
+    __syncthreads();
+    for (int32_t z = 0; z < nq; z++) {
+        const int32_t zr = z / 2 * 64, zc = z % 2 * 64;
+        const int64_t zi = i0 + (int64_t)zr * K + zc;
+        if (WIDE && a.update) load_adam(a, zi, K, st);
+        float g[UP_E];
 #pragma unroll
-    for (int d = 0; d < D; d++) issue(d, d);
-    for (int32_t s = D; s < ns; s += D) {
+        for (int e = 0; e < UP_E; e++) {
+            const uint32_t o = sum_at(w + e * KSPLIT, lane);
+            g[e] = 0.f;
+            if (wide)
+                g[e] += sums[z][o];
+            else
 #pragma unroll
-        for (int d = 0; d < D; d++) {
-            mul(d);
-            issue(d, s + d);
+                for (int y = 0; y < KSPLIT; y++) g[e] += sums[y][o];
         }
+        finish_tile(a, l, r0 + zr, c0 + zc, zi, g, st, sums[z]);
     }
-#pragma unroll
-    for (int d = 0; d < D; d++) mul(d);
-    /* lane holds rows 16 i + 4 (lane / 16) + r, column 16 j + lane % 16 */
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) sums[w][(i * 4 + r) * UP_IR + j * UP_JS + lane] = acc[i][j][r];
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < E; e++) {
-        const uint32_t row = w + e * KSPLIT;
-        const uint32_t o = (row / 16 * 4 + row % 4) * UP_IR + lane / 16 * UP_JS + row % 16 / 4 * 16 + lane % 16;
-        g[e] = 0.f;
-#pragma unroll
-        for (int z = 0; z < KSPLIT; z++) g[e] += sums[z][o];
-    }
-    if (a.grad)
-#pragma unroll
-        for (int e = 0; e < E; e++) a.grad[i0 + (int64_t)e * KSPLIT * K] = g[e];
-    if (!a.update) return;                                      /* uniform */
-    __syncthreads();                                            /* the sums are read */
-    WTile &tile = *reinterpret_cast<WTile *>(&sums[0][0]);
-#pragma unroll
-    for (int e = 0; e < E; e++)
-        tile[w + e * KSPLIT][lane] = f2bf(adam(a, i0 + (int64_t)e * KSPLIT * K, g[e], po[e], mo[e], vo[e]));
-    __syncthreads();
-    put_weights(tile, a.w + a.woff[l], a.wt + a.woff[l], N, K, r0, c0);
 }
 
 /* Input conversion: f32 [rows][in_dim] -> bf16 [n][kin] (zero padded). */
@@ -1168,12 +1249,17 @@ int update(bsim_mlp *m, int32_t batch, bool upd, float lr, float *grad_out, floa
 {
     const int L = m->nlin, t = m->step + 1;
     UpdateArgs a{};
+    bool any_wide = false;
     a.nlin = L;
     a.batch = batch;
     for (int l = 0; l < L; l++) {
         a.n[l] = m->kdim[l + 1];
         a.k[l] = m->kdim[l];
-        a.tfirst[l + 1] = a.tfirst[l] + (a.n[l] / 64) * (a.k[l] / 64);
+        const int32_t nt = (a.n[l] / 64) * (a.k[l] / 64);
+        a.wide[l] = a.n[l] % 128 == 0 && a.k[l] % 128 == 0 && nt / 4 >= UP_WIDE_TILES &&
+                    (int64_t)(a.n[l] + a.k[l]) * batch * 2 >= UP_WIDE_BYTES;
+        any_wide |= a.wide[l] != 0;
+        a.tfirst[l + 1] = a.tfirst[l] + (a.wide[l] ? nt / 4 : nt);
         a.bfirst[l + 1] = a.bfirst[l] + (a.n[l] + UP_THREADS - 1) / UP_THREADS;
         a.woff[l] = m->woff[l];
         a.boff[l] = m->boff[l];
@@ -1200,7 +1286,9 @@ int update(bsim_mlp *m, int32_t batch, bool upd, float lr, float *grad_out, floa
     a.lscale = 1.0f / ((float)batch * (float)m->cfg.out_dim);
     a.loss = loss_dev;
     (void)hipGetLastError();   /* the check after the launch reports it alone */
-    hipLaunchKernelGGL(mlp_update, dim3((uint32_t)(a.nbias + a.tfirst[L])), dim3(UP_THREADS), 0, m->stream, a);
+    const dim3 grid((uint32_t)(a.nbias + a.tfirst[L]));
+    if (any_wide) hipLaunchKernelGGL((mlp_update<true>), grid, dim3(UP_THREADS), 0, m->stream, a);
+    else hipLaunchKernelGGL((mlp_update<false>), grid, dim3(UP_THREADS), 0, m->stream, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_check(e, "update launch");
     if (upd) m->step++;
