@@ -163,7 +163,8 @@ int32_t layout_tile(int64_t n, int32_t tile, int32_t dmax)
      * units of twice the targets read fewer.  ms per cycle of the stress network
      * with delays up to 50 steps in tiles of 768 / 1,536 (units of 256 / 512): 150,000
      * neurons 1.43 / 1.69, 210,000 1.49 / 1.50, 290,000 2.07 / 2.03, 410,000 3.15 /
-     * 2.38, 1,010,000 11.1 / 5.7. */
+     * 2.38, 1,010,000 11.1 / 5.7.  A tile that build_layout refuses stays as it is. */
+    if (tile <= 0 || tile % BSIM_TILE_ALIGN != 0) return tile;
     const int64_t units = BSIM_NWAVE * ((n + tile - 1) / tile);
     return dmax > 24 && tile >= 3 * BSIM_TILE_ALIGN && tile <= 4 * BSIM_TILE_ALIGN && units > 1024 ? 2 * tile : tile;
 }

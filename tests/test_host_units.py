@@ -11,7 +11,7 @@ SRC = os.path.join(os.path.dirname(os.path.dirname(CPP)), "bsim_amd", "csrc")
 
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="no g++")
-@pytest.mark.parametrize("prog", ["unit_table_check"])
+@pytest.mark.parametrize("prog", ["unit_table_check", "sim_layout_check"])
 def test_host_program(prog, tmp_path):
     exe = str(tmp_path / prog)
     subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-fopenmp", "-fsanitize=address,undefined",
