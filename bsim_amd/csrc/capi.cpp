@@ -367,11 +367,10 @@ bsim_sim *bsim_sim_create(const bsim_network *net, float dt, const bsim_sim_conf
     if (check_config(c, N, "bsim_sim_create") != 0) return nullptr;
     const int32_t dmax = bsim::max_delay_steps(net->net, dt);
     const int32_t tile = c.tile > 0 ? c.tile : bsim::default_tile(dmax);
-    const int32_t lt = bsim::layout_tile(N, tile, dmax);
     bsim::Layout L;
     std::string err;
     try {
-        if (bsim::build_layout(net->net, dt, lt, L, err, 0, bsim::default_parts(N, lt)) != 0) {
+        if (bsim::build_sim_layout(net->net, dt, tile, dmax, L, err) != 0) {
             fail(BSIM_E_NETWORK, err);
             return nullptr;
         }

@@ -170,7 +170,7 @@ int32_t layout_tile(int64_t n, int32_t tile, int32_t dmax)
 }
 
 int build_layout(const HostNet &net, float dt, int32_t tile, Layout &L, std::string &err,
-                 int32_t dmax_min, int32_t parts)
+                 int32_t dmax_min, int32_t parts, int64_t group_max)
 {
     const int32_t N = net.n();
     const int64_t S = net.s();
@@ -501,9 +501,9 @@ int build_layout(const HostNet &net, float dt, int32_t tile, Layout &L, std::str
     const int32_t NG = (int32_t)gstart.size();
     gstart.push_back(NT);
     for (int32_t g = 0; g < NG; g++) {
-        if (L.tile_syn[gstart[g + 1]] - L.tile_syn[gstart[g]] >= ((int64_t)1 << 32)) {
+        if (L.tile_syn[gstart[g + 1]] - L.tile_syn[gstart[g]] >= group_max) {
             err = "a tile group receives 2^32 or more synapses; use a smaller tile";
-            return -6;
+            return kGroupTooLarge;
         }
     }
     /* group row tables: per group and range, entry
@@ -648,6 +648,19 @@ int build_layout(const HostNet &net, float dt, int32_t tile, Layout &L, std::str
             }
     }
     return 0;
+}
+
+int build_sim_layout(const HostNet &net, float dt, int32_t tile, int32_t dmax, Layout &L, std::string &err,
+                     int64_t group_max)
+{
+    const int32_t lt = layout_tile(net.n(), tile, dmax);
+    int rc = build_layout(net, dt, lt, L, err, 0, default_parts(net.n(), lt), group_max);
+    if (rc == kGroupTooLarge && lt != tile) {
+        L = Layout();
+        err.clear();
+        rc = build_layout(net, dt, tile, L, err, 0, default_parts(net.n(), tile), group_max);
+    }
+    return rc;
 }
 
 int append_layout(Layout &A, Layout &B, std::string &err)

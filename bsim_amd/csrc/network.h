@@ -104,12 +104,21 @@ int32_t default_parts(int64_t n, int32_t tile);
  * the caller's. */
 int32_t layout_tile(int64_t n, int32_t tile, int32_t dmax);
 
+/* Synapses that a target group may not reach: row-table entries are 32-bit offsets in it. */
+constexpr int64_t kGroupSynapses = (int64_t)1 << 32;
+constexpr int kGroupTooLarge = -6;
+
 /* Returns 0 or a negative code with a message in err.  The delay ring is at
  * least dmax_min steps deep (a part of a larger layout uses the whole
  * network's depth).  parts: row-table entries per tile and row (1 or
- * BSIM_NWAVE). */
+ * BSIM_NWAVE).  kGroupTooLarge: a group receives group_max synapses or more. */
 int build_layout(const HostNet &net, float dt, int32_t tile, Layout &out, std::string &err,
-                 int32_t dmax_min = 0, int32_t parts = 1);
+                 int32_t dmax_min = 0, int32_t parts = 1, int64_t group_max = kGroupSynapses);
+
+/* The layout of a simulation in tiles of the caller's size, or of layout_tile's
+ * where its groups, twice as large then, stay below group_max synapses. */
+int build_sim_layout(const HostNet &net, float dt, int32_t tile, int32_t dmax, Layout &out, std::string &err,
+                     int64_t group_max = kGroupSynapses);
 
 /* Appends layout B -- built, with the same tile and delay ring depth, for a
  * network placed after A's neurons, with no synapse between the two -- to A:
