@@ -967,8 +967,15 @@ int32_t bsim_sim_set_schedule(bsim_sim *sim, int32_t rank_every)
     if (sim->d.rank_every == rank_every) return 0;
     hipError_t e;
     /* the captured launches hold the kernel arguments: capture again; the
-     * loads of a tile ranked later start from zero */
+     * loads of a tile ranked later start from zero; which of the two orders a
+     * launch reads depends on rank_every, so both become the one that the next
+     * launch would have read */
+    const bsim_dev &d = sim->d;
+    const size_t order = (size_t)d.nslots * sizeof(int32_t);
+    const int32_t half = d.rank_every > 0 && sim->cycle > 0 ? (sim->cycle - 1) / d.rank_every & 1 : 0;
     if ((e = hipStreamSynchronize(sim->stream)) != hipSuccess ||
+        (order > 0 && (e = hipMemcpyAsync(d.perm + (half ^ 1) * (int64_t)d.nslots, d.perm + half * (int64_t)d.nslots,
+                                          order, hipMemcpyDeviceToDevice, sim->stream)) != hipSuccess) ||
         (e = hipMemsetAsync(sim->d.tile_load, 0, (size_t)(sim->d.ntiles > 0 ? sim->d.ntiles : 1) * 16,
                             sim->stream)) != hipSuccess ||
         (e = hipStreamSynchronize(sim->stream)) != hipSuccess)

@@ -170,7 +170,7 @@ typedef struct bsim_dev {
                                    ranking and the one before */
     uint64_t *tile_load;        /* [2][ntiles] work of a launch before a ranking (x 16), by cycle parity */
     int32_t rank_every;         /* units ranked heaviest first every this many cycles (0: never,
-                                   the units stay in their initial order) */
+                                   the units stay in their last order) */
     int32_t rank_wgs;           /* workgroups before the slots' (the first ranks): 8, or 0 where the
                                    units run in their initial order */
     uint8_t *tile_cls;          /* [ntiles] half-octave class of a unit's work */

@@ -220,8 +220,7 @@ void *bsim_sim_stream(bsim_sim *sim);
  * step's workgroups take the tiles.  Every rank_every cycles one
  * workgroup ranks the tiles for the launches after it by their work in the
  * launch before, heaviest first (the default, 2); 0 keeps the tiles in their
- * first order.  So many workgroups run at a time that a small network's
- * order is nothing; it is not ranked.
+ * last order.  A small network's workgroups all run at a time; it is not ranked.
  * Results do not depend on it.  Takes effect from the next step. */
 int32_t bsim_sim_set_schedule(bsim_sim *sim, int32_t rank_every);
 
