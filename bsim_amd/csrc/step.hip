@@ -635,7 +635,12 @@ __device__ void owner_wave(const Shared &S, uint32_t U, uint32_t K, uint32_t &pa
 __device__ __forceinline__ void prepare_batch(const Shared &S, const bsim_dev &d, const bsim_unit *un, int32_t rb,
                                               int32_t nrb, int32_t list, uint32_t buf)
 {
-    const uint32_t lane = threadIdx.x & (WAVE - 1);
+    uint32_t lane = threadIdx.x & (WAVE - 1);
+#ifdef STEP_MANY
+    /* keeps the addresses below from being held in registers from batch to batch,
+     * where the one too many went to private memory */
+    asm volatile("" : "+v"(lane));
+#endif
     const uint32_t *cnt = d.seg_count + (int64_t)list * d.nwords;
     for (int32_t c = (int32_t)wave_index(); c < nrb; c += NEV) {
         uint64_t ob;
