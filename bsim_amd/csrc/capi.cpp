@@ -320,12 +320,6 @@ static T *dev_upload(bsim_sim *sim, const std::vector<T> &v, hipError_t &e)
     return e == hipSuccess ? p : nullptr;
 }
 
-extern "C" {
-
-}  // extern "C"
-
-/* Checks the simulation config and makes its device current (0, or a
- * failure code). */
 /* Tile schedule: the units are ranked heaviest first every kRankEvery cycles,
  * by their work in the launch before (the volleys of the standard network move
  * slowly against 2 cycles); bsim_sim_set_schedule changes it. */
@@ -336,6 +330,8 @@ static const int32_t kRankEvery = 2;
  * 110,000 neurons with delays up to 50 steps: in order 1,010, ranked 877. */
 static const int32_t kRanked = 256;
 
+/* Checks the simulation config and makes its device current (0, or a
+ * failure code). */
 static int32_t check_config(const bsim_sim_config &c, int32_t N, const char *who)
 {
     if (c.rec_steps < 0 || c.n_rec < 0 || (c.n_rec > 0 && !c.rec_ids))

@@ -30,9 +30,10 @@
  * entries (bsim_range, one per source chunk of BSIM_CHUNK pres) point at its
  * first entry of row (lo, 1) and give the entries per row.
  *
- * Workgroups are dispatched to the 8 XCDs round-robin; every group has an XCD
- * residue and its tiles run in workgroups of that residue, so that they share
- * the XCD's L2.
+ * Workgroups are dispatched to the 8 XCDs round-robin, workgroup slot s to XCD
+ * s % 8.  The units, in index order, are cut into eight runs, one per XCD, so
+ * that most of a group's units share an L2: runs of as many units at first, of
+ * equal cost where the units are ranked (rank_units in step.hip).
  *
  * Spike history: hist[n] bit j = neuron n fired j cycles ago (bit 0 = this
  * cycle).  After updating cycle t, a unit writes its neurons' history words

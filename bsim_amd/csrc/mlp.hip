@@ -356,9 +356,14 @@ __device__ inline void gemm_tile(const GemmArgs &g, int32_t bx, int32_t by)
  * 3 x 1,536 317 / 290, 2 x 4,096 and 4,096 outputs 2,020 / 1,560. */
 __device__ inline void band_tile(int32_t t, int32_t nx, int32_t ny, int32_t band, int32_t &bx, int32_t &by)
 {
+    if (band == 1) {
+        by = t / nx;
+        bx = t - by * nx;
+        return;
+    }
     const int32_t b = t / (band * nx) * band, h = min(band, ny - b), i = t - b * nx;
     bx = i / h;
-    by = b + i % h;
+    by = b + (i - bx * h);
 }
 
 template <int EPI>
@@ -1046,7 +1051,9 @@ int dalloc(bsim_mlp *m, T **p, int64_t count)
  * after: gradients of 2.6 million parameters 960 / 620, predict of 100,003 rows
  * with 200 outputs (80 MB, of which the caller's pages are now most) 14,300 /
  * 4,300.  Short copies stay with the calling thread: to wake others costs
- * more (800 KB: 110 / 95 us). */
+ * more (800 KB: 110 / 95 us).  A model's first calls cost more, by the host's
+ * first touch of its two buffers, a page fault per 4 KB: get_params of 3.8 MB takes
+ * 750 us the first time and 200 after. */
 constexpr size_t PIN_BYTES = 4u << 20;
 constexpr size_t OMP_COPY_BYTES = 1u << 20;
 constexpr int COPY_THREADS = 4;            /* as good as 8 or 16: the page faults of a process take turns */

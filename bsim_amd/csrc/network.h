@@ -68,6 +68,8 @@ struct Layout {
     std::vector<bsim_range> rng;
     int32_t parts = 1;                       /* step workgroups per tile (1 or BSIM_NWAVE) */
     std::vector<uint32_t> off_tab;
+    /* the rest but tile_base and tile_nsyn describes the layout to its checks: the
+     * device reads rng, off_tab and the synapses only */
     std::vector<int32_t> src_lo, src_hi;     /* distinct source ranges */
     std::vector<int64_t> src_list_base;      /* list capacity (hi - lo) * D each */
     int64_t src_list_len = 0;

@@ -724,19 +724,24 @@ __device__ __forceinline__ void count_done(const bsim_dev &d, uint64_t cycles)
  * two cycles).  The hardware deals the workgroups out to the XCDs in turn, slot s
  * to XCD s % 8, and starts an XCD's in order.  The units are cut, in index order,
  * into eight runs of equal cost, one per XCD: units of a group, which read the
- * same rows at the same time, so share an L2.  Within an XCD the heavy units come
- * first, by half-octave classes (counting sort).  Within a class the order is
- * arbitrary up to delays of RANK_ORDERED_DMAX steps, and while two workgroups per
- * compute unit hold all units; past them, where most lines are row-table entries
- * that a group's units share while they run together, units keep their order: 1,010,000 neurons with delays up to 50 steps 7.65 / 6.14
- * ms, 410,000 2.51 / 2.36, but 330,000 with delays up to 6 56.5 / 57.9 us.  An XCD has slots for an eighth of the units; the lightest of a
- * longer run fill what others leave free, so that no XCD starts more workgroups
- * than another.  us per cycle with whole groups on XCDs / with the units dealt
- * out in turn where those were uneven / with runs: 330,000 neurons at ~100 Hz
- * 59.9 / 54.5 / 55.0, 650,000 108 / 101 / 98.9, 110,000 with delays up to 50
- * steps 950 / 1,046 / 877, a sweep of 96 chains 27.6 / 27.9 / 27.1, the same in
- * units of half the size 21.7 / 21.9 / 21.2.  Twice the slots, so that runs stay
- * whole: 59.5, 110, 875, 26.9, 22.9 (XCDs with few heavy units start more).
+ * same rows at the same time, so share an L2.  An XCD has slots for an eighth of
+ * the units; the lightest of a longer run fill what others leave free, so that no
+ * XCD starts more workgroups than another.  us per cycle with whole groups on XCDs
+ * / with the units dealt out in turn where those were uneven / with runs: 330,000
+ * neurons at ~100 Hz 59.9 / 54.5 / 55.0, 650,000 108 / 101 / 98.9, 110,000 with
+ * delays up to 50 steps 950 / 1,046 / 877, a sweep of 96 chains 27.6 / 27.9 /
+ * 27.1, the same in units of half the size 21.7 / 21.9 / 21.2.  Twice the slots,
+ * so that runs stay whole: 59.5, 110, 875, 26.9, 22.9 (XCDs with few heavy units
+ * start more).
+ *
+ * Within an XCD the heavy units come first, by half-octave classes (counting
+ * sort).  Within a class the order is arbitrary up to delays of RANK_ORDERED_DMAX
+ * steps, and while two workgroups per compute unit hold all units; past them,
+ * where most lines are row-table entries that a group's units share while they
+ * run together, units keep their order: 1,010,000 neurons with delays up to 50
+ * steps 7.65 / 6.14 ms, 410,000 2.51 / 2.36, but 330,000 with delays up to 6 56.5
+ * / 57.9 us.
+ *
  * Runs in one workgroup, beside the others of the launch, and clears the loads
  * that it has read.  The classes of the units are kept in LDS where they fit. */
 #define RANK_CLASSES 64

@@ -229,7 +229,8 @@ def autotune(points, steps=128, preroll=256, tiles=(192, 384, 768), ranks=(0, 1,
     r cycles, 0 = never, Simulation.set_schedule) with the fastest run of
     `steps` cycles of the batch, timed after `preroll` cycles so that the
     probe sees the swept regime rather than the cold start (no recording;
-    results do not depend on either choice).  Returns ((tile, rank_every),
+    results do not depend on either choice).  0 is timed in the order that the
+    probe's last ranking left, not in a new simulation's.  Returns ((tile, rank_every),
     {(tile, rank_every): seconds})."""
     times = {}
     b = build(points)
